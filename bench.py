@@ -332,7 +332,8 @@ def cpu_baseline(config, seconds):
 
 
 def forward_kernel_name(cfg, cus):
-    """Name rocprofv3 reports for the forward kernel instance that runs on this config (every config is causal).
+    """Name rocprofv3 reports for the FP32-MFMA forward kernel instance of this config's size (every config is causal); it
+    runs where forward_split_kernel_name is None.
     Template arguments: head width, statistics-only, 16-byte vector loads, waves per 32-query item and items per
     persistent workgroup (0: dispatch order), chosen as rk::launch_mapped and rk::dispatch_split
     (rocmkernels_amd/csrc/attention_forward.hip) choose them."""
@@ -351,6 +352,38 @@ def forward_kernel_name(cfg, cus):
         slots = cus * 4 * (2 if cfg["width"] == 64 else 3)
         split = 1 if items >= slots else 2 if 2 * items >= slots else 4
     return f"rk::attention_forward_kernel<{cfg['width']}, false, true, {split}, 0>"
+
+
+def forward_split_kernel_name(cfg, cus):
+    """Name rocprofv3 reports for the split-product forward instance that runs on this config, or None where the FP32-MFMA
+    kernel of forward_kernel_name runs: rk::forward_split_pays and rk::dispatch
+    (rocmkernels_amd/csrc/attention_forward_split.hip). Template arguments: head width, 16-byte vector loads, query tiles
+    per workgroup, key streams, waves per SIMD the registers are held to."""
+    width, length, radius = cfg["width"], cfg["length"], cfg["radius"]
+    qtiles = (length + 31) // 32
+    items = qtiles * cfg["batch"] * cfg["heads"]
+    ramp = radius < 0  # every config is causal
+
+    def tiles(qt):
+        first = max(0, 32 * qt - radius) if radius >= 0 else 0
+        return -(-(min(length, 32 * qt + 32) - first) // 32)
+
+    widest = max(tiles(qtiles // 2), tiles(qtiles - 1))
+    if items <= cus or (ramp and items < 2 * cus):
+        return None
+    if width == 32 and not (widest >= 9 if items <= 2 * cus else radius < 0 or widest >= 5 or items >= 16 * cus):
+        return None
+    if items <= 2 * cus:
+        shape = (2, 4, 2) if width == 32 and widest >= 20 else (2, 2, 2 if width == 32 else 1)
+    elif items <= 4 * cus and width == 32 and ramp:
+        shape = (2, 2, 2)
+    elif items <= 4 * cus and widest >= (16 if width == 32 else 24):
+        shape = (4, 2, 2)
+    elif 4 * cus < items <= 8 * cus and ramp and widest >= (32 if width == 32 else 48):
+        shape = (4, 2, 2)
+    else:  # (the eight-tile instance is for calls without a causal mask)
+        shape = (4, 1, 3 if width == 32 else 2)
+    return f"rk::attention_forward_split_kernel<{width}, true, {shape[0]}, {shape[1]}, {shape[2]}>"
 
 
 def traffic_table():
@@ -654,7 +687,8 @@ def main():
         return
     measured = measure(cfg, args.steps, args.warmup, backward=not args.no_backward)
     fwd = measured["forward"]
-    kernel = forward_kernel_name(cfg, torch.cuda.get_device_properties(0).multi_processor_count)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    kernel = forward_split_kernel_name(cfg, cus) or forward_kernel_name(cfg, cus)
     result = {
         "metric": METRIC,
         "value": round(fwd["tflops_convention"], 4),

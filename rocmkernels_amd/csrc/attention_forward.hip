@@ -1,4 +1,6 @@
-// FP32 online-softmax attention forward for gfx950 (MI355X), head width 16, 32 or 64.
+// FP32 online-softmax attention forward for gfx950 (MI355X), head width 16, 32 or 64, on FP32 MFMAs: the kernel of 16-wide
+// heads, of the statistics-only entry point and of small launches; the others run attention_forward_split.hip (the rule is
+// forward_split_pays there).
 //
 // Replaces the reference's forward kernels: attention_query<false> (Attention.hip:32-115),
 // attention_query_tiled_body (AttentionTile32.h:12-208), attention_query_flash_body (AttentionFlash32.h:23-170),
@@ -437,6 +439,9 @@ void dispatch(const bool statistics_only, const ForwardArgs &a, const int64_t it
         if (vec) launch_mapped<D, true, true>(a, items, cus, stream);
         else launch_mapped<D, true, false>(a, items, cus, stream);
     } else {
+        if constexpr (D >= 32) {
+            if (forward_split_pays(D, a, cus)) return launch_forward_split(D, vec, a, cus, stream);
+        }
         if (vec) launch_mapped<D, false, true>(a, items, cus, stream);
         else launch_mapped<D, false, false>(a, items, cus, stream);
     }

@@ -1,0 +1,742 @@
+// FP32 attention forward for gfx950 (MI355X) on the fp16 matrix cores, head width 32 or 64: the maths of
+// attention_forward.hip (Attention.hip:32-115, AttentionFlash32.h:23-170, Attention64.hip:34-129 in the reference), with
+// each FP32 product formed from three fp16 products of two-term operands (attention_split.hpp).
+//
+// Mapping. A workgroup owns QB query tiles of 32 of one sequence, one per wave of a key stream; its KS key streams take
+// alternate 64-key tiles of the workgroup's window. The QB waves of a stream load each K and V tile together (a share of
+// the rows each, whole lines, a step ahead), split it into terms once, and write the terms to the stream's double-buffered
+// LDS stage, from which all of them read their MFMA operands; so the loads and the splitting of K and V cost each wave
+// 1 / QB of a tile. Q's terms stay in registers; P is split in registers (its accumulator layout is the PV operand's).
+//   * Sᵀ = K·Qᵀ: operands K rows (128-bit LDS reads), Q rows; the small products first.
+//   * Oᵀ += Vᵀ·Pᵀ: operands V through transposing LDS reads (ds_read_b64_tr_b16), P in place.
+// A step is one barrier and a 64-key tile in two halves A and B of 32 keys, in four groups of MFMAs, each beside VALU work
+// that does not depend on it: Sᵀ of A beside the split of the next tile's K; Sᵀ of B beside A's softmax; Oᵀ of A beside B's
+// softmax; Oᵀ of B beside the split of the next tile's V. The source spreads that work evenly over a group's MFMAs and pins
+// the order (the compiler's own order puts the MFMAs first, and the two no longer co-execute).
+//
+// Scales (powers of two): each query row its own; K and V one each for the workgroup, from the largest magnitudes of rows
+// sampled over its window. They put those at 2^8, so rows up to 128 times larger than any sampled one are still in range;
+// larger ones make the result NaN, and a wave that finds a non-finite result computes its query tile again with FP32 MFMAs
+// (as it must anyway for infinities, whose meaning the split products lose).
+#include <algorithm>
+#include <type_traits>
+
+#include "attention_launch.hpp"
+#include "attention_split.hpp"
+
+namespace rk {
+
+namespace {
+
+constexpr int kMaxExponent = 100; // largest scale exponent: 2^±100 times a sum of products stays far inside FP32's range
+constexpr int kStep = 2 * kTile;  // keys of a step
+
+struct SplitForwardParams {
+    Tensor q, k, v;
+    const uint8_t *mask;
+    float *out;
+    int osb, osh, ost;
+    float *lse;
+    Shape s;
+    float scale;
+};
+
+// Position (in 2-byte elements) of element 0 of 16-byte chunk c of row r in a staged plane of D columns: rows are
+// unpadded and their chunks permuted. K's row-layout reads (16 lanes: 16 rows, one chunk each) then meet 16 distinct
+// 16-byte bank groups; V's transposing reads (32 lanes: 4 rows of 64 bytes) cover all 64 banks once.
+template<int D>
+__device__ __forceinline__ int k_chunk(const int r, const int c) {
+    const int swizzle = D == 64 ? ((r & 7) ^ ((r >> 3) & 1)) : ((r >> 2) & 3);
+    return r * D + 8 * (c ^ swizzle);
+}
+template<int D>
+__device__ __forceinline__ int v_chunk(const int r, const int c) {
+    return r * D + 8 * (D == 64 ? c ^ (2 * (r & 3)) : c);
+}
+
+// Calls f(0), .., f(N - 1) with compile-time indexes.
+template<int N, int I = 0, class F>
+__device__ __forceinline__ void unrolled(const F &f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        unrolled<N, I + 1>(f);
+    }
+}
+
+__device__ __forceinline__ u32x2 read_transposed(const uint16_t *p) {
+    typedef short v4s __attribute__((ext_vector_type(4)));
+    return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s *)(p)));
+}
+
+// Writes the output rows and statistics of a wave's query tile: state (m_raw, l) with l summed over both half-waves, O
+// = o / l times 2^ev, the row maximum m_raw·2^e, and l relative to the true maximum `sum`.
+template<int D, bool VEC>
+__device__ __forceinline__ void store_rows(const SplitForwardParams &P, const int seq, const int query, const int h, const f32x16 (&o)[D / 32],
+        const float l, const float row_max, const float sum, const int ev) {
+    if (query >= P.s.queries) return;
+    const int b = seq / P.s.heads, head = seq - b * P.s.heads;
+    const bool nan_row = isnan(l);
+    const bool has_keys = l > 0.0f;
+    const float factor = has_keys ? __builtin_amdgcn_ldexpf(1.0f / l, ev) : (nan_row ? NAN : 0.0f);
+    float *orow = P.out + static_cast<int64_t>(b) * P.osb + static_cast<int64_t>(head) * P.osh + static_cast<int64_t>(query) * P.ost;
+#pragma unroll
+    for (int t = 0; t < D / 32; ++t) {
+        if (has_keys) {
+            store_tile_row<VEC>(orow + 32 * t, o[t], factor, h);
+        } else {
+            const f32x16 fill{};
+            store_tile_row<VEC>(orow + 32 * t, fill + factor, 1.0f, h);
+        }
+    }
+    if (h == 0) {
+        const int64_t row = static_cast<int64_t>(seq) * P.s.queries + query;
+        P.lse[2 * row] = has_keys ? row_max : (nan_row ? NAN : -INFINITY);
+        P.lse[2 * row + 1] = has_keys ? sum : (nan_row ? NAN : 0.0f);
+    }
+}
+
+// One query tile on FP32 MFMAs by one wave, for inputs that the split products cannot carry: the arithmetic of
+// attention_forward.hip, operands straight from memory. Kept out of line (and given the kernel's arguments by address), so
+// that the main loop's registers do not depend on it.
+template<int D, bool VEC>
+__device__ __attribute__((noinline)) void exact_query_tile(const SplitForwardParams *params, const int seq_, const int q0_) {
+    const auto address = reinterpret_cast<uint64_t>(params);
+    const uint64_t uniform = static_cast<uint64_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(address >> 32))) << 32 |
+            static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(address)));
+    const SplitForwardParams &P = *reinterpret_cast<const SplitForwardParams *>(uniform);
+    const int seq = __builtin_amdgcn_readfirstlane(seq_), q0 = __builtin_amdgcn_readfirstlane(q0_);
+    constexpr int HALF = D / 2, DT = D / 32;
+    const Shape s = P.s;
+    const int lane = threadIdx.x & (kWave - 1), col = lane & 31, h = lane >> 5;
+    const int query = q0 + col;
+    const int b = seq / s.heads, head = seq - b * s.heads;
+    const Buffer qbuf = make_buffer(sequence(P.q, b, head), sequence_bytes(s.queries, P.q.st, D));
+    const Buffer kbuf = make_buffer(sequence(P.k, b, head), sequence_bytes(s.keys, P.k.st, D));
+    const Buffer vbuf = make_buffer(sequence(P.v, b, head), sequence_bytes(s.keys, P.v.st, D));
+    const Buffer mbuf = make_buffer(P.mask + static_cast<int64_t>(b) * s.keys, static_cast<uint32_t>(s.keys));
+    const uint32_t kstep = 4u * P.k.st, vstep = 4u * P.v.st;
+    const float c2 = P.scale * kLog2e;
+    const int wlo = window_lo(s, query), whi = window_hi(s, query);
+    int first, last;
+    forward_key_range(s, q0 / kTile, first, last);
+
+    float qr[HALF];
+    buffer_load_span<VEC>(qr, qbuf, static_cast<uint32_t>(query) * (4u * P.q.st) + 4u * h * HALF);
+    float m = -INFINITY, base = -INFINITY, l = 0.0f; // m over this half-wave's keys; base of l and o, in log2 units
+    f32x16 o[DT];
+#pragma unroll
+    for (int t = 0; t < DT; ++t) o[t] = f32x16{};
+#pragma unroll 1
+    for (int key0 = first; key0 < last; key0 += kTile) {
+        const uint32_t bits = static_cast<uint32_t>(__ballot(buffer_load_byte(mbuf, static_cast<uint32_t>(key0 + col)) != 0));
+        if (bits == 0) continue;
+        f32x16 sc{};
+        {
+            float kr[HALF];
+            buffer_load_span<VEC>(kr, kbuf, static_cast<uint32_t>(key0 + col) * kstep + 4u * h * HALF);
+#pragma unroll
+            for (int c = 0; c < HALF; ++c) sc = mfma(kr[c], qr[c], sc);
+        }
+        const uint32_t visible = (bits & bit_range(wlo - key0, whi - key0)) >> (4 * h);
+        float mx = m;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            sc[j] = (visible >> (8 * (j >> 2) + (j & 3))) & 1u ? sc[j] : -INFINITY;
+            mx = fmaxf(mx, sc[j]);
+        }
+        m = mx;
+        const float row = halves_max(m);
+        const float base_new = row == -INFINITY ? -INFINITY : row * c2;
+        const float alpha = base_new == -INFINITY ? 1.0f : exp2_fast(base - base_new);
+        base = base_new;
+        l *= alpha;
+#pragma unroll
+        for (int t = 0; t < DT; ++t) o[t] *= alpha;
+        const float offset = base == -INFINITY ? 0.0f : base;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            sc[j] = exp2_fast(fmaf(sc[j], c2, -offset));
+            l += sc[j];
+        }
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const int r = tile_row(j, h);
+#pragma unroll
+            for (int t = 0; t < DT; ++t) {
+                // Masked keys contribute exactly nothing, whatever their stored values hold.
+                const uint32_t at = (bits >> r) & 1u ? static_cast<uint32_t>(key0 + r) * vstep + 4u * (32 * t + col) : kNoRow;
+                o[t] = mfma(buffer_load(vbuf, at, 0), sc[j], o[t]);
+            }
+        }
+    }
+    const float m_all = halves_max(m);
+    l = halves_sum(l);
+    const float sum = m_all == -INFINITY ? l : l * exp2_fast((base == -INFINITY ? 0.0f : base) - m_all * c2);
+    store_rows<D, VEC>(P, seq, query, h, o, l, m_all * P.scale, sum, 0);
+}
+
+} // namespace
+
+template<int D, bool VEC, int QB, int KS, int WPE>
+__global__ __launch_bounds__(kWave * QB * KS) __attribute__((amdgpu_waves_per_eu(WPE))) void attention_forward_split_kernel(
+        const SplitForwardParams P) {
+    constexpr int KC = D / 16;                       // 16-feature steps of Sᵀ
+    constexpr int DT = D / 32;                       // 32-feature slices of the output
+    constexpr int CPR = D / 4;                       // 4-float chunks per row
+    constexpr int CH = kStep * CPR / (kWave * QB);   // chunks per lane of a K tile, and of a V tile
+    static_assert(CH >= 1 && CH * kWave * QB == kStep * CPR);
+    constexpr int PLANE = kStep * D;                 // elements of one term of one tile
+    constexpr int STAGE = 4 * PLANE;                 // K's two terms, high and low, then V's
+    constexpr int NREG = 16 * DT + 3;                // merged per lane: maximum, sum, base and the accumulators
+    constexpr int STAGE_BYTES = 2 * KS * STAGE * 2;
+    constexpr int MERGE_BYTES = (KS - 1) * QB * NREG * kWave * 4;
+    __shared__ __align__(16) unsigned char smem[STAGE_BYTES > MERGE_BYTES ? STAGE_BYTES : MERGE_BYTES];
+    __shared__ float amax[2][QB * KS];               // largest sampled |K| and |V| of each wave
+
+    const Shape &s = P.s;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int qi = wave % QB;     // query tile of the block
+    const int stream = wave / QB; // key stream
+    const int col = lane & 31;
+    const int h = lane >> 5;
+    const float one = split_unit_scale();
+
+    // Workgroup g takes a query block of sequence g mod B·H, the heaviest blocks first: with B·H a multiple of 8 each XCD
+    // (workgroup g runs on XCD g mod 8) streams the K/V rows of its own eighth of the sequences from its L2.
+    const int seqs = s.batch * s.heads;
+    const int seq = static_cast<int>(blockIdx.x) % seqs;
+    const int rank = static_cast<int>(blockIdx.x) / seqs;
+    const int b = seq / s.heads, head = seq - b * s.heads;
+    const int nblocks = (s.queries + QB * kTile - 1) / (QB * kTile);
+
+    const Buffer qbuf = make_buffer(sequence(P.q, b, head), sequence_bytes(s.queries, P.q.st, D));
+    const Buffer kbuf = make_buffer(sequence(P.k, b, head), sequence_bytes(s.keys, P.k.st, D));
+    const Buffer vbuf = make_buffer(sequence(P.v, b, head), sequence_bytes(s.keys, P.v.st, D));
+    const Buffer mbuf = make_buffer(P.mask + static_cast<int64_t>(b) * s.keys, static_cast<uint32_t>(s.keys));
+    const uint32_t qstep = 4u * P.q.st, kstep = 4u * P.k.st, vstep = 4u * P.v.st;
+
+    // This lane's chunks of a tile: chunk i is row crow + RPC·i, 4 floats from column 4 (lane mod CPR).
+    constexpr int RPC = kWave * QB / CPR;
+    const int crow = (qi * kWave + lane) / CPR;
+    const uint32_t kofs = static_cast<uint32_t>(crow) * kstep + 16u * static_cast<uint32_t>(lane % CPR);
+    const uint32_t vofs = static_cast<uint32_t>(crow) * vstep + 16u * static_cast<uint32_t>(lane % CPR);
+    int kwrite[CH], vwrite[CH];
+#pragma unroll
+    for (int i = 0; i < CH; ++i) {
+        const int chunk = lane % CPR;
+        kwrite[i] = k_chunk<D>(crow + RPC * i, chunk >> 1) + 4 * (chunk & 1);
+        vwrite[i] = v_chunk<D>(crow + RPC * i, chunk >> 1) + 4 * (chunk & 1);
+    }
+    int kread[KC], vread[DT];
+#pragma unroll
+    for (int i = 0; i < KC; ++i) kread[i] = k_chunk<D>(col, 2 * i + h);
+    // Transposing reads: lane L of each 16-lane group points at row r0 + (L mod 16) / 4, features f0 + 4 (L mod 4) .. + 3,
+    // and receives feature f0 + L mod 16 of rows r0 .. r0 + 3, with r0 = 16u + 8p + 4h and f0 = 32 t2 + 16 (col / 16).
+#pragma unroll
+    for (int t2 = 0; t2 < DT; ++t2)
+        vread[t2] = v_chunk<D>(4 * h + ((lane & 15) >> 2), 4 * t2 + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) + 4 * (lane & 1);
+    uint16_t *const stages = reinterpret_cast<uint16_t *>(smem) + stream * (2 * STAGE);
+
+    auto load4 = [&](const Buffer r, const uint32_t voffset, const uint32_t soffset) __attribute__((always_inline)) {
+        if constexpr (VEC) return buffer_load4(r, voffset, soffset);
+        else return f32x4{buffer_load(r, voffset, soffset), buffer_load(r, voffset + 4u, soffset), buffer_load(r, voffset + 8u, soffset),
+                buffer_load(r, voffset + 12u, soffset)};
+    };
+
+    const int qb = s.causal ? nblocks - 1 - rank : rank;
+    const int q0 = (qb * QB + qi) * kTile;
+    const int query = q0 + col;
+    const bool tile_valid = q0 < s.queries;
+
+    // This wave's window of keys [first, last) and the workgroup's union of windows, in tiles from ufirst.
+    int first, last, ufirst, ulast, unused;
+    forward_key_range(s, q0 / kTile, first, last);
+    forward_key_range(s, qb * QB, ufirst, unused);
+    forward_key_range(s, min(qb * QB + QB - 1, (s.queries - 1) / kTile), unused, ulast);
+    const int ntiles = ulast > ufirst ? (ulast - ufirst + kStep - 1) / kStep : 0;
+    const int nsteps = (ntiles + KS - 1) / KS; // tile of stream x at step i: i·KS + x
+    const int wlo = window_lo(s, query);
+    const int whi = window_hi(s, query);
+
+    // Rows in flight, and their mask (one byte per key, 64 lanes). Rows of masked keys are cleared before they are split:
+    // they contribute exactly nothing, whatever they hold.
+    f32x4 kraw[CH], vraw[CH];
+    auto tile_key = [&](const int i) { return ufirst + (i * KS + stream) * kStep; };
+    auto load_mask = [&](const int i) __attribute__((always_inline)) {
+        return buffer_load_byte_s(mbuf, static_cast<uint32_t>(lane), i * KS + stream < ntiles ? static_cast<uint32_t>(tile_key(i)) : kNoRow);
+    };
+    auto load_chunks = [&](f32x4 (&raw)[CH], const Buffer buf, const uint32_t at, const uint32_t step, const int i) __attribute__((always_inline)) {
+        const uint32_t row0 = i * KS + stream < ntiles ? static_cast<uint32_t>(tile_key(i)) * step : kNoRow;
+#pragma unroll
+        for (int c = 0; c < CH; ++c) raw[c] = load4(buf, at, row0 + static_cast<uint32_t>(RPC * c) * step);
+    };
+    // Scales. Every thread reads a chunk of K and V in one of ROWS rows spread over the workgroup's window; masked rows
+    // (keys past the end too) count as 0.
+    constexpr int ROWS = kWave * QB * KS / CPR;
+    int ek, ev; // K = K'·2^ek, V = V'·2^ev
+    f32x4 qraw[2 * KC];
+    int mask0;
+    bool plain; // magnitudes that FP32 powers of two cannot bring into range: FP32 MFMAs from the start
+    {
+        const int n = min(ulast, s.keys) - ufirst;
+        const int key = ufirst + (n > 0 ? static_cast<int>(static_cast<int64_t>(static_cast<int>(threadIdx.x) / CPR) * n / ROWS) : 0);
+        const uint32_t at = 16u * (threadIdx.x % CPR);
+        const int seen = buffer_load_byte(mbuf, static_cast<uint32_t>(key));
+        const f32x4 x = load4(kbuf, static_cast<uint32_t>(key) * kstep + at, 0), y = load4(vbuf, static_cast<uint32_t>(key) * vstep + at, 0);
+        // Q and the first tile behind them: one round trip for all.
+#pragma unroll
+        for (int i = 0; i < KC; ++i) {
+            const uint32_t at = tile_valid ? static_cast<uint32_t>(query) * qstep + 4u * (16 * i + 8 * h) : kNoRow;
+            qraw[2 * i] = load4(qbuf, at, 0);
+            qraw[2 * i + 1] = load4(qbuf, at + 16u, 0);
+        }
+        load_chunks(kraw, kbuf, kofs, kstep, 0);
+        load_chunks(vraw, vbuf, vofs, vstep, 0);
+        mask0 = load_mask(0);
+        __builtin_amdgcn_sched_barrier(0);
+        float mk = fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3])));
+        float mv = fmaxf(fmaxf(fabsf(y[0]), fabsf(y[1])), fmaxf(fabsf(y[2]), fabsf(y[3])));
+        mk = seen != 0 ? mk : 0.0f;
+        mv = seen != 0 ? mv : 0.0f;
+#pragma unroll
+        for (int m = 1; m < kWave; m <<= 1) {
+            mk = fmaxf(mk, __shfl_xor(mk, m));
+            mv = fmaxf(mv, __shfl_xor(mv, m));
+        }
+        if (lane == 0) {
+            amax[0][wave] = mk;
+            amax[1][wave] = mv;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < QB * KS; ++w) {
+            mk = fmaxf(mk, amax[0][w]);
+            mv = fmaxf(mv, amax[1][w]);
+        }
+        ek = __builtin_amdgcn_readfirstlane(exponent_of(mk)) - 8;
+        ev = __builtin_amdgcn_readfirstlane(exponent_of(mv)) - 8;
+        plain = ek < -kMaxExponent || ek > kMaxExponent || ev < -kMaxExponent || ev > kMaxExponent;
+    }
+
+    // Q's terms, scaled so that the row's largest magnitude is in [2^14, 2^15).
+    h16x8 qh[KC], ql[KC];
+    int e; // S = S'·2^e
+    {
+        float span[KC][8], mq = 0.0f;
+#pragma unroll
+        for (int i = 0; i < KC; ++i) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                span[i][j] = qraw[2 * i][j];
+                span[i][4 + j] = qraw[2 * i + 1][j];
+            }
+#pragma unroll
+            for (int j = 0; j < 8; ++j) mq = fmaxf(mq, fabsf(span[i][j]));
+        }
+        const int eq = exponent_of(halves_max(mq)) - 14;
+        plain = plain || __ballot(eq < -kMaxExponent || eq > kMaxExponent) != 0;
+        const float factor = power_of_two(-min(max(eq, -kMaxExponent), kMaxExponent));
+#pragma unroll
+        for (int i = 0; i < KC; ++i) {
+            u32x4 hi, lo;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                uint32_t x, y;
+                split_pair<true>(span[i][2 * j], span[i][2 * j + 1], factor, x, y);
+                hi[j] = x;
+                lo[j] = y;
+            }
+            qh[i] = __builtin_bit_cast(h16x8, hi);
+            ql[i] = __builtin_bit_cast(h16x8, lo);
+        }
+        e = eq + ek;
+    }
+    const float kfactor = power_of_two(-min(max(ek, -kMaxExponent), kMaxExponent));
+    const float vfactor = power_of_two(-min(max(ev, -kMaxExponent), kMaxExponent));
+
+    // Online-softmax state, as in attention_forward.hip (lazy re-basing: see there), in units of S' and V'. P is kept at
+    // 2^kShift times its value, so that its terms lose nothing above 2^-10 and at most 2^-32.
+    constexpr float kLazy = 8.0f, kShift = 7.0f;
+    const float c2 = __builtin_amdgcn_ldexpf(P.scale * kLog2e, e);
+    const float lazy_raw = fminf(kLazy / c2, 1e30f);
+    float m_half = -INFINITY, m_lazy = -INFINITY, mc = -INFINITY, mcx = 0.0f, l_run = 0.0f, alpha = 1.0f;
+    f32x16 o[DT];
+#pragma unroll
+    for (int t = 0; t < DT; ++t) o[t] = f32x16{};
+
+    auto clear_masked = [&](const uint64_t bits) __attribute__((always_inline)) {
+        if (__builtin_expect(bits != ~0ull, 0)) {
+#pragma unroll
+            for (int c = 0; c < CH; ++c) {
+                const int keep = -static_cast<int>((bits >> (crow + RPC * c)) & 1u);
+#pragma unroll
+                for (int x = 0; x < 4; ++x) {
+                    __asm__("v_and_b32 %0, %1, %0" : "+v"(kraw[c][x]) : "v"(keep)); // in place
+                    __asm__("v_and_b32 %0, %1, %0" : "+v"(vraw[c][x]) : "v"(keep));
+                }
+            }
+        }
+    };
+    // Splitting of the next tile's rows into stage p, in units of a pair of floats (the second of a chunk also writes).
+    u32x2 chunk[2];
+    auto split_unit = [&](auto unit, auto is_v, const int p) __attribute__((always_inline)) {
+        constexpr int C = decltype(unit)::value / 2, E = decltype(unit)::value % 2;
+        constexpr bool V = decltype(is_v)::value;
+        const f32x4 &raw = V ? vraw[C] : kraw[C];
+        uint32_t x, y;
+        split_pair<true>(raw[2 * E], raw[2 * E + 1], V ? vfactor : kfactor, x, y);
+        chunk[0][E] = x;
+        chunk[1][E] = y;
+        if constexpr (E == 1) {
+            uint16_t *const st = stages + p * STAGE + (V ? 2 * PLANE + vwrite[C] : kwrite[C]);
+            *reinterpret_cast<u32x2 *>(st) = chunk[0];
+            *reinterpret_cast<u32x2 *>(st + PLANE) = chunk[1];
+        }
+    };
+    constexpr std::integral_constant<bool, false> kOfK{};
+    constexpr std::integral_constant<bool, true> kOfV{};
+
+    // Operands of half x of the tile in stage p.
+    auto read_k = [&](h16x8 (&kt)[KC], const int p, const int x, const int term) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < KC; ++i)
+            kt[i] = *reinterpret_cast<const h16x8 *>(stages + p * STAGE + term * PLANE + x * kTile * D + kread[i]);
+    };
+    auto read_v = [&](h16x8 (&vt)[DT], const int p, const int x, const int u, const int term) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t2 = 0; t2 < DT; ++t2) {
+            const uint16_t *const at = stages + p * STAGE + (2 + term) * PLANE + (x * kTile + 16 * u) * D + vread[t2];
+            const u32x2 lo = read_transposed(at), hi = read_transposed(at + 8 * D);
+            vt[t2] = __builtin_bit_cast(h16x8, u32x4{lo[0], lo[1], hi[0], hi[1]});
+        }
+    };
+    // MFMA M of Sᵀ: K low with Q high, K high with Q low, K high with Q high.
+    auto score_mfma = [&](auto index, f32x16 &sc, const h16x8 (&kl)[KC], const h16x8 (&kh)[KC]) __attribute__((always_inline)) {
+        constexpr int M = decltype(index)::value;
+        sc = mfma_f16(M < KC ? kl[M % KC] : kh[M % KC], M < KC || M >= 2 * KC ? qh[M % KC] : ql[M % KC], sc);
+    };
+    uint32_t ps[2][8]; // P's terms: the PV operand of MFMA step u is words 4u .. 4u + 3
+    // MFMAs M of Oᵀ (DT each): V low with P high, V high with P low, V high with P high, for each half u of the 32 keys.
+    auto output_mfma = [&](auto index, const uint32_t (&pt)[2][8], const h16x8 (&vl)[DT], const h16x8 (&vh)[DT]) __attribute__((always_inline)) {
+        constexpr int M = decltype(index)::value;
+        constexpr int U = M / 3, Y = M % 3 == 1;
+        const h16x8 x = __builtin_bit_cast(h16x8, u32x4{pt[Y][4 * U], pt[Y][4 * U + 1], pt[Y][4 * U + 2], pt[Y][4 * U + 3]});
+#pragma unroll
+        for (int t2 = 0; t2 < DT; ++t2) o[t2] = mfma_f16(M % 3 == 0 ? vl[t2] : vh[t2], x, o[t2]);
+    };
+    auto mask_scores = [&](f32x16 &sc, const int key0, const uint32_t bits) __attribute__((always_inline)) {
+        const uint32_t visible = (bits & bit_range(wlo - key0, whi - key0)) >> (4 * h);
+#pragma unroll
+        for (int j = 0; j < 16; ++j) sc[j] = (visible >> (8 * (j >> 2) + (j & 3))) & 1u ? sc[j] : -INFINITY;
+    };
+    // Running maximum over half a tile's scores; when some row must be re-based, moves every row's base to its current
+    // maximum and returns true: o is then to be rescaled by alpha once the products already due are added.
+    auto maxima = [&](const f32x16 &sc) __attribute__((always_inline)) {
+        float mx = m_half;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) mx = fmaxf(mx, sc[j]);
+        m_half = mx;
+        const bool due = __ballot(m_half > m_lazy) != 0;
+        if (__builtin_expect(due, 0)) {
+            const float m_row = halves_max(m_half);
+            const float mc_new = m_row == -INFINITY ? -INFINITY : m_row * c2;
+            m_lazy = m_row + lazy_raw;
+            alpha = mc_new == -INFINITY ? 1.0f : exp2_fast(mc - mc_new);
+            l_run *= alpha;
+            mc = mc_new;
+            mcx = mc_new == -INFINITY ? 0.0f : mc_new - kShift;
+        }
+        return due;
+    };
+    auto rescale = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int t2 = 0; t2 < DT; ++t2) o[t2] *= alpha;
+    };
+    // Exponentials and terms of scores 2u and 2u + 1.
+    float psum = 0.0f;
+    auto softmax_unit = [&](auto unit, const f32x16 &sc, uint32_t (&pt)[2][8]) __attribute__((always_inline)) {
+        constexpr int U = decltype(unit)::value;
+        const float x = exp2_fast(fmaf(sc[2 * U], c2, -mcx)), y = exp2_fast(fmaf(sc[2 * U + 1], c2, -mcx));
+        psum = U == 0 ? x + y : psum + (x + y);
+        split_pair<false>(x, y, one, pt[0][U], pt[1][U]);
+        __asm__ volatile("" : "+v"(psum), "+v"(pt[1][U])); // here, not where they are next used (behind the next group's branch)
+    };
+
+    // A whole step, both halves seen by this wave; MASKED applies the boundary masks to both.
+    auto full_step = [&](auto masked, const int p, const int key0, const uint64_t bits) __attribute__((always_inline)) {
+        constexpr bool MASKED = decltype(masked)::value;
+        constexpr int NS = 3 * KC, UNITS = 2 * CH; // MFMAs of Sᵀ; units of K, and of V
+        h16x8 kl[KC], kh[KC], vl[DT], vh[DT];
+        f32x16 sa{}, sb{};
+        read_k(kl, p, 0, 1);
+        read_k(kh, p, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        unrolled<NS>([&](auto m) __attribute__((always_inline)) {
+            constexpr int M = decltype(m)::value, U0 = M * UNITS / NS, U1 = (M + 1) * UNITS / NS;
+            score_mfma(m, sa, kl, kh);
+            if constexpr (M == KC) read_k(kl, p, 1, 1);
+            unrolled<U1 - U0>([&](auto u) __attribute__((always_inline)) {
+                split_unit(std::integral_constant<int, U0 + decltype(u)::value>{}, kOfK, p ^ 1);
+            });
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        read_k(kh, p, 1, 0);
+        bool due = false;
+        uint32_t pa[2][8];
+        unrolled<NS>([&](auto m) __attribute__((always_inline)) {
+            constexpr int M = decltype(m)::value, LEAD = 2; // MFMAs before the maxima
+            score_mfma(m, sb, kl, kh);
+            if constexpr (M == LEAD - 1) {
+                if constexpr (MASKED) mask_scores(sa, key0, static_cast<uint32_t>(bits));
+                if (__builtin_expect(maxima(sa), 0)) rescale();
+            } else if constexpr (M >= LEAD) {
+                constexpr int U0 = (M - LEAD) * 8 / (NS - LEAD), U1 = (M - LEAD + 1) * 8 / (NS - LEAD);
+                unrolled<U1 - U0>([&](auto u) __attribute__((always_inline)) {
+                    softmax_unit(std::integral_constant<int, U0 + decltype(u)::value>{}, sa, pa);
+                });
+            }
+            if constexpr (M == NS - 2) read_v(vl, p, 0, 0, 1);
+            if constexpr (M == NS - 1) read_v(vh, p, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        l_run += psum;
+        unrolled<6>([&](auto m) __attribute__((always_inline)) {
+            constexpr int M = decltype(m)::value;
+            output_mfma(m, pa, vl, vh);
+            if constexpr (M % 3 == 0) read_v(vl, p, M / 3, 1 - M / 3, 1); // (half A, u = 1), then (half B, u = 0)
+            if constexpr (M % 3 == 2) read_v(vh, p, M / 3, 1 - M / 3, 0);
+            if constexpr (M == 0) {
+                if constexpr (MASKED) mask_scores(sb, key0 + kTile, static_cast<uint32_t>(bits >> 32));
+                due = maxima(sb);
+            } else {
+                constexpr int U0 = (M - 1) * 8 / 5, U1 = M * 8 / 5;
+                unrolled<U1 - U0>([&](auto u) __attribute__((always_inline)) {
+                    softmax_unit(std::integral_constant<int, U0 + decltype(u)::value>{}, sb, ps);
+                });
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        l_run += psum;
+        if (__builtin_expect(due, 0)) rescale();
+        unrolled<6>([&](auto m) __attribute__((always_inline)) {
+            constexpr int M = decltype(m)::value, U0 = M * UNITS / 6, U1 = (M + 1) * UNITS / 6;
+            output_mfma(m, ps, vl, vh);
+            if constexpr (M == 0) read_v(vl, p, 1, 1, 1);
+            if constexpr (M == 2) read_v(vh, p, 1, 1, 0);
+            unrolled<U1 - U0>([&](auto u) __attribute__((always_inline)) {
+                split_unit(std::integral_constant<int, U0 + decltype(u)::value>{}, kOfV, p ^ 1);
+            });
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    };
+    // Half x of a tile alone.
+    auto half_step = [&](const int p, const int x, const int key0, const uint32_t bits) __attribute__((always_inline)) {
+        h16x8 kl[KC], kh[KC], vl[DT], vh[DT];
+        f32x16 sc{};
+        read_k(kl, p, x, 1);
+        read_k(kh, p, x, 0);
+        unrolled<3 * KC>([&](auto m) __attribute__((always_inline)) { score_mfma(m, sc, kl, kh); });
+        mask_scores(sc, key0, bits);
+        if (maxima(sc)) rescale();
+        unrolled<8>([&](auto u) __attribute__((always_inline)) { softmax_unit(u, sc, ps); });
+        l_run += psum;
+        unrolled<6>([&](auto m) __attribute__((always_inline)) {
+            constexpr int M = decltype(m)::value;
+            if constexpr (M % 3 == 0) {
+                read_v(vl, p, x, M / 3, 1);
+                read_v(vh, p, x, M / 3, 0);
+            }
+            output_mfma(m, ps, vl, vh);
+        });
+    };
+    auto split_rows = [&](const int p) __attribute__((always_inline)) {
+        unrolled<2 * CH>([&](auto u) __attribute__((always_inline)) { split_unit(u, kOfK, p); });
+        unrolled<2 * CH>([&](auto u) __attribute__((always_inline)) { split_unit(u, kOfV, p); });
+    };
+
+    if (nsteps > 0 && !plain) {
+        uint64_t bits0 = __ballot(mask0 != 0);
+        clear_masked(bits0);
+        split_rows(0);
+        load_chunks(kraw, kbuf, kofs, kstep, 1);
+        load_chunks(vraw, vbuf, vofs, vstep, 1);
+        int mbyte = load_mask(1);
+        auto step = [&](const int i, const int p) __attribute__((always_inline)) {
+            __syncthreads(); // tile i is staged; every wave is done with the other stage
+            const int key0 = tile_key(i);
+            const bool live = i * KS + stream < ntiles && tile_valid;
+            const bool see_a = live && static_cast<uint32_t>(bits0) != 0 && key0 < last && key0 + kTile > first;
+            const bool see_b = live && static_cast<uint32_t>(bits0 >> 32) != 0 && key0 + kTile < last && key0 + kStep > first;
+            const bool inside = bits0 == ~0ull && tile_in_window(s, q0, key0) && tile_in_window(s, q0, key0 + kTile);
+            const uint64_t bits1 = __ballot(mbyte != 0);
+            clear_masked(bits1);
+            if (__builtin_expect(see_a && see_b && inside, 1)) {
+                full_step(std::integral_constant<bool, false>{}, p, key0, bits0);
+            } else if (see_a && see_b) {
+                full_step(std::integral_constant<bool, true>{}, p, key0, bits0);
+            } else {
+                if (see_a || see_b) {
+                    const int x = see_a ? 0 : 1;
+                    half_step(p, x, key0 + x * kTile, static_cast<uint32_t>(bits0 >> (32 * x)));
+                }
+                split_rows(p ^ 1);
+            }
+            load_chunks(kraw, kbuf, kofs, kstep, i + 2);
+            load_chunks(vraw, vbuf, vofs, vstep, i + 2);
+            mbyte = load_mask(i + 2);
+            bits0 = bits1;
+        };
+        for (int i = 0; i < nsteps; i += 2) {
+            step(i, 0);
+            if (i + 1 < nsteps) step(i + 1, 1);
+        }
+    }
+
+    float m_all = halves_max(m_half), mc_all = mc, l_all = l_run;
+    if constexpr (KS > 1) {
+        // Streams 1 .. KS - 1 hand (row maximum, sum, base, accumulators) to stream 0 through LDS, which adds them in
+        // order, each rescaled to the largest base.
+        float *const slots = reinterpret_cast<float *>(smem) + qi * (NREG * kWave) + lane;
+        constexpr int SLOT = QB * NREG * kWave;
+        __syncthreads(); // every wave is done with the stages
+        if (stream > 0) {
+            float *const slot = slots + (stream - 1) * SLOT;
+            slot[0] = m_all;
+            slot[kWave] = l_run;
+            slot[2 * kWave] = mc;
+#pragma unroll
+            for (int t = 0; t < DT; ++t) {
+#pragma unroll
+                for (int j = 0; j < 16; ++j) slot[(3 + 16 * t + j) * kWave] = o[t][j];
+            }
+        }
+        __syncthreads();
+        if (stream == 0) {
+#pragma unroll
+            for (int x = 0; x < KS - 1; ++x) {
+                m_all = fmaxf(m_all, slots[x * SLOT]);
+                mc_all = fmaxf(mc_all, slots[x * SLOT + 2 * kWave]);
+            }
+            const float base = mc_all == -INFINITY ? 0.0f : mc_all;
+            const float a0 = exp2_fast(mc - base);
+            l_all = l_run * a0;
+#pragma unroll
+            for (int t = 0; t < DT; ++t) o[t] *= a0;
+#pragma unroll
+            for (int x = 0; x < KS - 1; ++x) {
+                const float *const slot = slots + x * SLOT;
+                const float a = exp2_fast(slot[2 * kWave] - base);
+                l_all = fmaf(slot[kWave], a, l_all);
+#pragma unroll
+                for (int t = 0; t < DT; ++t) {
+#pragma unroll
+                    for (int j = 0; j < 16; ++j) o[t][j] = fmaf(slot[(3 + 16 * t + j) * kWave], a, o[t][j]);
+                }
+            }
+        }
+    }
+
+    if (stream == 0 && tile_valid) {
+        // A non-finite result: some input of the tile is not finite or out of its scale's range, or the result overflows.
+        float probe = l_all * 0.0f;
+#pragma unroll
+        for (int t = 0; t < DT; ++t) {
+#pragma unroll
+            for (int j = 0; j < 16; ++j) probe = fmaf(o[t][j], 0.0f, probe);
+        }
+        if (__builtin_expect(plain || __ballot(probe != 0.0f) != 0, 0)) {
+            exact_query_tile<D, VEC>((const SplitForwardParams *)__builtin_amdgcn_kernarg_segment_ptr(), seq, q0);
+        } else {
+            l_all = halves_sum(l_all); // each half-wave summed the exponentials of its own keys
+            const float base = mc_all == -INFINITY ? 0.0f : mc_all;
+            // O is o / l in any offset; lse's sum is Σ exp(s - max) = l · exp2(offset - max·c2).
+            const float sum = m_all == -INFINITY ? l_all : l_all * exp2_fast(base - kShift - m_all * c2);
+            store_rows<D, VEC>(P, seq, query, h, o, l_all, __builtin_amdgcn_ldexpf(m_all * P.scale, e), sum, ev);
+        }
+    }
+}
+
+namespace {
+
+template<int D, bool VEC, int QB, int KS, int WPE = 2>
+void launch(const ForwardArgs &a, hipStream_t stream) {
+    const int64_t blocks = static_cast<int64_t>(a.batch) * a.heads * ((a.queries + QB * kTile - 1) / (QB * kTile));
+    const SplitForwardParams params{Tensor{a.q, a.qs.batch, a.qs.head, a.qs.token}, Tensor{a.k, a.ks.batch, a.ks.head, a.ks.token},
+            Tensor{a.v, a.vs.batch, a.vs.head, a.vs.token}, reinterpret_cast<const uint8_t *>(a.mask), a.output, a.os.batch, a.os.head,
+            a.os.token, a.lse, Shape{a.batch, a.heads, a.queries, a.keys, a.radius, a.causal}, 1.0f / sqrtf(static_cast<float>(D))};
+    hipLaunchKernelGGL((attention_forward_split_kernel<D, VEC, QB, KS, WPE>), dim3(static_cast<unsigned>(blocks)), dim3(kWave * QB * KS), 0,
+            stream, params);
+}
+
+// Shape of the launch's work: 32-query items, 32-key tiles of the widest item, and whether item costs run from one tile to
+// all of them (a causal mask without a radius window).
+struct Work {
+    int64_t items;
+    int tiles;
+    bool ramp;
+};
+
+Work work_of(const ForwardArgs &a) {
+    const Shape s{a.batch, a.heads, a.queries, a.keys, a.radius, a.causal};
+    const int qtiles = (a.queries + kTile - 1) / kTile;
+    Work w{static_cast<int64_t>(qtiles) * a.batch * a.heads, 0, a.causal != 0 && a.radius < 0};
+    w.tiles = std::max(forward_item_tiles(s, qtiles / 2), forward_item_tiles(s, qtiles - 1));
+    return w;
+}
+
+// Workgroup shape. Every µs below: items, key tiles per item: this choice against the next best one.
+//   * Up to two items per CU: two query tiles per workgroup, so that every CU has work, and as many key streams as LDS
+//     holds (d = 64: 384, 32: 24.2 against 28.2 with four query tiles; d = 32, 512, 64: 24.1 with four streams, 28.0 with two;
+//     384, 16: 10.7 both).
+//   * Up to four items per CU: four query tiles and two streams if the items are long (d = 64: 768, 32: 29.7 against 32.4;
+//     d = 32: 768, 32: 20.2 against 23.0), one if not (d = 64: 768, 8: 13.1 against 14.3). Under a ramp at d = 32 two and two
+//     (768, up to 32: 16.9 against 20.0): the longest item ends sooner.
+//   * Above that four query tiles and one stream (d = 32 held to three waves per SIMD: 3072, 32: 51.5 against 55.8), except
+//     that a ramp up to eight items per CU keeps two streams (d = 64: 2048, up to 64: 68 against 74; d = 32: 2048, up to 128:
+//     74 against 86): there all workgroups are resident at once and the longest ones would end alone. At d = 64 eight query
+//     tiles split K and V half as often, and are taken where their workgroups fill whole rounds of the CUs (2048, 128: 195
+//     against 209; 1536, 32: 47.0 against 51.5; but 3072, 32, one and a half rounds: 97 against 88).
+template<int D, bool VEC>
+void dispatch(const ForwardArgs &a, const Work &w, const int cus, hipStream_t stream) {
+    if (w.items <= 2ll * cus) {
+        if constexpr (D == 32) {
+            if (w.tiles >= 20) return launch<D, VEC, 2, 4>(a, stream);
+        }
+        return launch<D, VEC, 2, 2, D == 32 ? 2 : 1>(a, stream); // d = 64: its 128 KB of LDS admit one workgroup per CU
+    }
+    if (w.items <= 4ll * cus) {
+        if constexpr (D == 32) {
+            if (w.ramp) return launch<D, VEC, 2, 2>(a, stream);
+        }
+        if (w.tiles >= (D == 32 ? 16 : 24)) return launch<D, VEC, 4, 2>(a, stream);
+    } else if (w.ramp && w.items <= 8ll * cus && w.tiles >= (D == 32 ? 32 : 48)) {
+        return launch<D, VEC, 4, 2>(a, stream);
+    }
+    if constexpr (D == 64) {
+        const int64_t wide = static_cast<int64_t>(a.batch) * a.heads * ((a.queries + 8 * kTile - 1) / (8 * kTile));
+        if (w.items > 4ll * cus && !w.ramp && a.radius < 0 && w.tiles >= 24 && (wide <= cus || wide >= 3ll * cus)) return launch<D, VEC, 8, 1>(a, stream);
+    }
+    launch<D, VEC, 4, 1, D == 32 ? 3 : 2>(a, stream);
+}
+
+} // namespace
+
+// Where the items are few, the FP32 kernel's four waves per item and shorter start win: up to one item per CU (d = 64, 128
+// items of 32 tiles: 22.3 against 23.9 µs; d = 32, 32 items of 8: 5.6 against 7.5), under a ramp up to two (d = 64, 384 items
+// of up to 16: 14.1 against 15.7; d = 32: 8.6 against 10.8), and at d = 32 for short items (512 of 5: 7.6 against 8.3; 1536 of
+// 3: 9.9 against 11.7).
+bool forward_split_pays(const int D, const ForwardArgs &a, const int cus) {
+    const Work w = work_of(a);
+    if (w.items <= cus || (w.ramp && w.items < 2ll * cus)) return false;
+    if (D == 64) return true;
+    return w.items <= 2ll * cus ? w.tiles >= 9 : a.radius < 0 || w.tiles >= 5 || w.items >= 16ll * cus;
+}
+
+void launch_forward_split(const int D, const bool vec, const ForwardArgs &a, const int cus, hipStream_t stream) {
+    const Work w = work_of(a);
+    if (D == 32) vec ? dispatch<32, true>(a, w, cus, stream) : dispatch<32, false>(a, w, cus, stream);
+    else vec ? dispatch<64, true>(a, w, cus, stream) : dispatch<64, false>(a, w, cus, stream);
+}
+
+} // namespace rk

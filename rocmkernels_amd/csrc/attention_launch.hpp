@@ -84,6 +84,11 @@ inline unsigned workgroups_for(const long long items, const int split) {
 // Forward pass for head width D (16, 32 or 64). statistics_only writes lse and skips V and the output.
 hipError_t launch_forward(int D, bool statistics_only, const ForwardArgs &a, hipStream_t stream);
 
+// FP32 forward on the fp16 matrix cores (attention_forward_split.hip), D = 32 or 64: whether it is the faster one for the
+// call, and its launch (vec: every pointer 16-byte aligned, every stride a multiple of 4).
+bool forward_split_pays(int D, const ForwardArgs &a, int cus);
+void launch_forward_split(int D, bool vec, const ForwardArgs &a, int cus, hipStream_t stream);
+
 struct RotaryArgs {
     const float *q, *k, *cos, *sin;
     float *oq, *ok;

@@ -1,0 +1,64 @@
+// FP32 matrix products on the fp16 matrix cores: every FP32 operand, scaled by a power of two, is split into two fp16 terms
+// and the product is summed from three fp16 products.
+//
+// x·2^s = h + l + e with h = fp16(x·2^s) and l = fp16(x·2^s - h), each rounded to nearest even: 22 significant bits and a
+// sign, |e| <= 2^-23 of |x·2^s| while l is a normal number (|x·2^s| >= 2^-3), and at most 2^-25 below that. x·y is then
+// hl + lh + hh; the term left out, ll, is below 2^-22 of |x·y|. fp16 products are exact in FP32, and
+// v_mfma_f32_32x32x16_f16 adds 16 of them per accumulator rounding, so a dot product rounds far less often than on
+// v_mfma_f32_32x32x2f32, which more than makes up for the two bits.
+//
+// The scales put the largest magnitude of an operand's rows at 2^8 or more, so what is lost below 2^-3 is at most 2^-33 of it,
+// far below FP32's own rounding of the sums that the small elements share with the large ones.
+//
+// An element that is not finite, or that passes 65504 after scaling, has h = ±inf and l = ∓inf or NaN: every result that it
+// enters is NaN (inf - inf, or 0·inf), never a wrong number. Callers test their results and compute again with FP32 MFMAs
+// where they find one.
+//
+// Cost: v_mfma_f32_32x32x16_f16 does 16 times the work of an FP32 MFMA per cycle, so three products take 3/16 of its time,
+// and unlike FP32 MFMAs they co-execute with VALU work. Splitting takes 2.5 VALU instructions per element (1.5
+// unscaled): v_fma_mixlo/mixhi_f16 scale, subtract and round in one. (Three bf16 terms and six products need no scale, but at twice the
+// MFMAs, 5.5 instructions per element and half as much LDS traffic again: the 64 x 1024 x 64 forward took 84 µs so.)
+#pragma once
+
+#include "attention_device.hpp"
+
+namespace rk {
+
+typedef _Float16 h16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 h16x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 h16x2 __attribute__((ext_vector_type(2)));
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ f32x16 mfma_f16(const h16x8 a, const h16x8 b, const f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+}
+
+// The two terms of a pair of floats times `scale` (a power of two), packed; SCALED = false takes them as they are. The high
+// terms are hidden from the compiler between their conversion and their use: it otherwise converts the two again one by one
+// (and, unscaled, turns each fused subtraction into a conversion and a subtraction).
+template<bool SCALED>
+__device__ __forceinline__ void split_pair(const float a, const float b, const float scale, uint32_t &h, uint32_t &l) {
+    h = __builtin_bit_cast(uint32_t, __builtin_convertvector((SCALED ? f32x2{a * scale, b * scale} : f32x2{a, b}), h16x2));
+    __asm__("" : "+v"(h));
+    const h16x2 hi = __builtin_bit_cast(h16x2, h);
+    const h16x2 lo{static_cast<_Float16>(fmaf(a, scale, -static_cast<float>(hi[0]))),
+            static_cast<_Float16>(fmaf(b, scale, -static_cast<float>(hi[1])))};
+    l = __builtin_bit_cast(uint32_t, lo);
+}
+
+// 1.0 in a scalar register, the scale of an unscaled split (as a constant it would fold the fused subtraction away).
+__device__ __forceinline__ float split_unit_scale() {
+    float one = 1.0f;
+    __asm__("" : "+s"(one));
+    return one;
+}
+
+// Exponent e of a non-zero magnitude in [2^e, 2^(e + 1)); 0 for zero (denormals count as 2^-127).
+__device__ __forceinline__ int exponent_of(const float magnitude) {
+    return magnitude > 0.0f ? static_cast<int>(__float_as_uint(magnitude) >> 23) - 127 : 0;
+}
+
+// 2^e for e in -126 .. 127.
+__device__ __forceinline__ float power_of_two(const int e) { return __uint_as_float(static_cast<uint32_t>(e + 127) << 23); }
+
+} // namespace rk

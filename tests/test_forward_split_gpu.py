@@ -1,0 +1,99 @@
+"""GPU parity of the split-product FP32 forward (attention_forward_split.hip): every workgroup shape at ragged sizes, with
+padding, radius windows and unaligned views, against the CPU oracle; magnitudes far from 1, rows that leave the sampled
+range, infinities and NaN, where the kernel hands query tiles to FP32 MFMAs."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from parity import check_forward, host, normal_case, padding_mask, to_dev
+from rocmkernels_amd import attention
+
+pytestmark = pytest.mark.gpu
+
+# (width, batch, heads, queries, keys, radius, causal): each workgroup shape on a 256-CU device, sizes off every tile edge.
+SHAPES = [
+    (32, 8, 1, 2043, 2043, -1, True),     # two query tiles, four key streams
+    (32, 24, 1, 500, 470, -1, False),     # two and two
+    (32, 24, 1, 1000, 1000, -1, True),    # two and two, causal ramp
+    (32, 24, 1, 1001, 999, -1, False),    # four and two
+    (32, 48, 2, 515, 515, 100, True),     # four and one
+    (64, 24, 1, 500, 530, -1, False),     # two and two
+    (64, 24, 1, 1001, 799, -1, False),    # four and two
+    (64, 64, 1, 1000, 1030, -1, False),   # eight and one
+    (64, 48, 2, 515, 515, 77, False),     # four and one
+    (64, 17, 1, 1023, 33, -1, False),     # fewer keys than one 64-key step
+]
+
+
+@pytest.mark.parametrize("aligned", [True, False])
+@pytest.mark.parametrize("width,batch,heads,queries,keys,radius,causal", SHAPES)
+def test_workgroup_shapes_match_oracle(device, width, batch, heads, queries, keys, radius, causal, aligned):
+    q, k, v, _ = normal_case(300 + width + queries, width, batch, heads, queries, keys)
+    mask = padding_mask(301, batch, keys, keys // 2)
+    mask[0, :40] = 0
+    k[0, :, :40] = np.inf  # masked keys: whatever they hold
+    v[0, :, :40] = np.nan
+    want = oracle.attention(q, np.nan_to_num(k, posinf=0.0), np.nan_to_num(v), mask, radius=radius, causal=causal)
+    tensors = to_dev(device, q, k, v)
+    if not aligned:  # one float past alignment: the 32-bit load path
+        tensors = [torch.cat([t.new_zeros(1), t.reshape(-1)])[1:].view(t.shape) for t in tensors]
+    out, lse = attention.forward(*tensors, *to_dev(device, mask), radius=radius, causal=causal)
+    check_forward(*host(out, lse), want, f"split d{width}")
+
+
+@pytest.mark.parametrize("width", [32, 64])
+@pytest.mark.parametrize("gain_q,gain_k,gain_v", [(1e-12, 1e12, 1e-20), (3e15, 1e-15, 1e25), (1.0, 1.0, 1e-33), (1e-20, 1e-20, 1e35)])
+def test_magnitudes(device, width, gain_q, gain_k, gain_v):
+    # Powers of two keep the scaled problem's exact results: O scales with V, scores with Q and K.
+    q, k, v, _ = normal_case(310, width, 24, 1, 480, 480)
+    q, k, v = (x * np.float32(2.0 ** np.round(np.log2(g))) for x, g in ((q, gain_q), (k, gain_k), (v, gain_v)))
+    mask = np.ones((24, 480), np.uint8)
+    out, lse = host(*attention.forward(*to_dev(device, q, k, v, mask)))
+    unit = np.float64(2.0 ** np.round(np.log2(gain_v)))
+    want = oracle.attention(q, k, (v / unit).astype(np.float32), mask)
+    check_forward(out.astype(np.float64) / unit, lse, want, f"gains {gain_q} {gain_k} {gain_v}")
+
+
+@pytest.mark.parametrize("width", [32, 64])
+def test_rows_beyond_the_sampled_range(device, width):
+    # Two keys and a value row thousands of times larger than the rows around them.
+    q, k, v, _ = normal_case(320, width, 24, 1, 480, 480)
+    k[3, 0, 101] *= 3e4
+    v[5, 0, 257] *= 1e6
+    mask = np.ones((24, 480), np.uint8)
+    want = oracle.attention(q, k, v, mask)
+    out, lse = host(*attention.forward(*to_dev(device, q, k, v, mask)))
+    # Against the largest magnitude of each sequence: FP32 scores of thousands round to about 1e-3 (sequence 3 is compared
+    # where the large key's weight is exactly 0 or 1 to that rounding, by its row maxima).
+    for b in range(24):
+        scale = np.abs(want["output"][b]).max()
+        if b != 3:
+            assert np.abs(out[b] - want["output"][b]).max() <= 1e-5 * max(1.0, scale), b
+    assert np.abs(lse[..., 0] - want["lse"][..., 0]).max() <= 1e-6 * np.abs(want["lse"][..., 0]).max()
+
+
+@pytest.mark.parametrize("width", [32, 64])
+def test_infinities_and_nan(device, width):
+    q, k, v, _ = normal_case(330, width, 24, 1, 480, 480)
+    q[..., 0] = np.abs(q[..., 0]) + 0.1
+    mask = np.ones((24, 480), np.uint8)
+    clean = oracle.attention(q, k, v, mask)
+    k[2, 0, 7, 0] = -np.inf  # a score of -inf for every query: the key weighs nothing
+    v[4, 0, 9, 3] = np.inf   # one feature of every row
+    v[6, 0, 11, 5] = np.nan
+    q[8, 0, 13, 2] = np.nan  # one row
+    out, lse = host(*attention.forward(*to_dev(device, q, k, v, mask)))
+    without = mask.copy()
+    without[2, 7] = 0
+    keyless = k.copy()
+    keyless[2, 0, 7] = 0
+    want = oracle.attention(q[2:3], keyless[2:3], v[2:3], without[2:3])
+    assert np.abs(out[2] - want["output"][0]).max() <= 1e-5
+    for b, feature, value in ((4, 3, np.inf), (6, 5, np.nan)):
+        others = [f for f in range(width) if f != feature]
+        assert np.array_equal(out[b, ..., feature], np.full_like(out[b, ..., feature], value), equal_nan=True)
+        assert np.abs(out[b][..., others] - clean["output"][b][..., others]).max() <= 1e-5
+    assert np.isnan(out[8, 0, 13]).all() and np.isnan(lse[8, 0, 13]).all()
+    rows = [r for r in range(480) if r != 13]
+    assert np.abs(out[8, 0, rows] - clean["output"][8, 0, rows]).max() <= 1e-5
