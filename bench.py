@@ -386,6 +386,44 @@ def forward_split_kernel_name(cfg, cus):
     return f"rk::attention_forward_split_kernel<{width}, true, {shape[0]}, {shape[1]}, {shape[2]}>"
 
 
+def backward_split_kernel_names(cfg, cus, deterministic):
+    """Names rocprofv3 reports for the split-product dQ and dK/dV instances that run on this config, or None where other
+    kernels run: rk::backward_split_pays, rk::dispatch_dq and rk::dispatch_dkdv
+    (rocmkernels_amd/csrc/attention_backward_split.hip). Template arguments: head width, 16-byte vector loads, tiles per
+    workgroup, streams."""
+    width, length, radius = cfg["width"], cfg["length"], cfg["radius"]
+    tiles = (length + 31) // 32
+    items = tiles * cfg["batch"] * cfg["heads"]
+    ramp = radius < 0 or radius >= length // 2  # every config is causal
+
+    def keys_of(qt):  # 32-key tiles a query tile sees
+        return -(-(min(length, 32 * qt + 32) - (max(0, 32 * qt - radius) if radius >= 0 else 0)) // 32)
+
+    def queries_of(kt):  # 32-query tiles that see a key tile
+        return -(-((min(length, 32 * kt + 32 + radius) if radius >= 0 else length) - 32 * kt) // 32)
+
+    dq, dkdv = max(keys_of(tiles // 2), keys_of(tiles - 1)), max(queries_of(0), queries_of(tiles // 2))
+    widest = max(dq, dkdv)
+    if not (deterministic and widest >= 32):
+        if items <= cus:
+            return None
+        if ramp and width == 32 and (deterministic or radius >= 0) and items < 2 * cus:
+            return None
+        if ramp and width == 64 and not (items > 2 * cus or widest <= 4 or (deterministic and radius < 0)):
+            return None
+    if (dq > 2) if items <= 2 * cus else (ramp and items <= 4 * cus and dq >= width // 2):
+        first = (2, 2)
+    else:
+        first = (4, 2) if dq >= 64 and items <= (8 if ramp else 4) * cus else (4, 1)
+    second = (4, 1)
+    if items <= 2 * cus:
+        second = (2, 4) if dkdv >= 16 else (2, 2) if dkdv > 2 else (4, 1)
+    elif (width == 32 or dkdv > 4) if items <= 4 * cus else (ramp and items <= 8 * cus and dkdv >= width // 2):
+        second = (4, 2) if width == 64 or (not ramp and dkdv >= 16) else (2, 2)
+    return [f"rk::attention_{name}_split_kernel<{width}, true, {shape[0]}, {shape[1]}>"
+            for name, shape in (("dq", first), ("dkdv", second))]
+
+
 def traffic_table():
     path = os.path.join(ROOT, "profiles", "traffic.json")
     if not os.path.exists(path):
@@ -404,16 +442,17 @@ def load_traffic(kernel, config):
     return traffic_table().get(f"{kernel} config{profile_config(config)}", {}).get("hbm_bytes_per_launch")
 
 
-def backward_traffic(config, part):
-    """HBM and algorithmic bytes per launch of the kernels one backward call runs, from profiles/traffic.json: the fused
-    pre-pass and the fused (no radius window) or band kernel (radius window) for the default backward, which the library
-    takes for inputs with 128-bit access, as every bench input has (rk::run in attention_backward.hip); the dQ and
-    dK/dV kernels for the deterministic backward."""
+def backward_traffic(config, part, names=None):
+    """HBM and algorithmic bytes per launch of the kernels one backward call runs, from profiles/traffic.json, or None.
+    ``names``: those of backward_split_kernel_names. Without it, the kernels that run where the split pair does not pay: the
+    fused pre-pass and the fused (no radius window) or band kernel (radius window) for the default backward with 128-bit
+    access (rk::run in attention_backward.hip), the FP32 dQ and dK/dV kernels for the deterministic one."""
     suffix = f" config{profile_config(config)}"
-    rows = {k[:-len(suffix)]: v for k, v in traffic_table().items() if k.endswith(suffix) and "forward_kernel" not in k}
-    fused = part == "backward"
-    names = sorted(n for n in rows if ("fused" in n or "band" in n) == fused)
-    if not names:
+    rows = {k[:-len(suffix)]: v for k, v in traffic_table().items() if k.endswith(suffix)}
+    if names is None:
+        fused = part == "backward"
+        names = sorted(n for n in rows if "forward" not in n and "split" not in n and ("fused" in n or "band" in n) == fused)
+    if not names or any(n not in rows for n in names):
         return None
     return {"kernels": names, "hbm_bytes_per_launch": sum(rows[n]["hbm_bytes_per_launch"] for n in names),
             "algorithmic_bytes_per_launch": sum(rows[n]["algorithmic_bytes_per_launch"] for n in names)}
@@ -447,7 +486,7 @@ def measure(cfg, steps, warmup, backward=True, forward_timed=True):
     def forward():
         attention.forward(q, k, v, mask, radius=cfg["radius"], causal=True, output=out, lse=lse)
 
-    def backward_step():  # the _ex default: the faster backward for the call (fused where it exists)
+    def backward_step():  # the _ex default: the faster backward for the call
         attention.backward(q, k, v, mask, out, lse, du, radius=cfg["radius"], causal=True, grads=grads)
 
     def backward_deterministic():
@@ -722,7 +761,8 @@ def main():
     for part in ("backward", "backward_deterministic"):
         if part in measured:
             result[part] = rounded(measured[part])
-            result[part]["traffic"] = backward_traffic(args.config, part)
+            names = backward_split_kernel_names(cfg, cus, part == "backward_deterministic")
+            result[part]["traffic"] = backward_traffic(args.config, part, names)
     result["rotary"] = measure_rotary(cfg, args.steps, args.warmup)
     result["generic_forward"] = measure_generic(cfg, args.steps)
     if args.config == 2:

@@ -31,10 +31,12 @@
  *     accumulated with FP32 atomics, and so are dK/dV of the key blocks whose query range is split over several
  *     workgroups, so those values' low-order bits may differ from run to run (delta is bit-reproducible);
  *   - deterministic: the reference's arrangement, a query-major dQ kernel and a key-major dK/dV kernel (7 matrix
- *     products per tile, S and dP computed in both); bit-identical results run to run.
- *   With neither bit 1 nor bit 2 set the library takes the faster one for the call: fused for inputs with 128-bit
- *   access (16-byte aligned pointers, strides multiples of 4), under a radius window the band kernel when there are at
- *   least 5/8 as many 128-key blocks (batch x heads x ceil(keys / 128)) as compute units; deterministic otherwise.
+ *     products per tile, S and dP computed in both); bit-identical results run to run. Where there is enough work its
+ *     products are formed from fp16 products of two-term operands, with no larger errors than FP32 ones.
+ *   With neither bit 1 nor bit 2 set the library takes the faster one for the call: deterministic from about one
+ *   32-row tile of queries and keys per compute unit on; below that fused for inputs with 128-bit access (16-byte
+ *   aligned pointers, strides multiples of 4), under a radius window the band kernel when there are at least 5/8 as many
+ *   128-key blocks (batch x heads x ceil(keys / 128)) as compute units, and deterministic otherwise.
  *   Bit 1 (ROCMKERNELS_ATTENTION_FUSED_BACKWARD) asks for fused wherever it exists (inputs with 128-bit access); bit 2
  *   (ROCMKERNELS_ATTENTION_DETERMINISTIC) asks for deterministic. Setting both, or any other bit, returns
  *   hipErrorInvalidValue.

@@ -227,8 +227,8 @@ def backward(q, k, v, mask, output, lse, upstream, radius=-1, causal=False, entr
     """dQ, dK, dV, delta of attention; gradients packed [B][H][L][D], delta [B][H][Lq].
 
     A causal mask, ``entry="ex"``, ``fused`` or ``deterministic`` go through the *_ex entry points, whose default
-    takes the faster backward for the call (the fused one, whose dQ is accumulated with atomics, for 128-bit aligned
-    inputs); ``fused`` asks for the fused backward, ``deterministic`` for the bit-reproducible two-kernel one. Otherwise
+    takes the faster backward for the call (for small launches of 128-bit aligned inputs the fused one, whose dQ is
+    accumulated with atomics); ``fused`` asks for the fused backward, ``deterministic`` for the bit-reproducible two-kernel one. Otherwise
     ``entry`` picks the reference entry point ("simple", "tiled", "tuned", "profile", "query_profile"), which always
     runs the deterministic kernels."""
     torch = _torch()

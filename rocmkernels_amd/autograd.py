@@ -6,8 +6,8 @@ the ctypes binding).
 ``attention_fp32(q, k, v, mask, radius, causal)`` returns O = softmax(QKᵀ/√D + mask) V for q/k/v [B][H][L][D]
 float32 CUDA tensors (D = 32 or 64). The forward keeps O and the {max, sum} statistics; the backward runs the
 library's *_ex backward entry point on them. Which backward: ``deterministic=True`` the bit-reproducible two-kernel
-one, ``deterministic=False`` the faster one for the call (the fused one, whose dQ is accumulated with atomics, for
-128-bit aligned inputs); left at None, the bit-reproducible one exactly when torch's deterministic mode is on
+one, ``deterministic=False`` the faster one for the call (for small launches of 128-bit aligned inputs the fused one,
+whose dQ is accumulated with atomics); left at None, the bit-reproducible one exactly when torch's deterministic mode is on
 (``torch.use_deterministic_algorithms(True)``).
 Everything runs on the GPU through the C ABI; there is no CPU path.
 """

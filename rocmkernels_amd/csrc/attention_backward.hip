@@ -17,6 +17,9 @@
 // (Attention.hip:211-221). Streamed operands are read through buffer resources (see attention_device.hpp), and
 // each tile's row-layout operands are loaded one tile ahead, after the current tile's MFMAs are issued.
 //
+// They run where the pair on the fp16 matrix cores (attention_backward_split.hip) does not pay: launches of few tiles, and the
+// stages of the profile entry points.
+//
 // Per-key-tile fused variant (the fused flag's choice for inputs without 128-bit access; with it the key-block kernels
 // of attention_backward_fused.hip and attention_backward_band.hip run): kernel 1 only computes δ and zeroes dQ;
 // kernel 2 also forms dQ = dS·K/√D for each tile it visits and adds it into dQ with FP32 atomics. That is 5
@@ -821,16 +824,14 @@ template<int D, bool VEC>
 hipError_t run(BackwardStage stage, const BackwardArgs &a, const int cus, hipStream_t stream) {
     const int64_t kitems = static_cast<int64_t>((a.keys + kTile - 1) / kTile) * a.batch * a.heads;
     const int64_t kblocks = static_cast<int64_t>((a.keys + kBlockKeys - 1) / kBlockKeys) * a.batch * a.heads;
-    // The fused key-block kernels need 128-bit access; without it the deterministic kernels measured faster.
-    // Auto takes the fused kernels wherever they exist (128-bit access): under a radius window the band kernel against
-    // the deterministic pair, causal, measured 146.4 against 160.3 us at D = 32 (16 sequences x 8192 tokens, radius
-    // 256), 124.9 against 147.8 us (32 x 2048, radius 512), 101.9 against 103.4 us (32 x 4096, radius 128), and 258
-    // against 287 us at D = 64 (config 5). The band kernel runs one persistent workgroup per 128-key block and never
-    // splits a block, so with fewer blocks than a grid that fills the CUs it leaves them idle while the deterministic
-    // pair spreads 32-row tiles over every CU: measured, causal, 1 x 8192 at D = 64, radius 256 (64 blocks) 64.9
-    // against 40.0 us, 2 x 8192 (128 blocks) 67.5 against 59.0 us, 4 x 8192 (256 blocks) 74.0 against 105.8 us; at
-    // D = 32, 64 / 128 / 256 blocks 38.0 / 39.1 / 42.4 against 22.2 / 32.0 / 58.3 us. So under a radius window Auto
-    // takes the band kernel only from kBandMinBlocksPerCu blocks per CU.
+    // Auto and the deterministic backward take the pair on the fp16 matrix cores wherever it pays (backward_split_pays: more
+    // than about one 32-row item per CU). Below, Auto takes the fused kernels wherever they exist (128-bit access; without it
+    // the deterministic FP32 pair measured faster), under a radius window only if they fill the CUs: the band kernel runs one
+    // persistent workgroup per 128-key block and never splits a block, while the pair spreads 32-row tiles over every CU:
+    // measured, causal, 1 x 8192 at D = 64, radius 256 (64 blocks) 64.9 against 40.0 us, 2 x 8192 (128 blocks) 67.5 against
+    // 59.0 us; at D = 32, 64 / 128 blocks 38.0 / 39.1 against 22.2 / 32.0 us; 256 blocks 42.4 against 58.3.
+    if ((stage == kBackwardAuto || stage == kBackwardAll) && backward_split_pays(D, a, cus, VEC, stage == kBackwardAll || !VEC))
+        return launch_backward_split(D, VEC, a, cus, stream);
     if (stage == kBackwardAuto) {
         const bool band_fills = a.radius < 0 || kblocks * kBandMinBlocksPerCu.den >= static_cast<int64_t>(cus) * kBandMinBlocksPerCu.num;
         stage = VEC && band_fills ? kBackwardFused : kBackwardAll;

@@ -28,7 +28,6 @@ namespace rk {
 
 namespace {
 
-constexpr int kMaxExponent = 100; // largest scale exponent: 2^±100 times a sum of products stays far inside FP32's range
 constexpr int kStep = 2 * kTile;  // keys of a step
 
 struct SplitForwardParams {
@@ -52,20 +51,6 @@ __device__ __forceinline__ int k_chunk(const int r, const int c) {
 template<int D>
 __device__ __forceinline__ int v_chunk(const int r, const int c) {
     return r * D + 8 * (D == 64 ? c ^ (2 * (r & 3)) : c);
-}
-
-// Calls f(0), .., f(N - 1) with compile-time indexes.
-template<int N, int I = 0, class F>
-__device__ __forceinline__ void unrolled(const F &f) {
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        unrolled<N, I + 1>(f);
-    }
-}
-
-__device__ __forceinline__ u32x2 read_transposed(const uint16_t *p) {
-    typedef short v4s __attribute__((ext_vector_type(4)));
-    return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s *)(p)));
 }
 
 // Writes the output rows and statistics of a wave's query tile: state (m_raw, l) with l summed over both half-waves, O

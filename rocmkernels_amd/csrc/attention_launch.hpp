@@ -113,6 +113,12 @@ enum BackwardStage {
 
 hipError_t launch_backward(int D, BackwardStage stage, const BackwardArgs &a, hipStream_t stream);
 
+// Deterministic FP32 backward on the fp16 matrix cores (attention_backward_split.hip), D = 32 or 64: whether it is faster for
+// the call than the deterministic FP32 pair (deterministic) or what kBackwardAuto would run instead, and its launch (vec: every
+// pointer 16-byte aligned, every stride a multiple of 4).
+bool backward_split_pays(int D, const BackwardArgs &a, int cus, bool vec, bool deterministic);
+hipError_t launch_backward_split(int D, bool vec, const BackwardArgs &a, int cus, hipStream_t stream);
+
 // Fused single-kernel backward over key blocks (attention_backward_fused.hip) for D = 32 or 64 with 128-bit access
 // (every pointer 16-byte aligned, every stride a multiple of 4); called by launch_backward for kBackwardFused.
 hipError_t launch_fused_backward(int D, const BackwardArgs &a, int cus, hipStream_t stream);

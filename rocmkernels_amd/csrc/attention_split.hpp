@@ -20,6 +20,8 @@
 // MFMAs, 5.5 instructions per element and half as much LDS traffic again: the 64 x 1024 x 64 forward took 84 µs so.)
 #pragma once
 
+#include <type_traits>
+
 #include "attention_device.hpp"
 
 namespace rk {
@@ -60,5 +62,56 @@ __device__ __forceinline__ int exponent_of(const float magnitude) {
 
 // 2^e for e in -126 .. 127.
 __device__ __forceinline__ float power_of_two(const int e) { return __uint_as_float(static_cast<uint32_t>(e + 127) << 23); }
+
+constexpr int kMaxExponent = 100; // largest scale exponent: 2^±100 times a sum of products stays far inside FP32's range
+
+// 2^-e, e clamped to the exponents a scale may have (beyond them callers use FP32 MFMAs).
+__device__ __forceinline__ float scale_down(const int e) { return power_of_two(-min(max(e, -kMaxExponent), kMaxExponent)); }
+__device__ __forceinline__ bool scale_fits(const int e) { return e >= -kMaxExponent && e <= kMaxExponent; }
+
+__device__ __forceinline__ float largest(const f32x4 x) { return fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3]))); }
+
+// Eight floats times `scale` as an operand's two terms.
+__device__ __forceinline__ void split_operand(const f32x4 x, const f32x4 y, const float scale, h16x8 &high, h16x8 &low) {
+    u32x4 hi, lo;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        uint32_t h, l;
+        split_pair<true>(x[2 * j], x[2 * j + 1], scale, h, l);
+        hi[j] = h;
+        lo[j] = l;
+        split_pair<true>(y[2 * j], y[2 * j + 1], scale, h, l);
+        hi[2 + j] = h;
+        lo[2 + j] = l;
+    }
+    high = __builtin_bit_cast(h16x8, hi);
+    low = __builtin_bit_cast(h16x8, lo);
+}
+
+// Calls f(0), .., f(N - 1) with compile-time indexes.
+template<int N, int I = 0, class F>
+__device__ __forceinline__ void unrolled(const F &f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        unrolled<N, I + 1>(f);
+    }
+}
+
+// Transposing LDS read: lane L of each 16-lane group points at row L / 4 of four rows, elements 4 (L mod 4) .. + 3 of their
+// sixteen, and receives element L of the four rows.
+__device__ __forceinline__ u32x2 read_transposed(const uint16_t *p) {
+    typedef short v4s __attribute__((ext_vector_type(4)));
+    return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s *)(p)));
+}
+
+// Position (in 2-byte elements) of element 0 of 16-byte chunk c of row r in a staged plane of D columns that is read both by
+// rows (16 lanes: 16 rows, one chunk each) and transposed (32 lanes: 4 rows of 64 bytes). Rows are unpadded; their chunks are
+// permuted so that either read meets every bank once: at D = 64 (8 chunks, two rows to the 64 banks) the even and the odd
+// rows of 16 take all eight permutations, and rows r and r + 2 of four lie in different halves of their row.
+template<int D>
+__device__ __forceinline__ int staged_chunk(const int r, const int c) {
+    const int swizzle = D == 64 ? ((r & 2) << 1 | (r & 4) >> 1 | (r & 8) >> 3) : ((r >> 2) & 3);
+    return r * D + 8 * (c ^ swizzle);
+}
 
 } // namespace rk

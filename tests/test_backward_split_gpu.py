@@ -1,0 +1,106 @@
+"""GPU parity of the split-product FP32 backward (attention_backward_split.hip): every workgroup shape of both kernels at ragged
+sizes, with padding, garbage behind the mask, radius windows and unaligned views, against the CPU oracle; magnitudes far from
+1, rows that leave the sampled range, infinities and NaN, where the kernels hand tiles to FP32 MFMAs; bit-reproducibility."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from parity import check_backward, host, normal_case, padding_mask, to_dev
+from rocmkernels_amd import attention
+
+pytestmark = pytest.mark.gpu
+
+# (width, batch, heads, queries, keys, radius, causal), sizes off every tile edge. Behind each: query tiles and key streams of
+# the dQ kernel's workgroups, key tiles and query streams of the dK/dV kernel's, on a 256-CU device.
+SHAPES = [
+    (32, 12, 1, 1003, 999, -1, False),    # 2 x 2, 2 x 4
+    (32, 24, 1, 500, 333, -1, False),     # 2 x 2, 2 x 2
+    (32, 24, 1, 1001, 1001, -1, True),    # 2 x 2, 2 x 2, causal ramp
+    (32, 9, 1, 2900, 2001, -1, False),    # 4 x 2, 4 x 2
+    (32, 48, 2, 515, 515, 100, True),     # 4 x 1, 4 x 1
+    (32, 300, 1, 61, 35, -1, False),      # 4 x 1, 4 x 1: a tile or two per item
+    (64, 12, 1, 1003, 999, -1, False),    # 2 x 2, 2 x 4
+    (64, 24, 1, 500, 333, -1, False),     # 2 x 2, 2 x 2
+    (64, 11, 1, 2100, 2055, -1, True),    # 2 x 2, 4 x 2, causal ramp
+    (64, 9, 1, 2900, 2001, -1, False),    # 4 x 2, 4 x 2
+    (64, 48, 2, 515, 515, 77, False),     # 4 x 1, 4 x 1
+    (64, 300, 1, 35, 61, -1, True),       # 4 x 1, 4 x 1
+]
+
+
+def gradients(device, q, k, v, du, mask, radius=-1, causal=False, aligned=True):
+    tensors = to_dev(device, q, k, v, du)
+    if not aligned:  # one float past alignment: the 32-bit load path
+        tensors = [torch.cat([t.new_zeros(1), t.reshape(-1)])[1:].view(t.shape) for t in tensors]
+    tq, tk, tv, tdu = tensors
+    (tm,) = to_dev(device, mask)
+    out, lse = attention.forward(tq, tk, tv, tm, radius=radius, causal=causal)
+    run = lambda: attention.backward(tq, tk, tv, tm, out, lse, tdu, radius=radius, causal=causal, deterministic=True)  # noqa: E731
+    first, second = run(), run()
+    assert all(torch.equal(a.view(torch.int32), b.view(torch.int32)) for a, b in zip(first, second)), "not bit-reproducible"
+    return host(*first)
+
+
+@pytest.mark.parametrize("aligned", [True, False])
+@pytest.mark.parametrize("width,batch,heads,queries,keys,radius,causal", SHAPES)
+def test_workgroup_shapes_match_oracle(device, width, batch, heads, queries, keys, radius, causal, aligned):
+    q, k, v, du = normal_case(400 + width + queries, width, batch, heads, queries, keys)
+    mask = padding_mask(401, batch, keys, keys // 2)
+    mask[0, :33] = 0
+    clean = k.copy(), v.copy()
+    k[0, :, :33] = np.inf  # masked keys: whatever they hold
+    v[0, :, :33] = np.nan
+    want = oracle.attention(q, *clean, mask, upstream=du, radius=radius, causal=causal)
+    gq, gk, gv, delta = gradients(device, q, k, v, du, mask, radius, causal, aligned)
+    check_backward(gq, gk, gv, delta, want, f"split d{width}")
+    assert not gk[0, :, :33].any() and not gv[0, :, :33].any()
+
+
+@pytest.mark.parametrize("width", [32, 64])
+@pytest.mark.parametrize("eq,ev,eu", [(-40, -40, 27), (48, 30, -83), (0, -100, 0)])
+def test_magnitudes(device, width, eq, ev, eu):
+    # Powers of two scale the problem exactly: dQ and dK by those of K or Q, V and dO, dV by that of dO; scores keep theirs.
+    q, k, v, du = normal_case(410, width, 24, 1, 480, 480)
+    mask = np.ones((24, 480), np.uint8)
+    want = oracle.attention(q, k, v, mask, upstream=du)
+    scaled = [np.ldexp(x, e).astype(np.float32) for x, e in ((q, eq), (k, -eq), (v, ev), (du, eu))]
+    gq, gk, gv, _ = gradients(device, *scaled, mask)
+    check_backward(np.ldexp(gq.astype(np.float64), eq - ev - eu), np.ldexp(gk.astype(np.float64), -eq - ev - eu),
+                   np.ldexp(gv.astype(np.float64), -eu), None, want, f"2^{eq} 2^{ev} 2^{eu}")
+
+
+@pytest.mark.parametrize("width", [32, 64])
+def test_rows_beyond_the_sampled_range(device, width):
+    # One row of each operand thousands of times larger than those around it.
+    q, k, v, du = normal_case(420, width, 24, 1, 480, 480)
+    v[2, 0, 257] *= 1e6
+    du[4, 0, 101] *= 1e6
+    k[6, 0, 33] *= 1e-7
+    q[8, 0, 400] *= 30.0
+    mask = np.ones((24, 480), np.uint8)
+    want = oracle.attention(q, k, v, mask, upstream=du)
+    gq, gk, gv, _ = gradients(device, q, k, v, du, mask)
+    for b in range(24):  # each sequence against its own largest gradient, at the normwise bound
+        for name, got in (("gq", gq), ("gk", gk), ("gv", gv)):
+            assert np.abs(got[b] - want[name][b]).max() <= 1e-4 * np.abs(want[name][b]).max(), (b, name)
+
+
+@pytest.mark.parametrize("width", [32, 64])
+def test_infinities_and_nan(device, width):
+    q, k, v, du = normal_case(430, width, 24, 1, 480, 480)
+    mask = np.ones((24, 480), np.uint8)
+    want = oracle.attention(q, k, v, mask, upstream=du)
+    du[2, 0, 7, 3] = np.inf  # dO·V and δ of that query are infinite, their differences infinite or NaN; dV's feature is infinite
+    q[4, 0, 13, 2] = np.nan  # that query's row, and every key's dK and dV
+    gq, gk, gv, _ = gradients(device, q, k, v, du, mask)
+    rows = [r for r in range(480) if r != 7]
+    others = [f for f in range(width) if f != 3]
+    assert np.isnan(gq[2, 0, 7]).all() and not np.isfinite(gk[2]).any() and np.isinf(gv[2, ..., 3]).all()
+    assert np.abs(gq[2, 0, rows] - want["gq"][2, 0, rows]).max() <= 1e-4 * np.abs(want["gq"]).max()
+    assert np.abs(gv[2][..., others] - want["gv"][2][..., others]).max() <= 1e-4 * np.abs(want["gv"]).max()
+    rows = [r for r in range(480) if r != 13]
+    assert np.isnan(gq[4, 0, 13]).all() and np.isnan(gk[4]).all() and np.isnan(gv[4]).all()
+    assert np.abs(gq[4, 0, rows] - want["gq"][4, 0, rows]).max() <= 1e-4 * np.abs(want["gq"]).max()
+    clean = [b for b in range(24) if b not in (2, 4)]
+    check_backward(gq[clean], gk[clean], gv[clean], None, {n: want[n][clean] for n in ("gq", "gk", "gv")}, "beside infinities")
