@@ -9,6 +9,7 @@ conveniences over the same calls; they never compute anything on the host and ra
 or a tensor is not on the GPU.
 """
 import ctypes
+import functools
 import os
 
 LIBRARY_NAME = "libROCmKernels.Kernels.Shared.so"
@@ -100,38 +101,64 @@ def check(name, *args):
 
 
 # ---- torch conveniences -------------------------------------------------------------------------------------
+# A small launch is bound by what is done here per call, so that is little: pointers and the stream pass as integers, the
+# strides of a tensor are read once and their structs shared by value. Host time of a call that allocates nothing: forward 7.0
+# µs (13.2 with an object per argument and per stream), rotary 6.5 (12.7); of a backward with its buffers 15.9 (23.0).
 
 
+@functools.lru_cache(maxsize=None)
 def _torch():
     import torch
 
     return torch
 
 
+@functools.lru_cache(maxsize=None)
+def _dtypes():
+    torch = _torch()
+    return frozenset((torch.float32, torch.float16, torch.bool, torch.uint8))
+
+
+@functools.lru_cache(maxsize=512)
+def _shared_strides(batch, head, token):
+    return Strides(batch, head, token)
+
+
+def _strides(t):
+    """strides(t) for passing on: the struct is shared between equal strides."""
+    s = t.stride()
+    if len(s) != 4 or s[3] != 1:
+        raise ValueError("expected a [batch][head][token][D] tensor with contiguous features")
+    return _shared_strides(s[0], s[1], s[2])
+
+
 def strides(t):
     """Strides of a 4-D [batch][head][token][D] view with contiguous features."""
-    if t.dim() != 4 or t.stride(3) != 1:
-        raise ValueError("expected a [batch][head][token][D] tensor with contiguous features")
-    return Strides(t.stride(0), t.stride(1), t.stride(2))
+    shared = _strides(t)
+    return Strides(shared.batch, shared.head, shared.token)
 
 
 def _ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def _device_check(*tensors):
+    dtypes = _dtypes()
     for t in tensors:
-        if t is not None and not t.is_cuda:
-            raise ValueError("the attention kernels run on the GPU only; move the tensor to a HIP device")
-        if t is not None and t.dtype not in (_torch().float32, _torch().float16, _torch().bool, _torch().uint8):
-            raise ValueError(f"unsupported dtype {t.dtype}")
+        if t is not None:
+            if not t.is_cuda:
+                raise ValueError("the attention kernels run on the GPU only; move the tensor to a HIP device")
+            if t.dtype not in dtypes:
+                raise ValueError(f"unsupported dtype {t.dtype}")
 
 
 def _stream(stream):
-    torch = _torch()
+    """Handle of ``stream``, by default the current device's current stream (torch.cuda.current_stream() without the object:
+    0.2 µs, 3.0 with it and 15 on autograd's own thread)."""
     if stream is None:
-        stream = torch.cuda.current_stream()
-    return ctypes.c_void_p(stream.cuda_stream)
+        torch_c = _torch()._C
+        return torch_c._cuda_getCurrentRawStream(torch_c._cuda_getDevice())
+    return stream.cuda_stream
 
 
 _FORWARD_NAMES = {
@@ -157,7 +184,7 @@ def forward(q, k, v, mask, radius=-1, causal=False, output=None, lse=None, entry
     if lse is None:
         lse = torch.empty((batch, heads, queries, 2), device=q.device, dtype=torch.float32)
     common = (_ptr(q), _ptr(k), _ptr(v), _ptr(mask), _ptr(output), _ptr(lse), batch, heads, queries, keys, radius)
-    views = (strides(q), strides(k), strides(v), strides(output), _stream(stream))
+    views = (_strides(q), _strides(k), _strides(v), _strides(output), _stream(stream))
     if causal:
         name = "attention_fp32_forward_flash_ex" if width == 32 else "attention64_fp32_forward_ex"
         check(name, *common, CAUSAL, *views)
@@ -182,15 +209,21 @@ def generic_forward(q, k, v, mask, radius=-1, output=None, lse=None, stream=None
         lse = torch.empty((batch, heads, queries, 2), device=q.device, dtype=torch.float32)
     dtype = DTYPE_FLOAT16 if q.dtype == torch.float16 else DTYPE_FLOAT32
     check("attention_generic_forward", _ptr(q), _ptr(k), _ptr(v), _ptr(mask), _ptr(output), _ptr(lse), batch, heads, queries,
-          k.shape[2], width, radius, strides(q), strides(k), strides(v), strides(output), dtype, _stream(stream))
+          k.shape[2], width, radius, _strides(q), _strides(k), _strides(v), _strides(output), dtype, _stream(stream))
     return output, lse
+
+
+def _table_strides(t):
+    s = t.stride()
+    if len(s) != 3 or s[2] != 1:
+        raise ValueError("expected a [batch][token][32] table with contiguous columns")
+    return _shared_strides(s[0], 0, s[1])
 
 
 def table_strides(t):
     """Strides of a [B][L][32] cos/sin table (the head entry is unused)."""
-    if t.dim() != 3 or t.stride(2) != 1:
-        raise ValueError("expected a [batch][token][32] table with contiguous columns")
-    return Strides(t.stride(0), 0, t.stride(1))
+    s = _table_strides(t)
+    return Strides(s.batch, s.head, s.token)
 
 
 def rotary(q, k, cos, sin, backward=False, out_q=None, out_k=None, stream=None):
@@ -206,7 +239,7 @@ def rotary(q, k, cos, sin, backward=False, out_q=None, out_k=None, stream=None):
     if out_k is None:
         out_k = torch.empty((batch, length, heads, 32), device=q.device, dtype=torch.float32)
     check("rotary_fp32", _ptr(q), _ptr(k), _ptr(cos), _ptr(sin), _ptr(out_q), _ptr(out_k), batch, heads, length,
-          1 if backward else 0, strides(q), strides(k), table_strides(cos), table_strides(sin), _stream(stream))
+          1 if backward else 0, _strides(q), _strides(k), _table_strides(cos), _table_strides(sin), _stream(stream))
     return out_q, out_k
 
 
@@ -218,7 +251,7 @@ def statistics(q, k, mask, radius=-1, lse=None, stream=None):
     if lse is None:
         lse = torch.empty((batch, heads, queries, 2), device=q.device, dtype=torch.float32)
     check("attention_fp32_statistics", _ptr(q), _ptr(k), _ptr(mask), _ptr(lse), batch, heads, queries, k.shape[2], radius,
-          strides(q), strides(k), _stream(stream))
+          _strides(q), _strides(k), _stream(stream))
     return lse
 
 
@@ -243,7 +276,7 @@ def backward(q, k, v, mask, output, lse, upstream, radius=-1, causal=False, entr
     gq, gk, gv, delta = grads
     common = (_ptr(q), _ptr(k), _ptr(v), _ptr(mask), _ptr(output), _ptr(lse), _ptr(upstream), _ptr(gq), _ptr(gk), _ptr(gv),
               _ptr(delta), batch, heads, queries, keys, radius)
-    views = (strides(q), strides(k), strides(v), strides(output), strides(upstream), _stream(stream))
+    views = (_strides(q), _strides(k), _strides(v), _strides(output), _strides(upstream), _stream(stream))
     if causal or fused or deterministic or entry == "ex":
         name = "attention_fp32_backward_ex" if width == 32 else "attention64_fp32_backward_ex"
         flags = (CAUSAL if causal else 0) | (FUSED_BACKWARD if fused else 0) | (DETERMINISTIC if deterministic else 0)
