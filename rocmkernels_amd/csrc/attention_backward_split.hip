@@ -17,9 +17,10 @@
 // in kernel 2; dS in units in which |dP - δ| of that size still fits fp16. Whatever leaves the range becomes NaN, and a wave
 // whose gradients are not finite computes its tile again with FP32 MFMAs.
 //
-// What bounds them: issue and power, nearly even. 21 (kernel 1: 18) fp16 MFMAs of 32 x 32 x 16 per 32 x 32 tile and 16 columns
-// of width do what 8 products' worth of FP32 ones did at an eighth of the rate, beside 16 exponentials' and 32 splits' VALU
-// work per lane and the staging; dense fp16 MFMAs alone clock the card down from 2.37 to about 1.8 GHz. Measured, whole
+// What bounds them: 21 fp16 MFMAs of 32 x 32 x 16 per 32 x 32 tile and 16 columns of width in the two (12 and 9) do what 7 x 8 FP32
+// ones of twice the time did, beside 16 exponentials and about 100 other VALU instructions per lane and kernel; at d = 64, 32 x
+// 2048 causal, MFMAs take a third of the SIMD cycles, VALU issue a fifth to a third, and waits a third of the wave cycles: with
+// the terms of two operands and the accumulators in registers only two waves fit a SIMD. Measured, whole
 // backward, against the faster FP32 one before (µs): d = 64, 32 x 2048 causal, padded 390 -> 215 (dQ 91, dK/dV 126), 16 x 8192
 // causal, radius 256 263 -> 174 (71 and 98), 96 x 2048 full 2109 -> 1128; d = 32, 24 x 1024 causal 54.8 -> 46.4 (19.2 and 27.0),
 // full and deterministic 99.6 -> 58.6, 96 x 2048 full 1069 -> 623. Errors against 64 bits fell too (dQ 3e-7, dK and dV 4e-7 to
