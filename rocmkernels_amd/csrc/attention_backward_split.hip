@@ -12,10 +12,10 @@
 // Streams are summed through LDS in a fixed order, so results are bit-identical from run to run.
 //
 // Scales (powers of two): the operands a wave keeps in registers by their own largest magnitude (rows in kernel 1, the
-// workgroup's block in kernel 2), the streamed ones by that of rows sampled over the workgroup's window, as in the forward. P
-// is kept at 2^9 times exp(s - max) in kernel 1 (the row's 1/sum is applied to dQ at the end) and at 2^14 times its value
-// in kernel 2; dS in units in which |dP - δ| of that size still fits fp16. Whatever leaves the range becomes NaN, and a wave
-// whose gradients are not finite computes its tile again with FP32 MFMAs.
+// workgroup's block in kernel 2), the streamed ones by that of rows sampled over the workgroup's window, as in the forward
+// (of all its rows where the sampled ones are 0). P is kept at 2^9 times exp(s - max) in kernel 1 (the row's 1/sum is applied
+// to dQ at the end) and at 2^14 times its value in kernel 2; dS in units in which |dP - δ| of that size still fits fp16.
+// Whatever leaves the range becomes NaN, and a wave whose gradients are not finite computes its tile again with FP32 MFMAs.
 //
 // What bounds them: 21 fp16 MFMAs of 32 x 32 x 16 per 32 x 32 tile and 16 columns of width in the two (12 and 9) do what 7 x 8 FP32
 // ones of twice the time did, beside 16 exponentials and about 100 other VALU instructions per lane and kernel; at d = 64, 32 x
@@ -184,34 +184,6 @@ __device__ __attribute__((noinline)) void exact_dkdv_tile(const SplitBackwardPar
     for (int t = 0; t < DT; ++t) {
         store_tile_row<VEC>(P.dk + krow + 32 * t, acc_k[t], P.scale, h);
         store_tile_row<VEC>(P.dv + krow + 32 * t, acc_v[t], 1.0f, h);
-    }
-}
-
-template<bool VEC>
-__device__ __forceinline__ f32x4 load_chunk(const Buffer r, const uint32_t voffset, const uint32_t soffset) {
-    if constexpr (VEC) return buffer_load4(r, voffset, soffset);
-    else return f32x4{buffer_load(r, voffset, soffset), buffer_load(r, voffset + 4u, soffset), buffer_load(r, voffset + 8u, soffset),
-            buffer_load(r, voffset + 12u, soffset)};
-}
-
-// Largest |x| and |y| over the workgroup's threads (each passes its own), by way of `slots`; contains a barrier.
-template<int WAVES>
-__device__ __forceinline__ void workgroup_largest(float &x, float &y, float (&slots)[2][WAVES]) {
-#pragma unroll
-    for (int m = 1; m < kWave; m <<= 1) {
-        x = fmaxf(x, __shfl_xor(x, m));
-        y = fmaxf(y, __shfl_xor(y, m));
-    }
-    const int wave = threadIdx.x / kWave;
-    if ((threadIdx.x & (kWave - 1)) == 0) {
-        slots[0][wave] = x;
-        slots[1][wave] = y;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int w = 0; w < WAVES; ++w) {
-        x = fmaxf(x, slots[0][w]);
-        y = fmaxf(y, slots[1][w]);
     }
 }
 
@@ -440,6 +412,16 @@ __global__ __launch_bounds__(kWave * QB * KS) __attribute__((amdgpu_waves_per_eu
 
     float mk = seen != 0 ? largest(sk) : 0.0f, mv = seen != 0 ? largest(sv) : 0.0f;
     workgroup_largest(mk, mv, amax);
+    if (n > ROWS && __builtin_amdgcn_readfirstlane(mk == 0.0f || mv == 0.0f)) {
+        window_largest<kWave * QB * KS, CPR>(mk, mv, n, [&](const int r) { return buffer_load_byte(mbuf, static_cast<uint32_t>(ufirst + r)) != 0; },
+                [&](const int r, const bool on, f32x4 &x, f32x4 &y) {
+                    const uint32_t at = 16u * (threadIdx.x % CPR), row = static_cast<uint32_t>(ufirst + r);
+                    x = load_chunk<VEC>(kbuf, on ? row * kstep + at : kNoRow, 0);
+                    y = load_chunk<VEC>(vbuf, on ? row * vstep + at : kNoRow, 0);
+                });
+        __syncthreads(); // amax is read
+        workgroup_largest(mk, mv, amax);
+    }
     const int ek = __builtin_amdgcn_readfirstlane(exponent_of(mk)) - 8; // K = K'·2^ek, V = V'·2^ev, sampled largest at 2^8
     const int ev = __builtin_amdgcn_readfirstlane(exponent_of(mv)) - 8;
 
@@ -741,6 +723,16 @@ __global__ __launch_bounds__(kWave * KB * QS) __attribute__((amdgpu_waves_per_eu
 
     float mq = largest(sq), mu = largest(su);
     workgroup_largest(mq, mu, amax);
+    if (n > ROWS && __builtin_amdgcn_readfirstlane(mq == 0.0f || mu == 0.0f)) {
+        window_largest<kWave * KB * QS, CPR>(mq, mu, n, [&](const int) { return true; },
+                [&](const int r, const bool on, f32x4 &x, f32x4 &y) {
+                    const uint32_t at = 16u * (threadIdx.x % CPR), row = static_cast<uint32_t>(ufirst + r);
+                    x = load_chunk<VEC>(qbuf, on ? row * qstep + at : kNoRow, 0);
+                    y = load_chunk<VEC>(ubuf, on ? row * ustep + at : kNoRow, 0);
+                });
+        __syncthreads(); // amax is read
+        workgroup_largest(mq, mu, amax);
+    }
     const int eq = __builtin_amdgcn_readfirstlane(exponent_of(mq)) - 8; // Q = Q'·2^eq, dO = dO'·2^eu, sampled largest at 2^8
     const int eu = __builtin_amdgcn_readfirstlane(exponent_of(mu)) - 8;
     float mk = 0.0f, mv = 0.0f;
@@ -751,7 +743,15 @@ __global__ __launch_bounds__(kWave * KB * QS) __attribute__((amdgpu_waves_per_eu
     }
     __syncthreads(); // amax is read
     workgroup_largest(mk, mv, amax);
-    const int ek = __builtin_amdgcn_readfirstlane(exponent_of(mk)) - 14, ev = __builtin_amdgcn_readfirstlane(exponent_of(mv)) - 14;
+    const int ek = __builtin_amdgcn_readfirstlane(exponent_of(mk)) - 14;
+    int ev = __builtin_amdgcn_readfirstlane(exponent_of(mv)) - 14;
+    if (__builtin_amdgcn_readfirstlane(mv == 0.0f)) { // dP = 0: the unit of dP - δ below comes from the largest |δ|, put at 2^-3
+        float md = 0.0f, none = 0.0f;
+        for (int r = threadIdx.x; r < n; r += kWave * KB * QS) md = fmaxf(md, fabsf(buffer_load(dbuf, 4u * static_cast<uint32_t>(ufirst + r), 0)));
+        __syncthreads(); // amax is read
+        workgroup_largest(md, none, amax);
+        if (md > 0.0f) ev = __builtin_amdgcn_readfirstlane(exponent_of(md)) - eu - 24;
+    }
     const bool plain = !scale_fits(ek) || !scale_fits(ev) || !scale_fits(eq) || !scale_fits(eu);
     const float qfactor = scale_down(eq), ufactor = scale_down(eu);
     h16x8 kh[KC], kl[KC], vh[KC], vl[KC];

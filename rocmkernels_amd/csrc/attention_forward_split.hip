@@ -15,9 +15,9 @@
 // the order (the compiler's own order puts the MFMAs first, and the two no longer co-execute).
 //
 // Scales (powers of two): each query row its own; K and V one each for the workgroup, from the largest magnitudes of rows
-// sampled over its window. They put those at 2^8, so rows up to 128 times larger than any sampled one are still in range;
-// larger ones make the result NaN, and a wave that finds a non-finite result computes its query tile again with FP32 MFMAs
-// (as it must anyway for infinities, whose meaning the split products lose).
+// sampled over its window (of all its rows where the sampled ones are 0). They put those at 2^8, so rows up to 128 times
+// larger than any sampled one are still in range; larger ones make the result NaN, and a wave that finds a non-finite result
+// computes its query tile again with FP32 MFMAs (as it must anyway for infinities, whose meaning the split products lose).
 #include <algorithm>
 #include <type_traits>
 
@@ -280,24 +280,17 @@ __global__ __launch_bounds__(kWave * QB * KS) __attribute__((amdgpu_waves_per_eu
         load_chunks(vraw, vbuf, vofs, vstep, 0);
         mask0 = load_mask(0);
         __builtin_amdgcn_sched_barrier(0);
-        float mk = fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3])));
-        float mv = fmaxf(fmaxf(fabsf(y[0]), fabsf(y[1])), fmaxf(fabsf(y[2]), fabsf(y[3])));
-        mk = seen != 0 ? mk : 0.0f;
-        mv = seen != 0 ? mv : 0.0f;
-#pragma unroll
-        for (int m = 1; m < kWave; m <<= 1) {
-            mk = fmaxf(mk, __shfl_xor(mk, m));
-            mv = fmaxf(mv, __shfl_xor(mv, m));
-        }
-        if (lane == 0) {
-            amax[0][wave] = mk;
-            amax[1][wave] = mv;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int w = 0; w < QB * KS; ++w) {
-            mk = fmaxf(mk, amax[0][w]);
-            mv = fmaxf(mv, amax[1][w]);
+        float mk = seen != 0 ? largest(x) : 0.0f, mv = seen != 0 ? largest(y) : 0.0f;
+        workgroup_largest(mk, mv, amax);
+        if (n > ROWS && __builtin_amdgcn_readfirstlane(mk == 0.0f || mv == 0.0f)) {
+            window_largest<kWave * QB * KS, CPR>(mk, mv, n, [&](const int r) { return buffer_load_byte(mbuf, static_cast<uint32_t>(ufirst + r)) != 0; },
+                    [&](const int r, const bool on, f32x4 &x, f32x4 &y) {
+                        const uint32_t at = 16u * (threadIdx.x % CPR), row = static_cast<uint32_t>(ufirst + r);
+                        x = load_chunk<VEC>(kbuf, on ? row * kstep + at : kNoRow, 0);
+                        y = load_chunk<VEC>(vbuf, on ? row * vstep + at : kNoRow, 0);
+                    });
+            __syncthreads(); // amax is read
+            workgroup_largest(mk, mv, amax);
         }
         ek = __builtin_amdgcn_readfirstlane(exponent_of(mk)) - 8;
         ev = __builtin_amdgcn_readfirstlane(exponent_of(mv)) - 8;

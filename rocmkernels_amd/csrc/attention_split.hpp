@@ -71,6 +71,64 @@ __device__ __forceinline__ bool scale_fits(const int e) { return e >= -kMaxExpon
 
 __device__ __forceinline__ float largest(const f32x4 x) { return fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3]))); }
 
+template<bool VEC>
+__device__ __forceinline__ f32x4 load_chunk(const Buffer r, const uint32_t voffset, const uint32_t soffset) {
+    if constexpr (VEC) return buffer_load4(r, voffset, soffset);
+    else return f32x4{buffer_load(r, voffset, soffset), buffer_load(r, voffset + 4u, soffset), buffer_load(r, voffset + 8u, soffset),
+            buffer_load(r, voffset + 12u, soffset)};
+}
+
+// Largest |x| and |y| over the workgroup's threads (each passes its own), by way of `slots`; contains a barrier.
+template<int WAVES>
+__device__ __forceinline__ void workgroup_largest(float &x, float &y, float (&slots)[2][WAVES]) {
+#pragma unroll
+    for (int m = 1; m < kWave; m <<= 1) {
+        x = fmaxf(x, __shfl_xor(x, m));
+        y = fmaxf(y, __shfl_xor(y, m));
+    }
+    const int wave = threadIdx.x / kWave;
+    if ((threadIdx.x & (kWave - 1)) == 0) {
+        slots[0][wave] = x;
+        slots[1][wave] = y;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+        x = fmaxf(x, slots[0][w]);
+        y = fmaxf(y, slots[1][w]);
+    }
+}
+
+// The same over every live row of a window of n rows, for a scale that the sampled rows don't tell: they may all be 0 where the
+// others are not (the gradient of one token's loss), and terms of a fixed scale would lose values far below it. A workgroup of
+// THREADS threads reads ROWS rows at a time, CPR 4-float chunks each: live(row) says whether a row counts, load(row, on, a, b)
+// fetches this thread's two chunks of it (zeros unless on). Costs a pass over the window (from L2), taken only where all sampled
+// rows are 0 or masked.
+template<int THREADS, int CPR, class Live, class Load>
+__device__ __forceinline__ void window_largest(float &x, float &y, const int n, const Live &live, const Load &load) {
+    constexpr int ROWS = THREADS / CPR, TRIP = 4;
+#pragma unroll 1
+    for (int r0 = threadIdx.x / CPR; r0 - static_cast<int>(threadIdx.x / CPR) < n; r0 += TRIP * ROWS) {
+        bool on[TRIP], any = false;
+#pragma unroll
+        for (int u = 0; u < TRIP; ++u) on[u] = live(r0 + u * ROWS);
+#pragma unroll
+        for (int u = 0; u < TRIP; ++u) {
+            on[u] = on[u] && r0 + u * ROWS < n;
+            any = any || on[u];
+        }
+        if (__ballot(any) == 0) continue;
+        f32x4 a[TRIP], b[TRIP];
+#pragma unroll
+        for (int u = 0; u < TRIP; ++u) load(r0 + u * ROWS, on[u], a[u], b[u]);
+#pragma unroll
+        for (int u = 0; u < TRIP; ++u) {
+            x = fmaxf(x, largest(a[u]));
+            y = fmaxf(y, largest(b[u]));
+        }
+    }
+}
+
 // Eight floats times `scale` as an operand's two terms.
 __device__ __forceinline__ void split_operand(const f32x4 x, const f32x4 y, const float scale, h16x8 &high, h16x8 &low) {
     u32x4 hi, lo;

@@ -87,6 +87,24 @@ def test_rows_beyond_the_sampled_range(device, width):
 
 
 @pytest.mark.parametrize("width", [32, 64])
+@pytest.mark.parametrize("operand", ["du", "q", "kv"])
+def test_zero_rows_around_small_ones(device, width, operand):
+    # The last row alone is not 0 (the loss of one token), and it is far below 1: no sampled row tells the scale,
+    # and with V's rows 0 the scale of dP - δ is δ's alone (dK of a block of zero V rows).
+    q, k, v, du = normal_case(425, width, 24, 1, 480, 480)
+    for x in {"du": (du,), "q": (q,), "kv": (k, v)}[operand]:
+        x[:, :, :479] = 0.0
+    mask = np.ones((24, 480), np.uint8)
+    want = oracle.attention(q, k, v, mask, upstream=du)
+    eq = {"du": 0, "q": -30, "kv": 30}[operand]  # scores keep their size
+    ev, eu = (-30, 0) if operand == "kv" else (0, -30)
+    scaled = [np.ldexp(x, e).astype(np.float32) for x, e in ((q, eq), (k, -eq), (v, ev), (du, eu))]
+    gq, gk, gv, _ = gradients(device, *scaled, mask)
+    check_backward(np.ldexp(gq.astype(np.float64), eq - ev - eu), np.ldexp(gk.astype(np.float64), -eq - ev - eu),
+                   np.ldexp(gv.astype(np.float64), -eu), None, want, operand)
+
+
+@pytest.mark.parametrize("width", [32, 64])
 def test_infinities_and_nan(device, width):
     q, k, v, du = normal_case(430, width, 24, 1, 480, 480)
     mask = np.ones((24, 480), np.uint8)

@@ -74,6 +74,25 @@ def test_rows_beyond_the_sampled_range(device, width):
 
 
 @pytest.mark.parametrize("width", [32, 64])
+def test_zero_rows_around_small_ones(device, width):
+    # Every sampled row is 0 (or masked), and the one row that is not is far below 1; the queries make up for the key's.
+    q, k, v, _ = normal_case(325, width, 24, 1, 480, 480)
+    k[:, :, :479] = 0.0
+    v[:, :, :479] = 0.0
+    mask = np.ones((24, 480), np.uint8)
+    mask[:12, 100:479] = 0
+    mask[5] = 0  # nothing visible
+    want = oracle.attention(q, k, v, mask)
+    q, k, v = (np.ldexp(x, e).astype(np.float32) for x, e in ((q, 30), (k, -30), (v, -40)))
+    out, lse = host(*attention.forward(*to_dev(device, q, k, v, mask)))
+    out = np.ldexp(out.astype(np.float64), 40)
+    for b in range(24):
+        assert np.abs(out[b] - want["output"][b]).max() <= 1e-5 * np.abs(want["output"][b]).max(), b
+    rows = [b for b in range(24) if b != 5]
+    assert np.abs(lse[rows] - want["lse"][rows]).max() <= 1e-6 * np.abs(want["lse"][rows]).max()
+
+
+@pytest.mark.parametrize("width", [32, 64])
 def test_infinities_and_nan(device, width):
     q, k, v, _ = normal_case(330, width, 24, 1, 480, 480)
     q[..., 0] = np.abs(q[..., 0]) + 0.1
