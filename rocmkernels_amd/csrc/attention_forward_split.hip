@@ -703,11 +703,14 @@ void dispatch(const ForwardArgs &a, const Work &w, const int cus, hipStream_t st
 // Where the items are few, the FP32 kernel's four waves per item and shorter start win: up to one item per CU (d = 64, 128
 // items of 32 tiles: 22.3 against 23.9 µs; d = 32, 32 items of 8: 5.6 against 7.5), under a ramp up to two (d = 64, 384 items
 // of up to 16: 14.1 against 15.7; d = 32: 8.6 against 10.8), and at d = 32 for short items (512 of 5: 7.6 against 8.3; 1536 of
-// 3: 9.9 against 11.7).
+// 3: 9.9 against 11.7). At d = 32 the FP32 kernel's planned grid, up to three items per CU, also balances what a ramp or a radius
+// window leaves uneven: it wins while the ramp is short (594 of up to 11: 9.5 against 10.4; but 768, 32: 18.2 against 17.1) or the
+// window's work small (280 of 21: 11.3 against 13.1; 552 of 11: 11.8 against 14.1; but 748 of 33: 34.3 against 23.6).
 bool forward_split_pays(const int D, const ForwardArgs &a, const int cus) {
     const Work w = work_of(a);
     if (w.items <= cus || (w.ramp && w.items < 2ll * cus)) return false;
     if (D == 64) return true;
+    if (w.items <= 3ll * cus && (w.ramp ? w.tiles < 24 : a.radius >= 0 && w.items * w.tiles < 32ll * cus)) return false;
     return w.items <= 2ll * cus ? w.tiles >= 9 : a.radius < 0 || w.tiles >= 5 || w.items >= 16ll * cus;
 }
 

@@ -57,6 +57,21 @@ def test_workgroup_shapes_match_oracle(device, width, batch, heads, queries, key
     assert not gk[0, :, :33].any() and not gv[0, :, :33].any()
 
 
+@pytest.mark.parametrize("width,batch,heads,length,causal", [
+    (32, 7, 1, 2208, True), (32, 7, 1, 2300, True),  # causal ramps either side of two items per CU
+    (64, 24, 1, 1023, True), (64, 24, 1, 991, True),  # and of three
+    (64, 21, 1, 412, False), (64, 24, 1, 415, False),  # 273 and 312 items
+])
+def test_default_backward_either_side_of_the_line(device, width, batch, heads, length, causal):
+    q, k, v, du = normal_case(415, width, batch, heads, length, length)
+    mask = padding_mask(416, batch, length, length // 2)
+    want = oracle.attention(q, k, v, mask, upstream=du, causal=causal)
+    tq, tk, tv, tm, tdu = to_dev(device, q, k, v, mask, du)
+    out, lse = attention.forward(tq, tk, tv, tm, causal=causal)
+    got = host(*attention.backward(tq, tk, tv, tm, out, lse, tdu, causal=causal, entry="ex", deterministic=False))
+    check_backward(*got, want, f"default d{width}")
+
+
 @pytest.mark.parametrize("width", [32, 64])
 @pytest.mark.parametrize("eq,ev,eu", [(-40, -40, 27), (48, 30, -83), (0, -100, 0)])
 def test_magnitudes(device, width, eq, ev, eu):

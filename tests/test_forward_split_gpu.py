@@ -23,6 +23,11 @@ SHAPES = [
     (64, 64, 1, 1000, 1030, -1, False),   # eight and one
     (64, 48, 2, 515, 515, 77, False),     # four and one
     (64, 17, 1, 1023, 33, -1, False),     # fewer keys than one 64-key step
+    # Either side of the line to the FP32 kernel's planned grid: short ramps, small windows.
+    (32, 32, 1, 735, 735, -1, True),
+    (32, 32, 1, 737, 737, -1, True),
+    (32, 24, 1, 711, 711, 300, True),
+    (32, 32, 1, 737, 737, 180, False),
 ]
 
 
