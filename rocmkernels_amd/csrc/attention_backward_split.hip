@@ -445,7 +445,9 @@ __global__ __launch_bounds__(kWave * QB * KS) __attribute__((amdgpu_waves_per_eu
         mu = fmaxf(mu, largest(uraw[i]));
     }
     const int eq = exponent_of(halves_max(mq)) - 14, eu = exponent_of(halves_max(mu)) - 14;
-    const bool plain = !scale_fits(ek) || !scale_fits(ev) || __ballot(!scale_fits(eq) || !scale_fits(eu)) != 0;
+    // Outside the range of scales: for K and V the whole workgroup keeps from the loop; for a wave's own queries only its
+    // products do, as its siblings need the rows that it stages and its barriers.
+    const bool unfit = !scale_fits(ek) || !scale_fits(ev), own_unfit = __ballot(!scale_fits(eq) || !scale_fits(eu)) != 0;
     const float kfactor = scale_down(ek), vfactor = scale_down(ev);
     h16x8 qh[KC], ql[KC], uh[KC], ul[KC];
 #pragma unroll
@@ -580,7 +582,7 @@ __global__ __launch_bounds__(kWave * QB * KS) __attribute__((amdgpu_waves_per_eu
         column_product<D, PLANE>(acc, reads, kt, ds);
     };
 
-    if (nsteps > 0 && !plain) {
+    if (nsteps > 0 && !unfit) {
         uint64_t bits0 = __ballot(mask0 != 0);
         clear_masked(bits0);
         stage(0);
@@ -589,7 +591,7 @@ __global__ __launch_bounds__(kWave * QB * KS) __attribute__((amdgpu_waves_per_eu
         auto step = [&](const int i, const int p) __attribute__((always_inline)) {
             __syncthreads(); // tile i is staged; every wave is done with the other stage
             const int key0 = tile_key(i);
-            const bool live = i * KS + stream < ntiles && tile_valid;
+            const bool live = i * KS + stream < ntiles && tile_valid && !own_unfit;
             const bool inside = live && bits0 == ~0ull && key0 >= first && key0 + kStep <= last && tile_in_window(s, q0, key0) &&
                     tile_in_window(s, q0, key0 + kTile);
             const uint64_t bits1 = __ballot(mbyte != 0);
@@ -616,7 +618,7 @@ __global__ __launch_bounds__(kWave * QB * KS) __attribute__((amdgpu_waves_per_eu
     }
     sum_streams<DT, KS>(acc, stream, reinterpret_cast<float *>(smem) + qi * (16 * DT * kWave) + lane, QB * 16 * DT * kWave);
     if (stream != 0 || !tile_valid) return;
-    if (__builtin_expect(plain || !finite(acc), 0)) {
+    if (__builtin_expect(unfit || own_unfit || !finite(acc), 0)) {
         exact_dq_tile<D, VEC>((const SplitBackwardParams *)__builtin_amdgcn_kernarg_segment_ptr(), seq, q0, dlt);
     } else if (valid) {
         const float factor = l > 0.0f ? __builtin_amdgcn_ldexpf(P.scale / l, ek + eu + ev + 23 - 9) : 0.0f;

@@ -262,7 +262,10 @@ __global__ __launch_bounds__(kWave * QB * KS) __attribute__((amdgpu_waves_per_eu
     int ek, ev; // K = K'·2^ek, V = V'·2^ev
     f32x4 qraw[2 * KC];
     int mask0;
-    bool plain; // magnitudes that FP32 powers of two cannot bring into range: FP32 MFMAs from the start
+    // Magnitudes that FP32 powers of two cannot bring into range: FP32 MFMAs from the start. Those of K and V keep the whole
+    // workgroup from the loop; those of a wave's own queries keep only its products from it, as its siblings need the rows that
+    // it stages and its barriers.
+    bool unfit, own_unfit;
     {
         const int n = min(ulast, s.keys) - ufirst;
         const int key = ufirst + (n > 0 ? static_cast<int>(static_cast<int64_t>(static_cast<int>(threadIdx.x) / CPR) * n / ROWS) : 0);
@@ -294,7 +297,7 @@ __global__ __launch_bounds__(kWave * QB * KS) __attribute__((amdgpu_waves_per_eu
         }
         ek = __builtin_amdgcn_readfirstlane(exponent_of(mk)) - 8;
         ev = __builtin_amdgcn_readfirstlane(exponent_of(mv)) - 8;
-        plain = ek < -kMaxExponent || ek > kMaxExponent || ev < -kMaxExponent || ev > kMaxExponent;
+        unfit = !scale_fits(ek) || !scale_fits(ev);
     }
 
     // Q's terms, scaled so that the row's largest magnitude is in [2^14, 2^15).
@@ -313,8 +316,8 @@ __global__ __launch_bounds__(kWave * QB * KS) __attribute__((amdgpu_waves_per_eu
             for (int j = 0; j < 8; ++j) mq = fmaxf(mq, fabsf(span[i][j]));
         }
         const int eq = exponent_of(halves_max(mq)) - 14;
-        plain = plain || __ballot(eq < -kMaxExponent || eq > kMaxExponent) != 0;
-        const float factor = power_of_two(-min(max(eq, -kMaxExponent), kMaxExponent));
+        own_unfit = __ballot(!scale_fits(eq)) != 0;
+        const float factor = scale_down(eq);
 #pragma unroll
         for (int i = 0; i < KC; ++i) {
             u32x4 hi, lo;
@@ -330,8 +333,7 @@ __global__ __launch_bounds__(kWave * QB * KS) __attribute__((amdgpu_waves_per_eu
         }
         e = eq + ek;
     }
-    const float kfactor = power_of_two(-min(max(ek, -kMaxExponent), kMaxExponent));
-    const float vfactor = power_of_two(-min(max(ev, -kMaxExponent), kMaxExponent));
+    const float kfactor = scale_down(ek), vfactor = scale_down(ev);
 
     // Online-softmax state, as in attention_forward.hip (lazy re-basing: see there), in units of S' and V'. P is kept at
     // 2^kShift times its value, so that its terms lose nothing above 2^-10 and at most 2^-32.
@@ -533,7 +535,7 @@ __global__ __launch_bounds__(kWave * QB * KS) __attribute__((amdgpu_waves_per_eu
         unrolled<2 * CH>([&](auto u) __attribute__((always_inline)) { split_unit(u, kOfV, p); });
     };
 
-    if (nsteps > 0 && !plain) {
+    if (nsteps > 0 && !unfit) {
         uint64_t bits0 = __ballot(mask0 != 0);
         clear_masked(bits0);
         split_rows(0);
@@ -543,7 +545,7 @@ __global__ __launch_bounds__(kWave * QB * KS) __attribute__((amdgpu_waves_per_eu
         auto step = [&](const int i, const int p) __attribute__((always_inline)) {
             __syncthreads(); // tile i is staged; every wave is done with the other stage
             const int key0 = tile_key(i);
-            const bool live = i * KS + stream < ntiles && tile_valid;
+            const bool live = i * KS + stream < ntiles && tile_valid && !own_unfit;
             const bool see_a = live && static_cast<uint32_t>(bits0) != 0 && key0 < last && key0 + kTile > first;
             const bool see_b = live && static_cast<uint32_t>(bits0 >> 32) != 0 && key0 + kTile < last && key0 + kStep > first;
             const bool inside = bits0 == ~0ull && tile_in_window(s, q0, key0) && tile_in_window(s, q0, key0 + kTile);
@@ -623,7 +625,7 @@ __global__ __launch_bounds__(kWave * QB * KS) __attribute__((amdgpu_waves_per_eu
 #pragma unroll
             for (int j = 0; j < 16; ++j) probe = fmaf(o[t][j], 0.0f, probe);
         }
-        if (__builtin_expect(plain || __ballot(probe != 0.0f) != 0, 0)) {
+        if (__builtin_expect(unfit || own_unfit || __ballot(probe != 0.0f) != 0, 0)) {
             exact_query_tile<D, VEC>((const SplitForwardParams *)__builtin_amdgcn_kernarg_segment_ptr(), seq, q0);
         } else {
             l_all = halves_sum(l_all); // each half-wave summed the exponentials of its own keys

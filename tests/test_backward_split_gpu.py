@@ -57,6 +57,27 @@ def test_workgroup_shapes_match_oracle(device, width, batch, heads, queries, key
     assert not gk[0, :, :33].any() and not gv[0, :, :33].any()
 
 
+@pytest.mark.parametrize("operand", ["q", "du"])
+@pytest.mark.parametrize("width,batch,heads,queries,keys,radius,causal", SHAPES)
+def test_query_row_outside_the_scales(device, width, batch, heads, queries, keys, radius, causal, operand):
+    # One row of Q or dO that no scale fits, in the tile of one wave of a dQ workgroup, whose other waves need the rows that it
+    # stages and its barriers: every other row of dQ against the oracle, and all of dK and dV where the row's size lets them be.
+    q, k, v, du = normal_case(440 + width + queries, width, batch, heads, queries, keys)
+    mask = padding_mask(441, batch, keys, keys // 2)
+    rows = ((0, 3, np.inf), (1, 5, 2.0**120), (2, min(37, queries - 1), 2.0**-100), (3, queries - 1, 2.0**120))
+    want = oracle.attention(q, k, v, mask, upstream=du, radius=radius, causal=causal)
+    for b, row, factor in rows:
+        {"q": q, "du": du}[operand][b, 0, row] *= np.float32(factor)
+    b, row, _ = rows[2]
+    small = oracle.attention(q[b:b + 1], k[b:b + 1], v[b:b + 1], mask[b:b + 1], upstream=du[b:b + 1], radius=radius, causal=causal)
+    for name in ("gq", "gk", "gv"):
+        want[name][b] = small[name][0]
+    gq, gk, gv, _ = gradients(device, q, k, v, du, mask, radius, causal)
+    for b, row, _ in (rows[0], rows[1], rows[3]):
+        gq[b, 0, row], gk[b], gv[b] = want["gq"][b, 0, row], want["gk"][b], want["gv"][b]
+    check_backward(gq, gk, gv, None, want, f"beside unfit rows of {operand} d{width}")
+
+
 @pytest.mark.parametrize("width,batch,heads,length,causal", [
     (32, 7, 1, 2208, True), (32, 7, 1, 2300, True),  # causal ramps either side of two items per CU
     (64, 24, 1, 1023, True), (64, 24, 1, 991, True),  # and of three

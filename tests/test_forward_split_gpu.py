@@ -47,6 +47,23 @@ def test_workgroup_shapes_match_oracle(device, width, batch, heads, queries, key
     check_forward(*host(out, lse), want, f"split d{width}")
 
 
+@pytest.mark.parametrize("width,batch,heads,queries,keys,radius,causal", SHAPES[:9])
+def test_query_row_outside_the_scales(device, width, batch, heads, queries, keys, radius, causal):
+    # One query row that no scale fits, in the tile of one wave: its workgroup's other waves still need the rows of K and V
+    # that this wave stages, and its barriers. Every other row against the oracle.
+    q, k, v, _ = normal_case(340 + width + queries, width, batch, heads, queries, keys)
+    mask = padding_mask(341, batch, keys, keys // 2)
+    want = oracle.attention(q, k, v, mask, radius=radius, causal=causal)
+    for b, row, factor in ((0, 37, np.inf), (1, 5, 2.0**120), (2, 70, 2.0**-100), (3, queries - 1, 2.0**120)):
+        q[b, 0, row] *= np.float32(factor)
+    out, lse = host(*attention.forward(*to_dev(device, q, k, v, mask), radius=radius, causal=causal))
+    uniform = oracle.attention(q[2:3], k[2:3], v[2:3], mask[2:3], radius=radius, causal=causal)  # the row of 2^-100
+    want["output"][2, 0, 70], want["lse"][2, 0, 70] = uniform["output"][0, 0, 70], uniform["lse"][0, 0, 70]
+    for b, row in ((0, 37), (1, 5), (3, queries - 1)):
+        out[b, 0, row], lse[b, 0, row] = want["output"][b, 0, row], want["lse"][b, 0, row]
+    check_forward(out, lse, want, f"beside unfit rows d{width}")
+
+
 @pytest.mark.parametrize("width", [32, 64])
 @pytest.mark.parametrize("gain_q,gain_k,gain_v", [(1e-12, 1e12, 1e-20), (3e15, 1e-15, 1e25), (1.0, 1.0, 1e-33), (1e-20, 1e-20, 1e35)])
 def test_magnitudes(device, width, gain_q, gain_k, gain_v):
