@@ -424,6 +424,7 @@ __global__ __launch_bounds__(kWave * QB * KS) __attribute__((amdgpu_waves_per_eu
     }
     const int ek = __builtin_amdgcn_readfirstlane(exponent_of(mk)) - 8; // K = K'·2^ek, V = V'·2^ev, sampled largest at 2^8
     const int ev = __builtin_amdgcn_readfirstlane(exponent_of(mv)) - 8;
+    const bool k_zero = __builtin_amdgcn_readfirstlane(mk == 0.0f), v_zero = __builtin_amdgcn_readfirstlane(mv == 0.0f);
 
     // δ in the order every backward path sums it (group_dot, pairwise tree): this lane holds groups 4i + 2h and 4i + 2h + 1.
     float dlt;
@@ -438,16 +439,26 @@ __global__ __launch_bounds__(kWave * QB * KS) __attribute__((amdgpu_waves_per_eu
         dlt = group_tree(part);
         if (stream == 0 && h == 0 && valid) P.delta[row] = dlt;
     }
-    float mq = 0.0f, mu = 0.0f;
+    float mq = 0.0f, mu = 0.0f, mo = 0.0f;
 #pragma unroll
     for (int i = 0; i < 2 * KC; ++i) {
         mq = fmaxf(mq, largest(qraw[i]));
         mu = fmaxf(mu, largest(uraw[i]));
+        mo = fmaxf(mo, largest(oraw[i]));
     }
-    const int eq = exponent_of(halves_max(mq)) - 14, eu = exponent_of(halves_max(mu)) - 14;
+    mq = halves_max(mq);
+    mu = halves_max(mu);
+    mo = halves_max(mo);
+    const int eq = exponent_of(mq) - 14, eu = exponent_of(mu) - 14;
+    // Rows that only use rows far below the ones that set the scales (hidden from them, or of no weight), whose terms are off by 2^-25
+    // in V' and K'. Of V': the row's weighted mean, which O is, must reach 2^-2. Of K': the largest score tells; |S'| of 2^17 takes
+    // a key of 2^-2 or more. Rows of dO = 0 have no gradient to lose, nor have those of one key of weight 1 (dP = δ).
+    const float top_s = __builtin_amdgcn_ldexpf(P.scale, eq + ek + 17);
+    const bool faint = valid && m != -INFINITY && l > 1.0f + 0x1p-22f && mu > 0.0f &&
+            ((!v_zero && mo < __builtin_amdgcn_ldexpf(1.0f, ev - 2)) || (!k_zero && fabsf(m) < top_s));
     // Outside the range of scales: for K and V the whole workgroup keeps from the loop; for a wave's own queries only its
     // products do, as its siblings need the rows that it stages and its barriers.
-    const bool unfit = !scale_fits(ek) || !scale_fits(ev), own_unfit = __ballot(!scale_fits(eq) || !scale_fits(eu)) != 0;
+    const bool unfit = !scale_fits(ek) || !scale_fits(ev), own_unfit = __ballot(!scale_fits(eq) || !scale_fits(eu) || faint) != 0;
     const float kfactor = scale_down(ek), vfactor = scale_down(ev);
     h16x8 qh[KC], ql[KC], uh[KC], ul[KC];
 #pragma unroll

@@ -15,9 +15,11 @@
 // the order (the compiler's own order puts the MFMAs first, and the two no longer co-execute).
 //
 // Scales (powers of two): each query row its own; K and V one each for the workgroup, from the largest magnitudes of rows
-// sampled over its window (of all its rows where the sampled ones are 0). They put those at 2^8, so rows up to 128 times
-// larger than any sampled one are still in range; larger ones make the result NaN, and a wave that finds a non-finite result
-// computes its query tile again with FP32 MFMAs (as it must anyway for infinities, whose meaning the split products lose).
+// sampled over its window (of all its rows where the sampled ones are 0). They put those at 2^8 (K) and 2^9 (V), so rows up to
+// 64 times larger than any sampled one are still in range; larger ones make the result NaN. A wave computes its query tile again
+// with FP32 MFMAs where it finds a non-finite result (as it must anyway for infinities, whose meaning the split products lose)
+// or a row whose keys and values all lie so far below the scales that their terms lost bits: the rows that set a scale may
+// be hidden from it by the masks, or have no weight.
 #include <algorithm>
 #include <type_traits>
 
@@ -265,7 +267,7 @@ __global__ __launch_bounds__(kWave * QB * KS) __attribute__((amdgpu_waves_per_eu
     // Magnitudes that FP32 powers of two cannot bring into range: FP32 MFMAs from the start. Those of K and V keep the whole
     // workgroup from the loop; those of a wave's own queries keep only its products from it, as its siblings need the rows that
     // it stages and its barriers.
-    bool unfit, own_unfit;
+    bool unfit, own_unfit, v_zero; // v_zero: every visible row of V is 0
     {
         const int n = min(ulast, s.keys) - ufirst;
         const int key = ufirst + (n > 0 ? static_cast<int>(static_cast<int64_t>(static_cast<int>(threadIdx.x) / CPR) * n / ROWS) : 0);
@@ -296,8 +298,9 @@ __global__ __launch_bounds__(kWave * QB * KS) __attribute__((amdgpu_waves_per_eu
             workgroup_largest(mk, mv, amax);
         }
         ek = __builtin_amdgcn_readfirstlane(exponent_of(mk)) - 8;
-        ev = __builtin_amdgcn_readfirstlane(exponent_of(mv)) - 8;
+        ev = __builtin_amdgcn_readfirstlane(exponent_of(mv)) - 9;
         unfit = !scale_fits(ek) || !scale_fits(ev);
+        v_zero = __builtin_amdgcn_readfirstlane(mv == 0.0f);
     }
 
     // Q's terms, scaled so that the row's largest magnitude is in [2^14, 2^15).
@@ -618,17 +621,27 @@ __global__ __launch_bounds__(kWave * QB * KS) __attribute__((amdgpu_waves_per_eu
     }
 
     if (stream == 0 && tile_valid) {
+        l_all = halves_sum(l_all); // each half-wave summed the exponentials of its own keys
         // A non-finite result: some input of the tile is not finite or out of its scale's range, or the result overflows.
-        float probe = l_all * 0.0f;
+        float probe = l_all * 0.0f, largest_o = 0.0f;
 #pragma unroll
         for (int t = 0; t < DT; ++t) {
 #pragma unroll
-            for (int j = 0; j < 16; ++j) probe = fmaf(o[t][j], 0.0f, probe);
+            for (int j = 0; j < 16; ++j) {
+                probe = fmaf(o[t][j], 0.0f, probe);
+                largest_o = fmaxf(largest_o, fabsf(o[t][j]));
+            }
         }
-        if (__builtin_expect(unfit || own_unfit || __ballot(probe != 0.0f) != 0, 0)) {
+        // A row that used only rows far below the ones that set the scales (hidden from it, or of no weight). Of V': where its terms
+        // are below 2^-3 they are off by 2^-25, and so are weights below 2^-10, here times at most 2^10 sampled; so the row's
+        // largest weighted mean must reach 1, as that of normal values does for 2^17 keys. Of K': an error of 2^-25 moves a score
+        // by up to 2^-7·c2 (Q' below 2^15, errors of D features adding up at random), which must be below 2^-23, or the row's
+        // largest |S'| at least 2^16, as where its keys are at 2^-2 or more.
+        largest_o = halves_max(largest_o);
+        const bool faint = query < s.queries && ((!v_zero && largest_o < l_all) || (c2 > 0x1p-16f && fabsf(m_all) < 0x1p16f));
+        if (__builtin_expect(unfit || own_unfit || __ballot(probe != 0.0f || faint) != 0, 0)) {
             exact_query_tile<D, VEC>((const SplitForwardParams *)__builtin_amdgcn_kernarg_segment_ptr(), seq, q0);
         } else {
-            l_all = halves_sum(l_all); // each half-wave summed the exponentials of its own keys
             const float base = mc_all == -INFINITY ? 0.0f : mc_all;
             // O is o / l in any offset; lse's sum is Σ exp(s - max) = l · exp2(offset - max·c2).
             const float sum = m_all == -INFINITY ? l_all : l_all * exp2_fast(base - kShift - m_all * c2);

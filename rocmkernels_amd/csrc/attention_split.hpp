@@ -1,5 +1,6 @@
 // FP32 matrix products on the fp16 matrix cores: every FP32 operand, scaled by a power of two, is split into two fp16 terms
-// and the product is summed from three fp16 products.
+// and the product is summed from three fp16 products (the splitting of Dekker 1971, doi:10.1007/BF01397083, and Ootomo and Yokota
+// 2022, doi:10.1177/10943420221090256).
 //
 // x·2^s = h + l + e with h = fp16(x·2^s) and l = fp16(x·2^s - h), each rounded to nearest even: 22 significant bits and a
 // sign, |e| <= 2^-23 of |x·2^s| while l is a normal number (|x·2^s| >= 2^-3), and at most 2^-25 below that. x·y is then
@@ -7,12 +8,13 @@
 // v_mfma_f32_32x32x16_f16 adds 16 of them per accumulator rounding, so a dot product rounds far less often than on
 // v_mfma_f32_32x32x2f32, which more than makes up for the two bits.
 //
-// The scales put the largest magnitude of an operand's rows at 2^8 or more, so what is lost below 2^-3 is at most 2^-33 of it,
-// far below FP32's own rounding of the sums that the small elements share with the large ones.
+// The scales put the largest magnitude of an operand's rows at 2^8 or more, so what is lost below 2^-3 is at most 2^-33 of it:
+// far below FP32's own rounding of any sum that small elements share with the large ones. A result that does not share its sums
+// with the rows that set the scale (a mask hides them, or their weights are 0) may lose more than FP32 does, up to all of it.
+// Callers therefore test how far a result's rows lie below the scale, and compute again with FP32 MFMAs where it is too far.
 //
 // An element that is not finite, or that passes 65504 after scaling, has h = ±inf and l = ∓inf or NaN: every result that it
-// enters is NaN (inf - inf, or 0·inf), never a wrong number. Callers test their results and compute again with FP32 MFMAs
-// where they find one.
+// enters is NaN (inf - inf, or 0·inf). Callers test for these too and compute them again in the same way.
 //
 // Cost: v_mfma_f32_32x32x16_f16 does 16 times the work of an FP32 MFMA per cycle, so three products take 3/16 of its time,
 // and unlike FP32 MFMAs they co-execute with VALU work. Splitting takes 2.5 VALU instructions per element (1.5

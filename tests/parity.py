@@ -102,6 +102,35 @@ def padding_mask(seed, batch, keys, low):
     return (np.arange(keys)[None, :] < lengths[:, None]).astype(np.uint8)
 
 
+def reference64(q, k, v, mask, du=None, radius=-1, causal=False):
+    """Dense attention of a few sequences in 64 bits: output, lse and, given dO, gq, gk, gv (packed [B][H][L][D])."""
+    q, k, v = (np.asarray(x, np.float64) for x in (q, k, v))
+    scale = 1.0 / np.sqrt(q.shape[3])
+    qi, ki = np.arange(q.shape[2])[:, None], np.arange(k.shape[2])[None, :]
+    window = np.ones((q.shape[2], k.shape[2]), bool)
+    if causal:
+        window &= ki <= qi
+    if radius >= 0:
+        window &= np.abs(qi - ki) <= radius
+    scores = np.where(window & (np.asarray(mask) != 0)[:, None, None, :], q @ k.swapaxes(2, 3) * scale, -np.inf)
+    m = scores.max(-1, keepdims=True)
+    p = np.exp(scores - m)
+    total = p.sum(-1, keepdims=True)
+    p /= total
+    out = {"output": p @ v, "lse": np.concatenate([m, total], -1)}
+    if du is not None:
+        du = np.asarray(du, np.float64)
+        ds = p * (du @ v.swapaxes(2, 3) - (du * out["output"]).sum(-1, keepdims=True))
+        out.update(gq=ds @ k * scale, gk=ds.swapaxes(2, 3) @ q * scale, gv=p.swapaxes(2, 3) @ du)
+    return out
+
+
+def norm_rel(got, want):
+    """2-norm of the difference over 2-norm of ``want``."""
+    got, want = np.asarray(got, np.float64), np.asarray(want, np.float64)
+    return float(np.linalg.norm(got - want) / np.linalg.norm(want))
+
+
 def fp32_score_floor(q, k, v, mask, radius=-1, causal=False):
     """Error of an FP32 forward whose scores are plain FP32 dot products: each score q.k accumulated feature by feature
     with one rounding per fused multiply-add (the reference GPU kernels' own arithmetic), everything after it in

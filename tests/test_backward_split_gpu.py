@@ -6,7 +6,7 @@ import pytest
 import torch
 
 import oracle
-from parity import check_backward, host, normal_case, padding_mask, to_dev
+from parity import check_backward, host, norm_rel, normal_case, padding_mask, reference64, to_dev
 from rocmkernels_amd import attention
 
 pytestmark = pytest.mark.gpu
@@ -138,6 +138,25 @@ def test_zero_rows_around_small_ones(device, width, operand):
     gq, gk, gv, _ = gradients(device, *scaled, mask)
     check_backward(np.ldexp(gq.astype(np.float64), eq - ev - eu), np.ldexp(gk.astype(np.float64), -eq - ev - eu),
                    np.ldexp(gv.astype(np.float64), -eu), None, want, operand)
+
+
+@pytest.mark.parametrize("exponent", [10, 14, 20, 30])
+@pytest.mark.parametrize("width", [32, 64])
+def test_large_keys_outside_the_gradient_of_q(device, width, exponent):
+    # As the forward's test of the same: keys 96 .. 99 set the scales of K or V and are causally hidden from queries 0 .. 95, or key 0
+    # does and has no weight. dQ of the other rows; an FP32 backward is at 1e-6 of 64 bits on them.
+    q, k, v, du = normal_case(450 + width, width, 24, 1, 1001, 1001)
+    mask = np.ones((24, 1001), np.uint8)
+    large = np.float32(2.0**exponent)
+    v[0, 0, 96:100] *= large
+    k[1, 0, 96:100] *= large
+    q[2:4, 0, :, 0] = np.abs(q[2:4, 0, :, 0]) + 1.0
+    k[2:4, 0, :4, 0] = -8.0 * max(64.0, 2.0**exponent / 64.0)
+    v[2, 0, :4] *= large
+    want = reference64(q[:4], k[:4], v[:4], mask[:4], du[:4], causal=True)
+    gq = gradients(device, q, k, v, du, mask, causal=True)[0]
+    for b, rows in ((0, slice(0, 96)), (1, slice(0, 96)), (2, slice(4, None)), (3, slice(4, None))):
+        assert norm_rel(gq[b, 0, rows], want["gq"][b, 0, rows]) <= 3e-6, b
 
 
 @pytest.mark.parametrize("width", [32, 64])

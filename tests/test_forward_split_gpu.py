@@ -6,7 +6,7 @@ import pytest
 import torch
 
 import oracle
-from parity import check_forward, host, normal_case, padding_mask, to_dev
+from parity import check_forward, host, norm_rel, normal_case, padding_mask, reference64, to_dev
 from rocmkernels_amd import attention
 
 pytestmark = pytest.mark.gpu
@@ -112,6 +112,29 @@ def test_zero_rows_around_small_ones(device, width):
         assert np.abs(out[b] - want["output"][b]).max() <= 1e-5 * np.abs(want["output"][b]).max(), b
     rows = [b for b in range(24) if b != 5]
     assert np.abs(lse[rows] - want["lse"][rows]).max() <= 1e-6 * np.abs(want["lse"][rows]).max()
+
+
+@pytest.mark.parametrize("exponent", [10, 14, 20, 30])
+@pytest.mark.parametrize("width,batch,heads,queries,keys,radius,causal", [SHAPES[2], (64, 24, 1, 1000, 1000, -1, True), SHAPES[4], SHAPES[7]])
+def test_large_rows_outside_the_result(device, width, batch, heads, queries, keys, radius, causal, exponent):
+    # Rows that set a workgroup's scales (four in a row: one is sampled) and that a query does not see, or gives no weight to, must
+    # not cost it accuracy. Hidden: keys 96 .. 99 under the causal mask; weightless: key 0, whose score is far below all others.
+    # An FP32 forward is at 4e-7 of 64 bits on these rows, and terms of the large rows' scale lose 2e-6 (2^14) to all of it.
+    q, k, v, _ = normal_case(350 + width, width, batch, heads, queries, keys)
+    mask = np.ones((batch, keys), np.uint8)
+    large = np.float32(2.0**exponent)
+    v[0, 0, 96:100] *= large
+    k[1, 0, 96:100] *= large
+    q[2:4, 0, :, 0] = np.abs(q[2:4, 0, :, 0]) + 1.0
+    k[2:4, 0, :4, 0] = -8.0 * max(64.0, 2.0**exponent / 64.0)  # a score of -90 or less
+    v[2, 0, :4] *= large
+    want = reference64(q[:4], k[:4], v[:4], mask[:4], radius=radius, causal=causal)
+    out, lse = host(*attention.forward(*to_dev(device, q, k, v, mask), radius=radius, causal=causal))
+    for b, rows in ((0, slice(0, 96)), (1, slice(0, 96)), (2, slice(4, None)), (3, slice(4, None))):
+        if b < 2 and not causal:
+            continue
+        for name, got in (("output", out), ("lse", lse)):
+            assert norm_rel(got[b, 0, rows], want[name][b, 0, rows]) <= 1e-6, (b, name)
 
 
 @pytest.mark.parametrize("width", [32, 64])
