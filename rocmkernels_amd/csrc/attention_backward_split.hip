@@ -15,7 +15,10 @@
 // workgroup's block in kernel 2), the streamed ones by that of rows sampled over the workgroup's window, as in the forward
 // (of all its rows where the sampled ones are 0). P is kept at 2^9 times exp(s - max) in kernel 1 (the row's 1/sum is applied
 // to dQ at the end) and at 2^14 times its value in kernel 2; dS in units in which |dP - δ| of that size still fits fp16.
-// Whatever leaves the range becomes NaN, and a wave whose gradients are not finite computes its tile again with FP32 MFMAs.
+// Whatever leaves the range becomes NaN, and a wave whose gradients are not finite computes its tile again with FP32 MFMAs. So
+// does one with a row or a key whose terms lost bits: the rows that set a scale may be hidden from it or have no weight, and a
+// key may have small weights only. Kernel 1 tells from O and the row maximum, kernel 2 from Σ P² and Σ dS² of each key (the
+// dot products of the high terms with themselves, 16 VALU instructions a tile: 2 to 4% of its time).
 //
 // What bounds them: 21 fp16 MFMAs of 32 x 32 x 16 per 32 x 32 tile and 16 columns of width in the two (12 and 9) do what 7 x 8 FP32
 // ones of twice the time did, beside 16 exponentials and about 100 other VALU instructions per lane and kernel; at d = 64, 32 x
@@ -307,6 +310,23 @@ __device__ __forceinline__ void sum_streams(f32x16 (&acc)[N], const int stream, 
             }
         }
     }
+}
+
+template<int N>
+__device__ __forceinline__ float largest(const f32x16 (&acc)[N]) {
+    float x = 0.0f;
+#pragma unroll
+    for (int t = 0; t < N; ++t) {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) x = fmaxf(x, fabsf(acc[t][j]));
+    }
+    return x;
+}
+
+// sum + x² + y² of a packed pair.
+__device__ __forceinline__ float add_squares(const uint32_t pair, const float sum) {
+    const h16x2 x = __builtin_bit_cast(h16x2, pair);
+    return __builtin_amdgcn_fdot2(x, x, sum, false);
 }
 
 template<int N>
@@ -650,6 +670,12 @@ __global__ __launch_bounds__(kWave * KB * QS) __attribute__((amdgpu_waves_per_eu
     __shared__ __align__(16) unsigned char smem[STAGE_BYTES > MERGE_BYTES ? STAGE_BYTES : MERGE_BYTES];
     __shared__ __align__(16) float stats[QS][2][2][kTile]; // per stage: exponent offset of P, and δ'
     __shared__ float amax[2][KB * QS];
+    // Operands in LDS instead of registers, V's low terms and then K's: what 256 registers don't hold at D = 64, as far as the
+    // workgroups of a CU have room. In scratch their reloads wait for the rows in flight (whole backward, 32 x 2048 causal 233
+    // against 251 µs, 15 x 777 x 1001 68 against 78).
+    constexpr int PARKED = D == 32 ? 0 : KB == 4 ? (QS == 1 ? 4 : 3) : (QS == 4 ? 8 : 6);
+    __shared__ __align__(16) uint16_t parked[PARKED > 0 ? KB * PARKED * kWave * 8 : 8];
+    __shared__ float norms[QS > 1 ? QS - 1 : 1][KB][2][kWave]; // of streams 1 ..: Σ P'² and Σ dS'² of each lane
 
     const Shape &s = P.s;
     const int lane = threadIdx.x & (kWave - 1);
@@ -746,7 +772,7 @@ __global__ __launch_bounds__(kWave * KB * QS) __attribute__((amdgpu_waves_per_eu
         __syncthreads(); // amax is read
         workgroup_largest(mq, mu, amax);
     }
-    const int eq = __builtin_amdgcn_readfirstlane(exponent_of(mq)) - 8; // Q = Q'·2^eq, dO = dO'·2^eu, sampled largest at 2^8
+    const int eq = __builtin_amdgcn_readfirstlane(exponent_of(mq)) - 11; // Q = Q'·2^eq, dO = dO'·2^eu, sampled largest at 2^11, 2^8
     const int eu = __builtin_amdgcn_readfirstlane(exponent_of(mu)) - 8;
     float mk = 0.0f, mv = 0.0f;
 #pragma unroll
@@ -754,18 +780,25 @@ __global__ __launch_bounds__(kWave * KB * QS) __attribute__((amdgpu_waves_per_eu
         mk = fmaxf(mk, largest(kraw[i]));
         mv = fmaxf(mv, largest(vraw[i]));
     }
+    const float own_k = halves_max(mk), own_v = halves_max(mv); // of this lane's key
     __syncthreads(); // amax is read
     workgroup_largest(mk, mv, amax);
     const int ek = __builtin_amdgcn_readfirstlane(exponent_of(mk)) - 14;
     int ev = __builtin_amdgcn_readfirstlane(exponent_of(mv)) - 14;
-    if (__builtin_amdgcn_readfirstlane(mv == 0.0f)) { // dP = 0: the unit of dP - δ below comes from the largest |δ|, put at 2^-3
-        float md = 0.0f, none = 0.0f;
+    // A key whose own row lies below 2^-2 beside the block's largest.
+    const bool faint_key = (own_k > 0.0f && own_k < __builtin_amdgcn_ldexpf(1.0f, ek - 2)) ||
+            (own_v > 0.0f && own_v < __builtin_amdgcn_ldexpf(1.0f, ev - 2));
+    float md = 1.0f;
+    if (__builtin_amdgcn_readfirstlane(mv == 0.0f)) { // dP = 0: the unit of dP - δ below comes from the largest |δ|, put at 2^-4
+        float none = 0.0f;
+        md = 0.0f;
         for (int r = threadIdx.x; r < n; r += kWave * KB * QS) md = fmaxf(md, fabsf(buffer_load(dbuf, 4u * static_cast<uint32_t>(ufirst + r), 0)));
         __syncthreads(); // amax is read
         workgroup_largest(md, none, amax);
-        if (md > 0.0f) ev = __builtin_amdgcn_readfirstlane(exponent_of(md)) - eu - 24;
+        if (md > 0.0f) ev = __builtin_amdgcn_readfirstlane(exponent_of(md)) - eu - 20;
     }
-    const bool plain = !scale_fits(ek) || !scale_fits(ev) || !scale_fits(eq) || !scale_fits(eu);
+    // Exactly 0 whatever the scales: dV and dK, and dK alone.
+    const bool no_dv = __builtin_amdgcn_readfirstlane(mu == 0.0f), no_dk = __builtin_amdgcn_readfirstlane(mu == 0.0f || mq == 0.0f || md == 0.0f);
     const float qfactor = scale_down(eq), ufactor = scale_down(eu);
     h16x8 kh[KC], kl[KC], vh[KC], vl[KC];
 #pragma unroll
@@ -773,14 +806,34 @@ __global__ __launch_bounds__(kWave * KB * QS) __attribute__((amdgpu_waves_per_eu
         split_operand(kraw[2 * i], kraw[2 * i + 1], scale_down(ek), kh[i], kl[i]);
         split_operand(vraw[2 * i], vraw[2 * i + 1], scale_down(ev), vh[i], vl[i]);
     }
-    // P' = 2^14·P = exp2(S'·c2 + offset); dP - δ in units of 2^(eu + ev + 27): r = dP'·2^-27 - δ'. P'·r stays below 2^16 while
-    // P·|dP - δ| is below 64 times twice the product of the largest |dO| (sampled) and |V|.
+    h16x8 *const park = reinterpret_cast<h16x8 *>(parked) + ki * PARKED * kWave + lane;
+    if (stream == 0) {
+#pragma unroll
+        for (int x = 0; x < PARKED; ++x) park[x * kWave] = x < KC ? vl[x % KC] : kl[x % KC];
+    }
+    // Low terms of K or V, from the first barrier of the loop on.
+    auto low_terms = [&](auto of_k, h16x8 (&x)[KC], const h16x8 (&held)[KC]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < KC; ++i) {
+            const int at = i + (decltype(of_k)::value ? KC : 0);
+            if (at < PARKED) x[i] = park[at * kWave];
+            else x[i] = held[i];
+        }
+    };
+    // P' = 2^14·P = exp2(S'·c2 + offset); dP - δ in units of 2^(eu + ev + 24): r = dP'·2^-24 - δ'. P'·r stays below 2^16 while
+    // P·|dP - δ| is below 4 times the product of the largest |dO| (sampled) and |V|.
     const float c2 = __builtin_amdgcn_ldexpf(P.scale * kLog2e, eq + ek);
-    constexpr float kUnit = 1.0f / (1 << 27);
+    constexpr float kUnit = 1.0f / (1 << 24);
+    // FP32 MFMAs from the start: for the whole workgroup where a scale does not fit, or where rows of Q below 2^-3, whose terms are
+    // off by 2^-25, could move a score by more than 2^-22 (2^-7·c2: K' below 2^15, errors of D features adding up at random); for one
+    // wave where a key of its own is faint (it goes on staging for the others).
+    const bool unfit = !scale_fits(ek) || !scale_fits(ev) || !scale_fits(eq) || !scale_fits(eu) || c2 > 0x1p-15f;
+    const bool own_unfit = __ballot(faint_key) != 0;
 
     f32x16 acc_k[DT], acc_v[DT];
 #pragma unroll
     for (int t = 0; t < DT; ++t) acc_k[t] = acc_v[t] = f32x16{};
+    float p_norm = 0.0f, ds_norm = 0.0f; // Σ P'² and Σ dS'² of the lane's key over its half of the rows, from the high terms
 
     auto stage = [&](const int i, const int p) __attribute__((always_inline)) {
         u32x2 terms[2];
@@ -794,16 +847,20 @@ __global__ __launch_bounds__(kWave * KB * QS) __attribute__((amdgpu_waves_per_eu
         if (ki == 0 && h == 0) {
             const bool ok = tile_query(i) + col < s.queries && i * QS + stream < ntiles && rm != -INFINITY;
             stats[stream][p][0][col] = ok ? 14.0f - fmaf(rm, kLog2e, __log2f(rl)) : -INFINITY;
-            stats[stream][p][1][col] = __builtin_amdgcn_ldexpf(-rd, -(eu + ev + 27));
+            stats[stream][p][1][col] = __builtin_amdgcn_ldexpf(-rd, -(eu + ev + 24));
         }
     };
-    // The tile in stage p. The order is left to the compiler: at D = 64 the step just fits 256 registers, and with its groups
-    // pinned as in kernel 1 50 of them are spilled (32 x 2048 causal 123 -> 256 µs; with one wave per SIMD instead 142).
+    // The tile in stage p. The order is left to the compiler: at D = 64, some operands in LDS, the step just fits 256 registers, and
+    // with its groups pinned as in kernel 1 50 of them are spilled (32 x 2048 causal 123 -> 256 µs; with one wave per SIMD
+    // instead 142).
     auto tile_step = [&](auto masked, const int p, const int q0) __attribute__((always_inline)) {
         const uint16_t *const qt = stages + p * STAGE;
         f32x16 sc{}, dp{};
-        row_product<D, PLANE>(sc, reads, qt, kh, kl);
-        row_product<D, PLANE>(dp, reads, qt + 2 * PLANE, vh, vl);
+        h16x8 low[KC];
+        low_terms(std::integral_constant<bool, true>{}, low, kl);
+        row_product<D, PLANE>(sc, reads, qt, kh, low);
+        low_terms(std::integral_constant<bool, false>{}, low, vl);
+        row_product<D, PLANE>(dp, reads, qt + 2 * PLANE, vh, low);
         uint32_t keep = 0;
         if constexpr (decltype(masked)::value) keep = visible ? bit_range(qlo - q0, qhi - q0) >> (4 * h) : 0u;
         uint32_t pt[2][8], ds[2][8];
@@ -822,18 +879,20 @@ __global__ __launch_bounds__(kWave * KB * QS) __attribute__((amdgpu_waves_per_eu
             split_pair<false>(x[2], x[3], one, pt[0][2 * u + 1], pt[1][2 * u + 1]);
             split_pair<false>(y[0], y[1], one, ds[0][2 * u], ds[1][2 * u]);
             split_pair<false>(y[2], y[3], one, ds[0][2 * u + 1], ds[1][2 * u + 1]);
+            p_norm = add_squares(pt[0][2 * u + 1], add_squares(pt[0][2 * u], p_norm));
+            ds_norm = add_squares(ds[0][2 * u + 1], add_squares(ds[0][2 * u], ds_norm));
         }
         column_product<D, PLANE>(acc_v, reads, qt + 2 * PLANE, pt);
         column_product<D, PLANE>(acc_k, reads, qt, ds);
     };
 
-    if (nsteps > 0 && !plain) {
+    if (nsteps > 0 && !unfit) {
         stage(0, 0);
         load_tile(1);
         auto step = [&](const int i, const int p) __attribute__((always_inline)) {
             __syncthreads(); // tile i is staged; every wave is done with the other stage
             const int q0 = tile_query(i);
-            const bool work = i * QS + stream < ntiles && bits != 0 && q0 < last && q0 + kTile > first;
+            const bool work = i * QS + stream < ntiles && bits != 0 && !own_unfit && q0 < last && q0 + kTile > first;
             stage(i + 1, p ^ 1);
             load_tile(i + 2);
             if (__builtin_expect(work, 1)) {
@@ -848,14 +907,42 @@ __global__ __launch_bounds__(kWave * KB * QS) __attribute__((amdgpu_waves_per_eu
         }
     }
     float *const slot = reinterpret_cast<float *>(smem) + ki * (16 * DT * kWave) + lane;
+    if (QS > 1 && stream > 0) {
+        norms[stream - 1][ki][0][lane] = p_norm;
+        norms[stream - 1][ki][1][lane] = ds_norm;
+    }
     sum_streams<DT, QS>(acc_k, stream, slot, KB * 16 * DT * kWave);
     sum_streams<DT, QS>(acc_v, stream, slot, KB * 16 * DT * kWave);
     if (stream != 0 || !tile_valid) return;
-    if (__builtin_expect(plain || !finite(acc_k) || !finite(acc_v), 0)) {
+#pragma unroll
+    for (int x = 0; x < QS - 1; ++x) {
+        p_norm += norms[x][ki][0][lane];
+        ds_norm += norms[x][ki][1][lane];
+    }
+    // Keys whose sums are made of terms that lost bits (below 2^-3 they are off by 2^-25): because the rows of dO or Q that count for
+    // the key lie far below the ones that set the scales (hidden from it, or without weight), or its weights or dS are small
+    // throughout. With Σ P'² of n rows, dV' is off by 2^-25·√(Σ P'²) from dO' and by 2^-26·√n·|dO'| from P': the first is below
+    // 2^-21 of the largest |dV'| if that reaches 2^-4·√(Σ P'²), the second below 2^-20 if Σ P'² reaches 2^-12·n. The same for dK' with
+    // dS' and Q', whose second loss also does no harm where it is below FP32's own rounding of dP (a key of weight near 1, whose
+    // dP - δ cancels): 2^-24·|dO'|·|V'|·√D in units of 2^24, |dO'| taken from dV'.
+    p_norm = halves_sum(p_norm);
+    ds_norm = halves_sum(ds_norm);
+    const float top_v = halves_max(largest(acc_v)), top_k = halves_max(largest(acc_k));
+    const float seen = static_cast<float>(qhi - max(qlo, 0) + 1);
+    bool faint = visible && ((!no_dv && (256.0f * top_v * top_v < p_norm || p_norm < 0x1p-12f * seen)) || (!no_dk && 256.0f * top_k * top_k < ds_norm));
+    const bool faint_ds = visible && !no_dk && ds_norm < 0x1p-12f * seen;
+    if (__builtin_expect(__ballot(faint_ds) != 0, 0)) {
+        float own = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 2 * KC; ++i)
+            own = fmaxf(own, largest(load_chunk<VEC>(vbuf, visible ? static_cast<uint32_t>(key) * (4u * P.v.st) + 4u * (16 * (i / 2) + 8 * h + 4 * (i % 2)) : kNoRow, 0)));
+        faint = faint || (faint_ds && top_v * 8.0f * halves_max(own) * scale_down(ev) < 0x1p24f * sqrtf(seen));
+    }
+    if (__builtin_expect(unfit || own_unfit || __ballot(faint) != 0 || !finite(acc_k) || !finite(acc_v), 0)) {
         exact_dkdv_tile<D, VEC>((const SplitBackwardParams *)__builtin_amdgcn_kernarg_segment_ptr(), seq, kt);
     } else if (key < s.keys) {
         const int64_t krow = (static_cast<int64_t>(seq) * s.keys + key) * D;
-        const float kscale = __builtin_amdgcn_ldexpf(P.scale, eq + eu + ev + 27 - 14), vscale = __builtin_amdgcn_ldexpf(1.0f, eu - 14);
+        const float kscale = __builtin_amdgcn_ldexpf(P.scale, eq + eu + ev + 24 - 14), vscale = __builtin_amdgcn_ldexpf(1.0f, eu - 14);
 #pragma unroll
         for (int t = 0; t < DT; ++t) {
             store_tile_row<VEC>(P.dk + krow + 32 * t, acc_k[t], kscale, h);

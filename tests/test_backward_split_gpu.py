@@ -159,6 +159,54 @@ def test_large_keys_outside_the_gradient_of_q(device, width, exponent):
         assert norm_rel(gq[b, 0, rows], want["gq"][b, 0, rows]) <= 3e-6, b
 
 
+@pytest.mark.parametrize("exponent", [10, 14, 20, 30])
+@pytest.mark.parametrize("width", [32, 64])
+def test_large_queries_outside_the_gradients_of_keys(device, width, exponent):
+    # Rows 0 .. 3 of dO or Q set the scales of the dK/dV kernel (row 0 is sampled), and only keys 0 .. 3 are seen by them; or one key's
+    # V or K is far larger than those of its block. dK and dV of the other keys; an FP32 backward is at 1e-6 of 64 bits on them.
+    q, k, v, du = normal_case(460 + width, width, 24, 1, 1001, 1001)
+    mask = np.ones((24, 1001), np.uint8)
+    du[0, 0, :4] *= np.float32(2.0**exponent)
+    q[1, 0, :4] *= np.float32(2.0**min(exponent, 20))
+    k[2, 0, 1000] = -np.abs(k[2, 0, 1000]) * np.float32(2.0**exponent)  # the last key: one query sees it, at a score far below the others
+    q[2, 0, 1000] = np.abs(q[2, 0, 1000])
+    v[3, 0, 0] *= np.float32(2.0**-exponent)
+    want = reference64(q[:4], k[:4], v[:4], mask[:4], du[:4], causal=True)
+    _, gk, gv, _ = gradients(device, q, k, v, du, mask, causal=True)
+    for b, rows in ((0, slice(4, None)), (1, slice(4, None)), (2, slice(0, 1000)), (3, slice(0, 1))):
+        for name, got in (("gk", gk), ("gv", gv)):
+            assert norm_rel(got[b, 0, rows], want[name][b, 0, rows]) <= 3e-6, (b, name)
+
+
+@pytest.mark.parametrize("width", [32, 64])
+def test_keys_of_small_weights(device, width):
+    # Keys 0 .. 299 have weights of about 2^-37 throughout: their rows of dK and dV are that small and still have FP32's accuracy (4e-6
+    # to 8e-6: scores of -25 to 25 round to 1e-6).
+    q, k, v, du = normal_case(470 + width, width, 24, 1, 1001, 1001)
+    mask = np.ones((24, 1001), np.uint8)
+    q[0, 0, :, 0] += 20.0
+    k[0, 0, :300, 0] -= 25.0 * np.sqrt(width) / 20.0
+    want = reference64(q[:1], k[:1], v[:1], mask[:1], du[:1])
+    _, gk, gv, _ = gradients(device, q, k, v, du, mask)
+    for name, got in (("gk", gk), ("gv", gv)):
+        for rows in (slice(0, 300), slice(300, None)):
+            assert norm_rel(got[0, 0, rows], want[name][0, 0, rows]) <= 2e-5, (name, rows)
+
+
+@pytest.mark.parametrize("width", [32, 64])
+def test_peaked_weights_row_by_row(device, width):
+    # Scores of standard deviation 4 under a causal mask: some of the last keys, which few queries see, have next to no weight. Every
+    # row of dK and dV against its own norm (FP32: up to 3e-5).
+    q, k, v, du = normal_case(480 + width, width, 24, 1, 1001, 1001)
+    mask = np.ones((24, 1001), np.uint8)
+    q *= 4.0
+    want = reference64(q[:4], k[:4], v[:4], mask[:4], du[:4], causal=True)
+    _, gk, gv, _ = gradients(device, q, k, v, du, mask, causal=True)
+    for name, got in (("gk", gk), ("gv", gv)):
+        errors = np.linalg.norm(got[:4] - want[name], axis=-1) / np.linalg.norm(want[name], axis=-1)
+        assert errors.max() <= 1e-4, (name, np.unravel_index(errors.argmax(), errors.shape))
+
+
 @pytest.mark.parametrize("width", [32, 64])
 def test_infinities_and_nan(device, width):
     q, k, v, du = normal_case(430, width, 24, 1, 480, 480)
