@@ -55,14 +55,42 @@ __device__ __forceinline__ const SplitBackwardParams &uniform_params(const Split
     return *reinterpret_cast<const SplitBackwardParams *>(uniform);
 }
 
-// dQ of one query tile on FP32 MFMAs by one wave, for inputs that the split products cannot carry; dlt is the lane's query's δ.
-template<int D, bool VEC>
-__device__ __attribute__((noinline)) void exact_dq_tile(const SplitBackwardParams *params, const int seq_, const int q0_, const float dlt) {
+// Sums acc over the workgroup's WAVES waves into wave 0 through `slots` (16 N floats a lane for each wave but one), in order.
+template<int WAVES, int N>
+__device__ __forceinline__ void sum_waves(f32x16 (&acc)[N], const int wave, const LdsFloats slots) {
+    constexpr int SLOT = 16 * N * kWave;
+    const int lane = threadIdx.x & (kWave - 1);
+    __syncthreads(); // the slots' last use
+    if (wave > 0) {
+#pragma unroll
+        for (int t = 0; t < N; ++t) {
+#pragma unroll
+            for (int j = 0; j < 16; ++j) slots[(wave - 1) * SLOT + (16 * t + j) * kWave + lane] = acc[t][j];
+        }
+    }
+    __syncthreads();
+    if (wave == 0) {
+#pragma unroll 1
+        for (int w = 0; w < WAVES - 1; ++w) {
+#pragma unroll
+            for (int t = 0; t < N; ++t) {
+#pragma unroll
+                for (int j = 0; j < 16; ++j) acc[t][j] += slots[w * SLOT + (16 * t + j) * kWave + lane];
+            }
+        }
+    }
+}
+
+// dQ of one query tile on FP32 MFMAs by the workgroup's WAVES waves, for inputs that the split products cannot carry: operands
+// straight from memory, alternate key tiles a wave.
+template<int D, bool VEC, int WAVES>
+__device__ __attribute__((noinline)) void exact_dq_tile(const SplitBackwardParams *params, const LdsFloats slots, const int seq_, const int q0_) {
     const SplitBackwardParams &P = uniform_params(params);
     const int seq = __builtin_amdgcn_readfirstlane(seq_), q0 = __builtin_amdgcn_readfirstlane(q0_);
     constexpr int HALF = D / 2, DT = D / 32;
     const Shape s = P.s;
     const int lane = threadIdx.x & (kWave - 1), col = lane & 31, h = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int query = q0 + col;
     const bool valid = query < s.queries;
     const int b = seq / s.heads, head = seq - b * s.heads;
@@ -80,24 +108,31 @@ __device__ __attribute__((noinline)) void exact_dq_tile(const SplitBackwardParam
     float qr[HALF], ur[HALF];
     buffer_load_span<VEC>(qr, qbuf, valid ? static_cast<uint32_t>(query) * (4u * P.q.st) + 4u * h * HALF : kNoRow);
     buffer_load_span<VEC>(ur, ubuf, valid ? static_cast<uint32_t>(query) * (4u * P.u.st) + 4u * h * HALF : kNoRow);
-    const float m = valid ? P.lse[2 * row] : -INFINITY, l = valid ? P.lse[2 * row + 1] : 0.0f;
+    const float m = valid ? P.lse[2 * row] : -INFINITY, l = valid ? P.lse[2 * row + 1] : 0.0f, dlt = valid ? P.delta[row] : 0.0f;
     const float mc = m != -INFINITY ? fmaf(m, kLog2e, __log2f(l)) : INFINITY;
     f32x16 acc[DT];
 #pragma unroll
     for (int t = 0; t < DT; ++t) acc[t] = f32x16{};
 #pragma unroll 1
-    for (int key0 = first; key0 < last; key0 += kTile) {
+    for (int key0 = first + wave * kTile; key0 < last; key0 += WAVES * kTile) {
         const uint32_t bits = static_cast<uint32_t>(__ballot(buffer_load_byte(mbuf, static_cast<uint32_t>(key0 + col)) != 0));
         if (bits == 0) continue;
+        float kr[HALF], vr[HALF];
+        buffer_load_span<VEC>(kr, kbuf, static_cast<uint32_t>(key0 + col) * kstep + 4u * h * HALF);
+        buffer_load_span<VEC>(vr, vbuf, static_cast<uint32_t>(key0 + col) * vstep + 4u * h * HALF);
         f32x16 sc{}, dp{};
-        {
-            float kr[HALF];
-            buffer_load_span<VEC>(kr, kbuf, static_cast<uint32_t>(key0 + col) * kstep + 4u * h * HALF);
 #pragma unroll
-            for (int c = 0; c < HALF; ++c) sc = mfma(kr[c], qr[c], sc);
-            buffer_load_span<VEC>(kr, vbuf, static_cast<uint32_t>(key0 + col) * vstep + 4u * h * HALF);
+        for (int c = 0; c < HALF; ++c) sc = mfma(kr[c], qr[c], sc);
+        __builtin_amdgcn_sched_barrier(0); // what follows takes the registers of K's rows
 #pragma unroll
-            for (int c = 0; c < HALF; ++c) dp = mfma(kr[c], ur[c], dp);
+        for (int c = 0; c < HALF; ++c) dp = mfma(vr[c], ur[c], dp);
+        float kc[16 * DT];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const int r = tile_row(j, h);
+            const uint32_t at = (bits >> r) & 1u ? static_cast<uint32_t>(key0 + r) * kstep + 4u * col : kNoRow;
+#pragma unroll
+            for (int t = 0; t < DT; ++t) kc[j * DT + t] = buffer_load(kbuf, at + 128u * t, 0);
         }
         const uint32_t visible = (bits & bit_range(wlo - key0, whi - key0)) >> (4 * h);
 #pragma unroll
@@ -107,27 +142,25 @@ __device__ __attribute__((noinline)) void exact_dq_tile(const SplitBackwardParam
         }
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
-            const int r = tile_row(j, h);
 #pragma unroll
-            for (int t = 0; t < DT; ++t) {
-                const uint32_t at = (bits >> r) & 1u ? static_cast<uint32_t>(key0 + r) * kstep + 4u * (32 * t + col) : kNoRow;
-                acc[t] = mfma(buffer_load(kbuf, at, 0), sc[j], acc[t]);
-            }
+            for (int t = 0; t < DT; ++t) acc[t] = mfma(kc[j * DT + t], sc[j], acc[t]);
         }
     }
-    if (!valid) return;
+    sum_waves<WAVES, DT>(acc, wave, slots);
+    if (wave > 0 || !valid) return;
 #pragma unroll
     for (int t = 0; t < DT; ++t) store_tile_row<VEC>(P.dq + row * D + 32 * t, acc[t], P.scale, h);
 }
 
-// dK and dV of one key tile on FP32 MFMAs by one wave.
-template<int D, bool VEC>
-__device__ __attribute__((noinline)) void exact_dkdv_tile(const SplitBackwardParams *params, const int seq_, const int kt_) {
+// dK and dV of one key tile on FP32 MFMAs by the workgroup's WAVES waves, alternate query tiles a wave.
+template<int D, bool VEC, int WAVES>
+__device__ __attribute__((noinline)) void exact_dkdv_tile(const SplitBackwardParams *params, const LdsFloats slots, const int seq_, const int kt_) {
     const SplitBackwardParams &P = uniform_params(params);
     const int seq = __builtin_amdgcn_readfirstlane(seq_), kt = __builtin_amdgcn_readfirstlane(kt_);
     constexpr int HALF = D / 2, DT = D / 32;
     const Shape s = P.s;
     const int lane = threadIdx.x & (kWave - 1), col = lane & 31, h = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int key = kt * kTile + col;
     const int b = seq / s.heads, head = seq - b * s.heads;
     const Buffer qbuf = make_buffer(sequence(P.q, b, head), sequence_bytes(s.queries, P.q.st, D));
@@ -150,38 +183,53 @@ __device__ __attribute__((noinline)) void exact_dkdv_tile(const SplitBackwardPar
 #pragma unroll
     for (int t = 0; t < DT; ++t) acc_k[t] = acc_v[t] = f32x16{};
 #pragma unroll 1
-    for (int q0 = first; q0 < last; q0 += kTile) {
+    for (int q0 = first + wave * kTile; q0 < last; q0 += WAVES * kTile) {
+        float qr[HALF], ur[HALF];
+        buffer_load_span<VEC>(qr, qbuf, static_cast<uint32_t>(q0 + col) * qstep + 4u * h * HALF);
+        buffer_load_span<VEC>(ur, ubuf, static_cast<uint32_t>(q0 + col) * ustep + 4u * h * HALF);
+        const float rm = buffer_load(lbuf, static_cast<uint32_t>(q0 + col) * 8u, 0), rl = buffer_load(lbuf, static_cast<uint32_t>(q0 + col) * 8u + 4u, 0);
+        const float delta = buffer_load(dbuf, static_cast<uint32_t>(q0 + col) * 4u, 0); // of row col
         f32x16 sc{}, dp{};
-        {
-            float qr[HALF];
-            buffer_load_span<VEC>(qr, qbuf, static_cast<uint32_t>(q0 + col) * qstep + 4u * h * HALF);
 #pragma unroll
-            for (int c = 0; c < HALF; ++c) sc = mfma(qr[c], kr[c], sc);
-            buffer_load_span<VEC>(qr, ubuf, static_cast<uint32_t>(q0 + col) * ustep + 4u * h * HALF);
+        for (int c = 0; c < HALF; ++c) sc = mfma(qr[c], kr[c], sc);
+        const float offset = rm != -INFINITY ? fmaf(rm, kLog2e, __log2f(rl)) : INFINITY;
 #pragma unroll
-            for (int c = 0; c < HALF; ++c) dp = mfma(qr[c], vr[c], dp);
-        }
+        for (int c = 0; c < HALF; ++c) dp = mfma(ur[c], vr[c], dp);
         const uint32_t keep = visible ? bit_range(qlo - q0, qhi - q0) >> (4 * h) : 0u;
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
-            const uint32_t qq = static_cast<uint32_t>(q0 + tile_row(j, h));
-            const float m = buffer_load(lbuf, qq * 8u, 0), l = buffer_load(lbuf, qq * 8u + 4u, 0), d = buffer_load(dbuf, qq * 4u, 0);
-            const bool ok = ((keep >> (8 * (j >> 2) + (j & 3))) & 1u) && m != -INFINITY;
-            const float p = ok ? exp2_fast(fmaf(sc[j], c2, -fmaf(m, kLog2e, __log2f(l)))) : 0.0f;
+            const float to = __shfl(offset, tile_row(j, h)), d = __shfl(delta, tile_row(j, h));
+            const bool ok = ((keep >> (8 * (j >> 2) + (j & 3))) & 1u) && to != INFINITY;
+            const float p = ok ? exp2_fast(fmaf(sc[j], c2, -to)) : 0.0f;
             sc[j] = p;
             dp[j] = ok ? p * (dp[j] - d) : 0.0f;
         }
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const uint32_t qq = static_cast<uint32_t>(q0 + tile_row(j, h));
+        for (int part = 0; part < 2; ++part) { // the columns of 8 rows a half-wave at a time: registers hold no more at D = 64
+            __builtin_amdgcn_sched_barrier(0);
+            float uc[8 * DT], qc[8 * DT];
 #pragma unroll
-            for (int t = 0; t < DT; ++t) {
-                acc_v[t] = mfma(buffer_load(ubuf, qq * ustep + 4u * (32 * t + col), 0), sc[j], acc_v[t]);
-                acc_k[t] = mfma(buffer_load(qbuf, qq * qstep + 4u * (32 * t + col), 0), dp[j], acc_k[t]);
+            for (int j = 0; j < 8; ++j) {
+                const uint32_t qq = static_cast<uint32_t>(q0 + tile_row(8 * part + j, h));
+#pragma unroll
+                for (int t = 0; t < DT; ++t) {
+                    uc[j * DT + t] = buffer_load(ubuf, qq * ustep + 4u * (32 * t + col), 0);
+                    qc[j * DT + t] = buffer_load(qbuf, qq * qstep + 4u * (32 * t + col), 0);
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+#pragma unroll
+                for (int t = 0; t < DT; ++t) {
+                    acc_v[t] = mfma(uc[j * DT + t], sc[8 * part + j], acc_v[t]);
+                    acc_k[t] = mfma(qc[j * DT + t], dp[8 * part + j], acc_k[t]);
+                }
             }
         }
     }
-    if (key >= s.keys) return;
+    sum_waves<WAVES, DT>(acc_k, wave, slots);
+    sum_waves<WAVES, DT>(acc_v, wave, slots);
+    if (wave > 0 || key >= s.keys) return;
     const int64_t krow = (static_cast<int64_t>(seq) * s.keys + key) * D;
 #pragma unroll
     for (int t = 0; t < DT; ++t) {
@@ -353,7 +401,9 @@ __global__ __launch_bounds__(kWave * QB * KS) __attribute__((amdgpu_waves_per_eu
     constexpr int RPC = kWave * QB / CPR;
     constexpr int STAGE_BYTES = 2 * KS * STAGE * 2, MERGE_BYTES = (KS - 1) * QB * 16 * DT * kWave * 4;
     __shared__ __align__(16) unsigned char smem[STAGE_BYTES > MERGE_BYTES ? STAGE_BYTES : MERGE_BYTES];
+    static_assert((QB * KS - 1) * 16 * DT * kWave * 4 <= STAGE_BYTES); // the slots of exact_dq_tile
     __shared__ float amax[2][QB * KS];
+    __shared__ int redone[QB]; // query tiles to compute again
 
     const Shape &s = P.s;
     const int lane = threadIdx.x & (kWave - 1);
@@ -471,11 +521,11 @@ __global__ __launch_bounds__(kWave * QB * KS) __attribute__((amdgpu_waves_per_eu
     mo = halves_max(mo);
     const int eq = exponent_of(mq) - 14, eu = exponent_of(mu) - 14;
     // Rows that only use rows far below the ones that set the scales (hidden from them, or of no weight), whose terms are off by 2^-25
-    // in V' and K'. Of V': the row's weighted mean, which O is, must reach 2^-2. Of K': the largest score tells; |S'| of 2^17 takes
+    // in V' and K'. Of V': the row's weighted mean, which O is, must reach 2^-3/√l (as in the forward). Of K': the largest score tells; |S'| of 2^17 takes
     // a key of 2^-2 or more. Rows of dO = 0 have no gradient to lose, nor have those of one key of weight 1 (dP = δ).
     const float top_s = __builtin_amdgcn_ldexpf(P.scale, eq + ek + 17);
     const bool faint = valid && m != -INFINITY && l > 1.0f + 0x1p-22f && mu > 0.0f &&
-            ((!v_zero && mo < __builtin_amdgcn_ldexpf(1.0f, ev - 2)) || (!k_zero && fabsf(m) < top_s));
+            ((!v_zero && mo * sqrtf(l) < __builtin_amdgcn_ldexpf(1.0f, ev - 3)) || (!k_zero && fabsf(m) < top_s));
     // Outside the range of scales: for K and V the whole workgroup keeps from the loop; for a wave's own queries only its
     // products do, as its siblings need the rows that it stages and its barriers.
     const bool unfit = !scale_fits(ek) || !scale_fits(ev), own_unfit = __ballot(!scale_fits(eq) || !scale_fits(eu) || faint) != 0;
@@ -648,13 +698,18 @@ __global__ __launch_bounds__(kWave * QB * KS) __attribute__((amdgpu_waves_per_eu
         }
     }
     sum_streams<DT, KS>(acc, stream, reinterpret_cast<float *>(smem) + qi * (16 * DT * kWave) + lane, QB * 16 * DT * kWave);
-    if (stream != 0 || !tile_valid) return;
-    if (__builtin_expect(unfit || own_unfit || !finite(acc), 0)) {
-        exact_dq_tile<D, VEC>((const SplitBackwardParams *)__builtin_amdgcn_kernarg_segment_ptr(), seq, q0, dlt);
-    } else if (valid) {
+    const bool redo = stream == 0 && tile_valid && (unfit || own_unfit || !finite(acc));
+    if (stream == 0 && valid && __builtin_expect(!redo, 1)) {
         const float factor = l > 0.0f ? __builtin_amdgcn_ldexpf(P.scale / l, ek + eu + ev + 23 - 9) : 0.0f;
 #pragma unroll
         for (int t = 0; t < DT; ++t) store_tile_row<VEC>(P.dq + row * D + 32 * t, acc[t], factor, h);
+    }
+    if (stream == 0 && lane == 0) redone[qi] = redo;
+    __syncthreads();
+#pragma unroll 1
+    for (int x = 0; x < QB; ++x) {
+        if (__builtin_expect(__builtin_amdgcn_readfirstlane(redone[x]), 0))
+            exact_dq_tile<D, VEC, QB * KS>((const SplitBackwardParams *)__builtin_amdgcn_kernarg_segment_ptr(), (LdsFloats)smem, seq, (qb * QB + x) * kTile);
     }
 }
 
@@ -669,7 +724,10 @@ __global__ __launch_bounds__(kWave * KB * QS) __attribute__((amdgpu_waves_per_eu
     constexpr int STAGE_BYTES = 2 * QS * STAGE * 2, MERGE_BYTES = (QS - 1) * KB * 16 * DT * kWave * 4;
     __shared__ __align__(16) unsigned char smem[STAGE_BYTES > MERGE_BYTES ? STAGE_BYTES : MERGE_BYTES];
     __shared__ __align__(16) float stats[QS][2][2][kTile]; // per stage: exponent offset of P, and δ'
+    static_assert((KB * QS - 1) * 16 * DT * kWave * 4 <= STAGE_BYTES); // the slots of exact_dkdv_tile
     __shared__ float amax[2][KB * QS];
+    __shared__ int redone[KB]; // key tiles to compute again
+    __shared__ int gradient_chunks; // at least the rows of dO in the window that are not 0, where they were counted
     // Operands in LDS instead of registers, V's low terms and then K's: what 256 registers don't hold at D = 64, as far as the
     // workgroups of a CU have room. In scratch their reloads wait for the rows in flight (whole backward, 32 x 2048 causal 233
     // against 251 µs, 15 x 777 x 1001 68 against 78).
@@ -762,14 +820,17 @@ __global__ __launch_bounds__(kWave * KB * QS) __attribute__((amdgpu_waves_per_eu
 
     float mq = largest(sq), mu = largest(su);
     workgroup_largest(mq, mu, amax);
+    if (threadIdx.x == 0) gradient_chunks = 0x40000000;
     if (n > ROWS && __builtin_amdgcn_readfirstlane(mq == 0.0f || mu == 0.0f)) {
-        window_largest<kWave * KB * QS, CPR>(mq, mu, n, [&](const int) { return true; },
+        if (threadIdx.x == 0) gradient_chunks = 0;
+        const int found = window_largest<kWave * KB * QS, CPR>(mq, mu, n, [&](const int) { return true; },
                 [&](const int r, const bool on, f32x4 &x, f32x4 &y) {
                     const uint32_t at = 16u * (threadIdx.x % CPR), row = static_cast<uint32_t>(ufirst + r);
                     x = load_chunk<VEC>(qbuf, on ? row * qstep + at : kNoRow, 0);
                     y = load_chunk<VEC>(ubuf, on ? row * ustep + at : kNoRow, 0);
                 });
         __syncthreads(); // amax is read
+        if (found != 0) atomicAdd(&gradient_chunks, found);
         workgroup_largest(mq, mu, amax);
     }
     const int eq = __builtin_amdgcn_readfirstlane(exponent_of(mq)) - 11; // Q = Q'·2^eq, dO = dO'·2^eu, sampled largest at 2^11, 2^8
@@ -913,34 +974,35 @@ __global__ __launch_bounds__(kWave * KB * QS) __attribute__((amdgpu_waves_per_eu
     }
     sum_streams<DT, QS>(acc_k, stream, slot, KB * 16 * DT * kWave);
     sum_streams<DT, QS>(acc_v, stream, slot, KB * 16 * DT * kWave);
-    if (stream != 0 || !tile_valid) return;
+    bool redo = false;
+    if (stream == 0 && tile_valid) {
 #pragma unroll
-    for (int x = 0; x < QS - 1; ++x) {
-        p_norm += norms[x][ki][0][lane];
-        ds_norm += norms[x][ki][1][lane];
-    }
-    // Keys whose sums are made of terms that lost bits (below 2^-3 they are off by 2^-25): because the rows of dO or Q that count for
-    // the key lie far below the ones that set the scales (hidden from it, or without weight), or its weights or dS are small
-    // throughout. With Σ P'² of n rows, dV' is off by 2^-25·√(Σ P'²) from dO' and by 2^-26·√n·|dO'| from P': the first is below
-    // 2^-21 of the largest |dV'| if that reaches 2^-4·√(Σ P'²), the second below 2^-20 if Σ P'² reaches 2^-12·n. The same for dK' with
-    // dS' and Q', whose second loss also does no harm where it is below FP32's own rounding of dP (a key of weight near 1, whose
-    // dP - δ cancels): 2^-24·|dO'|·|V'|·√D in units of 2^24, |dO'| taken from dV'.
-    p_norm = halves_sum(p_norm);
-    ds_norm = halves_sum(ds_norm);
-    const float top_v = halves_max(largest(acc_v)), top_k = halves_max(largest(acc_k));
-    const float seen = static_cast<float>(qhi - max(qlo, 0) + 1);
-    bool faint = visible && ((!no_dv && (256.0f * top_v * top_v < p_norm || p_norm < 0x1p-12f * seen)) || (!no_dk && 256.0f * top_k * top_k < ds_norm));
-    const bool faint_ds = visible && !no_dk && ds_norm < 0x1p-12f * seen;
-    if (__builtin_expect(__ballot(faint_ds) != 0, 0)) {
-        float own = 0.0f;
+        for (int x = 0; x < QS - 1; ++x) {
+            p_norm += norms[x][ki][0][lane];
+            ds_norm += norms[x][ki][1][lane];
+        }
+        // Keys whose sums are made of terms that lost bits (below 2^-3 they are off by 2^-25): because the rows of dO or Q that count for
+        // the key lie far below the ones that set the scales (hidden from it, or without weight), or its weights or dS are small
+        // throughout. With Σ P'² of n rows, dV' is off by 2^-25·√(Σ P'²) from dO' and by 2^-26·√n·|dO'| from P': the first is below
+        // 2^-21 of the largest |dV'| if that reaches 2^-4·√(Σ P'²), the second below 2^-20 if Σ P'² reaches 2^-12·n. The same for dK' with
+        // dS' and Q', whose second loss also does no harm where it is below FP32's own rounding of dP (a key of weight near 1, whose
+        // dP - δ cancels): 2^-24·|dO'|·|V'|·√D in units of 2^24, |dO'| taken from dV'.
+        p_norm = halves_sum(p_norm);
+        ds_norm = halves_sum(ds_norm);
+        const float top_v = halves_max(largest(acc_v)), top_k = halves_max(largest(acc_k));
+        const float seen = static_cast<float>(min(qhi - max(qlo, 0) + 1, gradient_chunks)); // rows that can be off (dO = 0: exact)
+        bool faint = visible && ((!no_dv && (256.0f * top_v * top_v < p_norm || p_norm < 0x1p-12f * seen)) || (!no_dk && 256.0f * top_k * top_k < ds_norm));
+        const bool faint_ds = visible && !no_dk && ds_norm < 0x1p-12f * seen;
+        if (__builtin_expect(__ballot(faint_ds) != 0, 0)) {
+            float own = 0.0f;
 #pragma unroll
-        for (int i = 0; i < 2 * KC; ++i)
-            own = fmaxf(own, largest(load_chunk<VEC>(vbuf, visible ? static_cast<uint32_t>(key) * (4u * P.v.st) + 4u * (16 * (i / 2) + 8 * h + 4 * (i % 2)) : kNoRow, 0)));
-        faint = faint || (faint_ds && top_v * 8.0f * halves_max(own) * scale_down(ev) < 0x1p24f * sqrtf(seen));
+            for (int i = 0; i < 2 * KC; ++i)
+                own = fmaxf(own, largest(load_chunk<VEC>(vbuf, visible ? static_cast<uint32_t>(key) * (4u * P.v.st) + 4u * (16 * (i / 2) + 8 * h + 4 * (i % 2)) : kNoRow, 0)));
+            faint = faint || (faint_ds && top_v * 8.0f * halves_max(own) * scale_down(ev) < 0x1p24f * sqrtf(seen));
+        }
+        redo = unfit || own_unfit || __ballot(faint) != 0 || !finite(acc_k) || !finite(acc_v);
     }
-    if (__builtin_expect(unfit || own_unfit || __ballot(faint) != 0 || !finite(acc_k) || !finite(acc_v), 0)) {
-        exact_dkdv_tile<D, VEC>((const SplitBackwardParams *)__builtin_amdgcn_kernarg_segment_ptr(), seq, kt);
-    } else if (key < s.keys) {
+    if (stream == 0 && key < s.keys && __builtin_expect(!redo, 1)) {
         const int64_t krow = (static_cast<int64_t>(seq) * s.keys + key) * D;
         const float kscale = __builtin_amdgcn_ldexpf(P.scale, eq + eu + ev + 24 - 14), vscale = __builtin_amdgcn_ldexpf(1.0f, eu - 14);
 #pragma unroll
@@ -948,6 +1010,13 @@ __global__ __launch_bounds__(kWave * KB * QS) __attribute__((amdgpu_waves_per_eu
             store_tile_row<VEC>(P.dk + krow + 32 * t, acc_k[t], kscale, h);
             store_tile_row<VEC>(P.dv + krow + 32 * t, acc_v[t], vscale, h);
         }
+    }
+    if (stream == 0 && lane == 0) redone[ki] = redo;
+    __syncthreads();
+#pragma unroll 1
+    for (int x = 0; x < KB; ++x) {
+        if (__builtin_expect(__builtin_amdgcn_readfirstlane(redone[x]), 0))
+            exact_dkdv_tile<D, VEC, KB * QS>((const SplitBackwardParams *)__builtin_amdgcn_kernarg_segment_ptr(), (LdsFloats)smem, seq, kb * KB + x);
     }
 }
 

@@ -16,8 +16,8 @@
 //
 // Scales (powers of two): each query row its own; K and V one each for the workgroup, from the largest magnitudes of rows
 // sampled over its window (of all its rows where the sampled ones are 0). They put those at 2^8 (K) and 2^9 (V), so rows up to
-// 64 times larger than any sampled one are still in range; larger ones make the result NaN. A wave computes its query tile again
-// with FP32 MFMAs where it finds a non-finite result (as it must anyway for infinities, whose meaning the split products lose)
+// 64 times larger than any sampled one are still in range; larger ones make the result NaN. A query tile is computed again with
+// FP32 MFMAs, by the whole workgroup, where its wave finds a non-finite result (as it must anyway for infinities, whose meaning the split products lose)
 // or a row whose keys and values all lie so far below the scales that their terms lost bits: the rows that set a scale may
 // be hidden from it by the masks, or have no weight.
 #include <algorithm>
@@ -82,19 +82,22 @@ __device__ __forceinline__ void store_rows(const SplitForwardParams &P, const in
     }
 }
 
-// One query tile on FP32 MFMAs by one wave, for inputs that the split products cannot carry: the arithmetic of
-// attention_forward.hip, operands straight from memory. Kept out of line (and given the kernel's arguments by address), so
-// that the main loop's registers do not depend on it.
-template<int D, bool VEC>
-__device__ __attribute__((noinline)) void exact_query_tile(const SplitForwardParams *params, const int seq_, const int q0_) {
+// One query tile on FP32 MFMAs by the workgroup's WAVES waves, for inputs that the split products cannot carry: the arithmetic of
+// attention_forward.hip, operands straight from memory, K a tile ahead. The waves take alternate key tiles and are merged in order
+// through `slots` (3 + D/2 floats a lane for each wave but one). Kept out of line (and given the kernel's arguments by
+// address), so that the main loop's registers do not depend on it, and one for each register budget of a kernel (WPE). With one wave a tile instead, a single tile that needed
+// it held its launch up for 200 µs (24 x 1024 at width 32).
+template<int D, bool VEC, int WAVES, int WPE>
+__device__ __attribute__((noinline)) void exact_query_tile(const SplitForwardParams *params, LdsFloats slots, const int seq_, const int q0_) {
     const auto address = reinterpret_cast<uint64_t>(params);
     const uint64_t uniform = static_cast<uint64_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(address >> 32))) << 32 |
             static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(address)));
     const SplitForwardParams &P = *reinterpret_cast<const SplitForwardParams *>(uniform);
     const int seq = __builtin_amdgcn_readfirstlane(seq_), q0 = __builtin_amdgcn_readfirstlane(q0_);
-    constexpr int HALF = D / 2, DT = D / 32;
+    constexpr int HALF = D / 2, DT = D / 32, SLOT = (3 + 16 * DT) * kWave;
     const Shape s = P.s;
     const int lane = threadIdx.x & (kWave - 1), col = lane & 31, h = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int query = q0 + col;
     const int b = seq / s.heads, head = seq - b * s.heads;
     const Buffer qbuf = make_buffer(sequence(P.q, b, head), sequence_bytes(s.queries, P.q.st, D));
@@ -107,23 +110,39 @@ __device__ __attribute__((noinline)) void exact_query_tile(const SplitForwardPar
     int first, last;
     forward_key_range(s, q0 / kTile, first, last);
 
-    float qr[HALF];
+    float qr[HALF], kr[HALF];
     buffer_load_span<VEC>(qr, qbuf, static_cast<uint32_t>(query) * (4u * P.q.st) + 4u * h * HALF);
+    int mbyte = 0;
+    auto load_keys = [&](const int key0) __attribute__((always_inline)) {
+        const bool live = key0 < last;
+        mbyte = buffer_load_byte(mbuf, live ? static_cast<uint32_t>(key0 + col) : kNoRow);
+        buffer_load_span<VEC>(kr, kbuf, live ? static_cast<uint32_t>(key0 + col) * kstep + 4u * h * HALF : kNoRow);
+    };
     float m = -INFINITY, base = -INFINITY, l = 0.0f; // m over this half-wave's keys; base of l and o, in log2 units
     f32x16 o[DT];
 #pragma unroll
     for (int t = 0; t < DT; ++t) o[t] = f32x16{};
+    load_keys(first + wave * kTile);
 #pragma unroll 1
-    for (int key0 = first; key0 < last; key0 += kTile) {
-        const uint32_t bits = static_cast<uint32_t>(__ballot(buffer_load_byte(mbuf, static_cast<uint32_t>(key0 + col)) != 0));
-        if (bits == 0) continue;
-        f32x16 sc{};
-        {
-            float kr[HALF];
-            buffer_load_span<VEC>(kr, kbuf, static_cast<uint32_t>(key0 + col) * kstep + 4u * h * HALF);
-#pragma unroll
-            for (int c = 0; c < HALF; ++c) sc = mfma(kr[c], qr[c], sc);
+    for (int key0 = first + wave * kTile; key0 < last; key0 += WAVES * kTile) {
+        const uint32_t bits = static_cast<uint32_t>(__ballot(mbyte != 0));
+        if (bits == 0) {
+            load_keys(key0 + WAVES * kTile);
+            continue;
         }
+        float vc[16 * DT];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const int r = tile_row(j, h);
+            // Masked keys contribute exactly nothing, whatever their stored values hold.
+            const uint32_t at = (bits >> r) & 1u ? static_cast<uint32_t>(key0 + r) * vstep + 4u * col : kNoRow;
+#pragma unroll
+            for (int t = 0; t < DT; ++t) vc[j * DT + t] = buffer_load(vbuf, at + 128u * t, 0);
+        }
+        f32x16 sc{};
+#pragma unroll
+        for (int c = 0; c < HALF; ++c) sc = mfma(kr[c], qr[c], sc);
+        load_keys(key0 + WAVES * kTile);
         const uint32_t visible = (bits & bit_range(wlo - key0, whi - key0)) >> (4 * h);
         float mx = m;
 #pragma unroll
@@ -147,19 +166,51 @@ __device__ __attribute__((noinline)) void exact_query_tile(const SplitForwardPar
         }
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
-            const int r = tile_row(j, h);
 #pragma unroll
-            for (int t = 0; t < DT; ++t) {
-                // Masked keys contribute exactly nothing, whatever their stored values hold.
-                const uint32_t at = (bits >> r) & 1u ? static_cast<uint32_t>(key0 + r) * vstep + 4u * (32 * t + col) : kNoRow;
-                o[t] = mfma(buffer_load(vbuf, at, 0), sc[j], o[t]);
-            }
+            for (int t = 0; t < DT; ++t) o[t] = mfma(vc[j * DT + t], sc[j], o[t]);
         }
     }
-    const float m_all = halves_max(m);
-    l = halves_sum(l);
-    const float sum = m_all == -INFINITY ? l : l * exp2_fast((base == -INFINITY ? 0.0f : base) - m_all * c2);
-    store_rows<D, VEC>(P, seq, query, h, o, l, m_all * P.scale, sum, 0);
+    m = halves_max(m);
+    if (wave > 0) {
+        const LdsFloats slot = slots + (wave - 1) * SLOT + lane;
+        slot[0] = m;
+        slot[kWave] = l;
+        slot[2 * kWave] = base;
+#pragma unroll
+        for (int t = 0; t < DT; ++t) {
+#pragma unroll
+            for (int j = 0; j < 16; ++j) slot[(3 + 16 * t + j) * kWave] = o[t][j];
+        }
+    }
+    __syncthreads();
+    if (wave == 0) {
+        float top = base;
+#pragma unroll
+        for (int w = 0; w < WAVES - 1; ++w) {
+            m = fmaxf(m, slots[w * SLOT + lane]);
+            top = fmaxf(top, slots[w * SLOT + 2 * kWave + lane]);
+        }
+        const float to = top == -INFINITY ? 0.0f : top;
+        const float own = exp2_fast(base - to);
+        l *= own;
+#pragma unroll
+        for (int t = 0; t < DT; ++t) o[t] *= own;
+#pragma unroll 1
+        for (int w = 0; w < WAVES - 1; ++w) {
+            const LdsFloats slot = slots + w * SLOT + lane;
+            const float a = exp2_fast(slot[2 * kWave] - to);
+            l = fmaf(slot[kWave], a, l);
+#pragma unroll
+            for (int t = 0; t < DT; ++t) {
+#pragma unroll
+                for (int j = 0; j < 16; ++j) o[t][j] = fmaf(slot[(3 + 16 * t + j) * kWave], a, o[t][j]);
+            }
+        }
+        l = halves_sum(l);
+        const float sum = m == -INFINITY ? l : l * exp2_fast(to - m * c2);
+        store_rows<D, VEC>(P, seq, query, h, o, l, m * P.scale, sum, 0);
+    }
+    __syncthreads(); // the slots are read
 }
 
 } // namespace
@@ -177,8 +228,10 @@ __global__ __launch_bounds__(kWave * QB * KS) __attribute__((amdgpu_waves_per_eu
     constexpr int NREG = 16 * DT + 3;                // merged per lane: maximum, sum, base and the accumulators
     constexpr int STAGE_BYTES = 2 * KS * STAGE * 2;
     constexpr int MERGE_BYTES = (KS - 1) * QB * NREG * kWave * 4;
+    static_assert((QB * KS - 1) * NREG * kWave * 4 <= STAGE_BYTES); // the slots of exact_query_tile
     __shared__ __align__(16) unsigned char smem[STAGE_BYTES > MERGE_BYTES ? STAGE_BYTES : MERGE_BYTES];
     __shared__ float amax[2][QB * KS];               // largest sampled |K| and |V| of each wave
+    __shared__ int redone[QB];                       // query tiles to compute again
 
     const Shape &s = P.s;
     const int lane = threadIdx.x & (kWave - 1);
@@ -620,6 +673,7 @@ __global__ __launch_bounds__(kWave * QB * KS) __attribute__((amdgpu_waves_per_eu
         }
     }
 
+    bool redo = false;
     if (stream == 0 && tile_valid) {
         l_all = halves_sum(l_all); // each half-wave summed the exponentials of its own keys
         // A non-finite result: some input of the tile is not finite or out of its scale's range, or the result overflows.
@@ -632,21 +686,26 @@ __global__ __launch_bounds__(kWave * QB * KS) __attribute__((amdgpu_waves_per_eu
                 largest_o = fmaxf(largest_o, fabsf(o[t][j]));
             }
         }
-        // A row that used only rows far below the ones that set the scales (hidden from it, or of no weight). Of V': where its terms
-        // are below 2^-3 they are off by 2^-25, and so are weights below 2^-10, here times at most 2^10 sampled; so the row's
-        // largest weighted mean must reach 1, as that of normal values does for 2^17 keys. Of K': an error of 2^-25 moves a score
-        // by up to 2^-7·c2 (Q' below 2^15, errors of D features adding up at random), which must be below 2^-23, or the row's
-        // largest |S'| at least 2^16, as where its keys are at 2^-2 or more.
         largest_o = halves_max(largest_o);
-        const bool faint = query < s.queries && ((!v_zero && largest_o < l_all) || (c2 > 0x1p-16f && fabsf(m_all) < 0x1p16f));
-        if (__builtin_expect(unfit || own_unfit || __ballot(probe != 0.0f || faint) != 0, 0)) {
-            exact_query_tile<D, VEC>((const SplitForwardParams *)__builtin_amdgcn_kernarg_segment_ptr(), seq, q0);
-        } else {
-            const float base = mc_all == -INFINITY ? 0.0f : mc_all;
-            // O is o / l in any offset; lse's sum is Σ exp(s - max) = l · exp2(offset - max·c2).
-            const float sum = m_all == -INFINITY ? l_all : l_all * exp2_fast(base - kShift - m_all * c2);
-            store_rows<D, VEC>(P, seq, query, h, o, l_all, __builtin_amdgcn_ldexpf(m_all * P.scale, e), sum, ev);
-        }
+        const float base = mc_all == -INFINITY ? 0.0f : mc_all;
+        // O is o / l in any offset; lse's sum is Σ exp(s - max) = l · exp2(offset - max·c2).
+        const float sum = m_all == -INFINITY ? l_all : l_all * exp2_fast(base - kShift - m_all * c2);
+        // A row that used only rows far below the ones that set the scales (hidden from it, or of no weight). Of V': where its terms
+        // are below 2^-3 they are off by 2^-25, and so are weights below 2^-10 of the largest, here times at most 2^10 sampled.
+        // Over a row of weights p / l these errors add up to at most 2^-25·√(Σ p²)/l, and Σ p² is at most l²/sum; so the row's
+        // largest |O'| must reach 2^-3/√sum, as that of normal values does by 2^10 and more. Of K': an error of 2^-25 moves a
+        // score by up to 2^-7·c2 (Q' below 2^15, errors of D features adding up at random), which must be below 2^-23, or the
+        // row's largest |S'| at least 2^16, as where its keys are at 2^-2 or more.
+        const bool faint = query < s.queries && ((!v_zero && 8.0f * largest_o * sqrtf(sum) < l_all) || (c2 > 0x1p-16f && fabsf(m_all) < 0x1p16f));
+        redo = unfit || own_unfit || __ballot(probe != 0.0f || faint) != 0;
+        if (__builtin_expect(!redo, 1)) store_rows<D, VEC>(P, seq, query, h, o, l_all, __builtin_amdgcn_ldexpf(m_all * P.scale, e), sum, ev);
+    }
+    if (stream == 0 && lane == 0) redone[qi] = redo;
+    __syncthreads(); // also: every wave is done with the stages and the merged state
+#pragma unroll 1
+    for (int x = 0; x < QB; ++x) {
+        if (__builtin_expect(__builtin_amdgcn_readfirstlane(redone[x]), 0))
+            exact_query_tile<D, VEC, QB * KS, WPE>((const SplitForwardParams *)__builtin_amdgcn_kernarg_segment_ptr(), (LdsFloats)smem, seq, (qb * QB + x) * kTile);
     }
 }
 

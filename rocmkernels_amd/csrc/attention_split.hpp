@@ -32,6 +32,7 @@ typedef _Float16 h16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h16x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 h16x2 __attribute__((ext_vector_type(2)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) float *LdsFloats;
 
 __device__ __forceinline__ f32x16 mfma_f16(const h16x8 a, const h16x8 b, const f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
@@ -104,11 +105,12 @@ __device__ __forceinline__ void workgroup_largest(float &x, float &y, float (&sl
 // The same over every live row of a window of n rows, for a scale that the sampled rows don't tell: they may all be 0 where the
 // others are not (the gradient of one token's loss), and terms of a fixed scale would lose values far below it. A workgroup of
 // THREADS threads reads ROWS rows at a time, CPR 4-float chunks each: live(row) says whether a row counts, load(row, on, a, b)
-// fetches this thread's two chunks of it (zeros unless on). Costs a pass over the window (from L2), taken only where all sampled
-// rows are 0 or masked.
+// fetches this thread's two chunks of it (zeros unless on). Returns how many of this thread's y chunks are not 0. Costs a pass
+// over the window (from L2), taken only where all sampled rows are 0 or masked.
 template<int THREADS, int CPR, class Live, class Load>
-__device__ __forceinline__ void window_largest(float &x, float &y, const int n, const Live &live, const Load &load) {
+__device__ __forceinline__ int window_largest(float &x, float &y, const int n, const Live &live, const Load &load) {
     constexpr int ROWS = THREADS / CPR, TRIP = 4;
+    int found = 0;
 #pragma unroll 1
     for (int r0 = threadIdx.x / CPR; r0 - static_cast<int>(threadIdx.x / CPR) < n; r0 += TRIP * ROWS) {
         bool on[TRIP], any = false;
@@ -126,9 +128,12 @@ __device__ __forceinline__ void window_largest(float &x, float &y, const int n, 
 #pragma unroll
         for (int u = 0; u < TRIP; ++u) {
             x = fmaxf(x, largest(a[u]));
-            y = fmaxf(y, largest(b[u]));
+            const float z = largest(b[u]);
+            y = fmaxf(y, z);
+            found += z > 0.0f;
         }
     }
+    return found;
 }
 
 // Eight floats times `scale` as an operand's two terms.
