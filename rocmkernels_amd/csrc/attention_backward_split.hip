@@ -404,6 +404,7 @@ __global__ __launch_bounds__(kWave * QB * KS) __attribute__((amdgpu_waves_per_eu
     static_assert((QB * KS - 1) * 16 * DT * kWave * 4 <= STAGE_BYTES); // the slots of exact_dq_tile
     __shared__ float amax[2][QB * KS];
     __shared__ int redone[QB]; // query tiles to compute again
+    __shared__ float norms[KS > 1 ? KS - 1 : 1][QB][kWave]; // of streams 1 ..: Σ dS'² of each lane
 
     const Shape &s = P.s;
     const int lane = threadIdx.x & (kWave - 1);
@@ -521,11 +522,11 @@ __global__ __launch_bounds__(kWave * QB * KS) __attribute__((amdgpu_waves_per_eu
     mo = halves_max(mo);
     const int eq = exponent_of(mq) - 14, eu = exponent_of(mu) - 14;
     // Rows that only use rows far below the ones that set the scales (hidden from them, or of no weight), whose terms are off by 2^-25
-    // in V' and K'. Of V': the row's weighted mean, which O is, must reach 2^-3/√l (as in the forward). Of K': the largest score tells; |S'| of 2^17 takes
-    // a key of 2^-2 or more. Rows of dO = 0 have no gradient to lose, nor have those of one key of weight 1 (dP = δ).
-    const float top_s = __builtin_amdgcn_ldexpf(P.scale, eq + ek + 17);
-    const bool faint = valid && m != -INFINITY && l > 1.0f + 0x1p-22f && mu > 0.0f &&
-            ((!v_zero && mo * sqrtf(l) < __builtin_amdgcn_ldexpf(1.0f, ev - 3)) || (!k_zero && fabsf(m) < top_s));
+    // in V' and K'. Of V': the row's weighted mean, which O is, must reach 2^-3/√l. Of K': scores must not move, as in the
+    // forward (both: see there); what K' loses in dQ' itself shows at the end. Rows of dO = 0 have no gradient to lose.
+    const float c2 = __builtin_amdgcn_ldexpf(P.scale * kLog2e, eq + ek);
+    const bool faint = valid && m != -INFINITY && mu > 0.0f && ((!v_zero && mo * sqrtf(l) < __builtin_amdgcn_ldexpf(1.0f, ev - 3)) ||
+            (c2 > 0x1p-16f && fabsf(m) < __builtin_amdgcn_ldexpf(P.scale, eq + ek + 16)));
     // Outside the range of scales: for K and V the whole workgroup keeps from the loop; for a wave's own queries only its
     // products do, as its siblings need the rows that it stages and its barriers.
     const bool unfit = !scale_fits(ek) || !scale_fits(ev), own_unfit = __ballot(!scale_fits(eq) || !scale_fits(eu) || faint) != 0;
@@ -538,7 +539,6 @@ __global__ __launch_bounds__(kWave * QB * KS) __attribute__((amdgpu_waves_per_eu
     }
     // P̃ = 2^9·exp(s - max) = exp2(S'·c2 + base); dP - δ in units of 2^(eu + ev + 23), twice the product of the largest |dO| of
     // the row and the largest sampled |V|: r = dP'·2^-23 - δ'. P̃·r then stays below 2^16 while |r| < 2^7.
-    const float c2 = __builtin_amdgcn_ldexpf(P.scale * kLog2e, eq + ek);
     const float base = m != -INFINITY ? fmaf(m, -kLog2e, 9.0f) : -INFINITY;
     const float dl = __builtin_amdgcn_ldexpf(dlt, -(eu + ev + 23));
     constexpr float kUnit = 1.0f / (1 << 23);
@@ -546,6 +546,7 @@ __global__ __launch_bounds__(kWave * QB * KS) __attribute__((amdgpu_waves_per_eu
     f32x16 acc[DT];
 #pragma unroll
     for (int t = 0; t < DT; ++t) acc[t] = f32x16{};
+    float ds_norm = 0.0f; // Σ dS'² of the lane's query over its half of the keys, from the high terms
 
     auto clear_masked = [&](const uint64_t bits) __attribute__((always_inline)) {
         if (__builtin_expect(bits != ~0ull, 0)) {
@@ -582,7 +583,8 @@ __global__ __launch_bounds__(kWave * QB * KS) __attribute__((amdgpu_waves_per_eu
     auto ds_unit = [&](auto unit, const f32x16 &sc, const f32x16 &dp, uint32_t (&ds)[2][8]) __attribute__((always_inline)) {
         constexpr int U = decltype(unit)::value, J = 2 * U;
         split_pair<false>(sc[J] * fmaf(dp[J], kUnit, -dl), sc[J + 1] * fmaf(dp[J + 1], kUnit, -dl), one, ds[0][U], ds[1][U]);
-        __asm__ volatile("" : "+v"(ds[1][U])); // here, not at its use behind the next group
+        ds_norm = add_squares(ds[0][U], ds_norm);
+        __asm__ volatile("" : "+v"(ds[1][U]), "+v"(ds_norm)); // here, not at its use behind the next group
     };
     // A whole 64-key tile without masks, halves A and B, and the staging of the next one: six groups of MFMAs, each beside
     // independent VALU work spread over it (as in the forward): Sᵀ of A with the staging of K, dPᵀ of A with A's exponentials,
@@ -697,8 +699,17 @@ __global__ __launch_bounds__(kWave * QB * KS) __attribute__((amdgpu_waves_per_eu
             if (i + 1 < nsteps) step(i + 1, 1);
         }
     }
+    if (KS > 1 && stream > 0) norms[stream - 1][qi][lane] = ds_norm;
     sum_streams<DT, KS>(acc, stream, reinterpret_cast<float *>(smem) + qi * (16 * DT * kWave) + lane, QB * 16 * DT * kWave);
-    const bool redo = stream == 0 && tile_valid && (unfit || own_unfit || !finite(acc));
+    bool redo = false;
+    if (stream == 0 && tile_valid) {
+#pragma unroll
+        for (int x = 0; x < KS - 1; ++x) ds_norm += norms[x][qi][lane];
+        // dQ' is off by 2^-25·√(Σ dS'²) from K', below 2^-21 of the largest |dQ'| if that reaches 2^-4·√(Σ dS'²).
+        const float top = halves_max(largest(acc));
+        const bool faint_k = valid && !k_zero && 256.0f * top * top < halves_sum(ds_norm);
+        redo = unfit || own_unfit || __ballot(faint_k) != 0 || !finite(acc);
+    }
     if (stream == 0 && valid && __builtin_expect(!redo, 1)) {
         const float factor = l > 0.0f ? __builtin_amdgcn_ldexpf(P.scale / l, ek + eu + ev + 23 - 9) : 0.0f;
 #pragma unroll
