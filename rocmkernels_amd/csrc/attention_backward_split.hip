@@ -1121,8 +1121,8 @@ hipError_t dispatch(const BackwardArgs &a, const int cus, hipStream_t stream) {
 // Long items (32 tiles and more) always beat the deterministic FP32 pair, whose waves pay more per tile (d = 32, 4 x 2048: 62
 // against 71 µs; d = 64, 4 x 1024: 68 against 72), if their loads are 128-bit ones (else 114 against 72). Otherwise the grid has
 // to be filled: from more than one item per CU on (d = 32, 384 items of 8 tiles: 19.6 µs against the key-block kernel's 28.8
-// and the pair's 25.4; 256 of 16: 25.5 against 24.1 for the pair) in both kernels (96 sequences, 64 queries of 2048 keys: 63
-// against 71; 6 sequences of 777 of 2001: 47.5 against 42.9), a little further at d = 64 against the key-block kernel (280 items of
+// and the pair's 25.4; 256 of 16: 25.5 against 24.1 for the pair) in both kernels (four fifths: 67 x 3 query
+// tiles, 12 key tiles: 25.9 against 20.7 for the key-block kernel; 6 sequences of 777 of 2001: 47.5 against 42.9), a little further at d = 64 against the key-block kernel (280 items of
 // 14: 47.0 against 44.3; 288, 48: 98.8 against 98.7; 308, 14: 52.4 against 63.1). Under a ramp half the pairs are seen but the
 // longest items last as long, so that the key-block kernel's balanced pieces win for longer, the more so the longer the items: at
 // d = 32 up to about two per CU (264, 88: 81 against 50; 384, 32: 38.6 against 34.5; 490, 70: 70.0 against 67.2; but 448, 8: 20.9
@@ -1130,12 +1130,20 @@ hipError_t dispatch(const BackwardArgs &a, const int cus, hipStream_t stream) {
 // 20: 69 against 67; but 768, 32: 92 against 98; 768, 8: 43.5 against 54.9; 384 of 4: 27.5 against 31.1). Against the pair d = 64
 // wins at once (384, 16: 49 against 58), and at d = 32 the pair's planned grid lasts to two per CU (384, up to 16: 26.1 against
 // 25.0; 512, up to 32: 38.7 against 46.0).
+// Sequences of one or two tiles leave most waves of a workgroup idle: against the pair's one item per wave that costs more than the
+// products save at d = 32 (600 x 1 query tile, 32: 121 against 145; 4096 x 1, 1: 44 against 90), at d = 64 only in large launches of
+// short items (4096 x 1, 1: 80 against 131). Nor do odd query tiles pay at d = 64 where they make more two-tile workgroups than
+// CUs (102 x 5, 3: 35.0 against 41.6), and short items of few launches at d = 32 (260, 3: 16.4 against 18.2).
 bool backward_split_pays(const int D, const BackwardArgs &a, const int cus, const bool vec, const bool deterministic) {
     const Work q = query_work(a), k = key_work(a);
     const int64_t items = (q.items + k.items) / 2, fewer = std::min(q.items, k.items);
-    const int tiles = std::max(q.tiles, k.tiles);
+    const int tiles = std::max(q.tiles, k.tiles), qtiles = (a.queries + kTile - 1) / kTile;
+    if (deterministic && D == 32 && qtiles == 1) return false;
     if (deterministic && vec && tiles >= 32) return true;
-    if (items <= cus || 4 * fewer < (vec ? 3ll : 4ll) * cus) return false;
+    if (items <= cus || 5 * fewer < (vec ? 4ll : 5ll) * cus) return false;
+    if (D == 32 && 4 * items <= 5ll * cus && tiles < 6) return false;
+    if (D == 64 && tiles < 16 && q.tiles > 2 && q.items <= 2ll * cus && static_cast<int64_t>(a.batch) * a.heads * ((qtiles + 1) / 2) > cus) return false;
+    if (deterministic && qtiles <= 2 && tiles <= 5 && items >= 8ll * cus) return false;
     if (!deterministic && a.radius < 0) { // against the key-block kernel
         if (!ramp(a)) return D == 32 || 8 * items > 9ll * cus;
         if (D == 32) return tiles * (2ll * cus - items) <= 5ll * cus;

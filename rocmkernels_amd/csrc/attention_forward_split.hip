@@ -721,10 +721,10 @@ void launch(const ForwardArgs &a, hipStream_t stream) {
             stream, params);
 }
 
-// Shape of the launch's work: 32-query items, 32-key tiles of the widest item, and whether item costs run from one tile to
-// all of them (a causal mask without a radius window).
+// Shape of the launch's work: sequences and their 32-query items, 32-key tiles of the widest item, and whether item costs run from
+// one tile to many over much of the sequence.
 struct Work {
-    int64_t items;
+    int64_t seqs, items;
     int tiles;
     bool ramp;
 };
@@ -732,10 +732,15 @@ struct Work {
 Work work_of(const ForwardArgs &a) {
     const Shape s{a.batch, a.heads, a.queries, a.keys, a.radius, a.causal};
     const int qtiles = (a.queries + kTile - 1) / kTile;
-    Work w{static_cast<int64_t>(qtiles) * a.batch * a.heads, 0, a.causal != 0 && a.radius < 0};
-    w.tiles = std::max(forward_item_tiles(s, qtiles / 2), forward_item_tiles(s, qtiles - 1));
-    return w;
+    const int64_t seqs = static_cast<int64_t>(a.batch) * a.heads;
+    return Work{seqs, qtiles * seqs, std::max(forward_item_tiles(s, qtiles / 2), forward_item_tiles(s, qtiles - 1)),
+            a.causal != 0 && (a.radius < 0 || a.radius >= a.queries / 2)};
 }
+
+// Query tiles and key streams of a workgroup.
+struct Workgroup {
+    int tiles, streams;
+};
 
 // Workgroup shape. Every µs below: items, key tiles per item: this choice against the next best one.
 //   * Up to two items per CU: two query tiles per workgroup, so that every CU has work, and as many key streams as LDS
@@ -749,43 +754,64 @@ Work work_of(const ForwardArgs &a) {
 //     74 against 86): there all workgroups are resident at once and the longest ones would end alone. At d = 64 eight query
 //     tiles split K and V half as often, and are taken where their workgroups fill whole rounds of the CUs (2048, 128: 195
 //     against 209; 1536, 32: 47.0 against 51.5; but 3072, 32, one and a half rounds: 97 against 88).
+Workgroup workgroup_of(const int D, const ForwardArgs &a, const Work &w, const int cus) {
+    const bool ramp = w.ramp && a.radius < 0;
+    if (w.items <= 2ll * cus) return D == 32 && w.tiles >= 20 ? Workgroup{2, 4} : Workgroup{2, 2};
+    if (w.items <= 4ll * cus) {
+        if (D == 32 && ramp) return Workgroup{2, 2};
+        if (w.tiles >= (D == 32 ? 16 : 24)) return Workgroup{4, 2};
+    } else if (ramp && w.items <= 8ll * cus && w.tiles >= (D == 32 ? 32 : 48)) {
+        return Workgroup{4, 2};
+    }
+    const int64_t wide = w.seqs * ((a.queries + 8 * kTile - 1) / (8 * kTile));
+    if (D == 64 && w.items > 4ll * cus && !ramp && a.radius < 0 && w.tiles >= 24 && (wide <= cus || wide >= 3ll * cus)) return Workgroup{8, 1};
+    return Workgroup{4, 1};
+}
+
 template<int D, bool VEC>
 void dispatch(const ForwardArgs &a, const Work &w, const int cus, hipStream_t stream) {
-    if (w.items <= 2ll * cus) {
+    const Workgroup g = workgroup_of(D, a, w, cus);
+    if (g.tiles == 2) {
         if constexpr (D == 32) {
-            if (w.tiles >= 20) return launch<D, VEC, 2, 4>(a, stream);
+            if (g.streams == 4) return launch<D, VEC, 2, 4>(a, stream);
         }
         return launch<D, VEC, 2, 2, D == 32 ? 2 : 1>(a, stream); // d = 64: its 128 KB of LDS admit one workgroup per CU
     }
-    if (w.items <= 4ll * cus) {
-        if constexpr (D == 32) {
-            if (w.ramp) return launch<D, VEC, 2, 2>(a, stream);
-        }
-        if (w.tiles >= (D == 32 ? 16 : 24)) return launch<D, VEC, 4, 2>(a, stream);
-    } else if (w.ramp && w.items <= 8ll * cus && w.tiles >= (D == 32 ? 32 : 48)) {
-        return launch<D, VEC, 4, 2>(a, stream);
-    }
     if constexpr (D == 64) {
-        const int64_t wide = static_cast<int64_t>(a.batch) * a.heads * ((a.queries + 8 * kTile - 1) / (8 * kTile));
-        if (w.items > 4ll * cus && !w.ramp && a.radius < 0 && w.tiles >= 24 && (wide <= cus || wide >= 3ll * cus)) return launch<D, VEC, 8, 1>(a, stream);
+        if (g.tiles == 8) return launch<D, VEC, 8, 1>(a, stream);
     }
+    if (g.streams == 2) return launch<D, VEC, 4, 2>(a, stream);
     launch<D, VEC, 4, 1, D == 32 ? 3 : 2>(a, stream);
 }
 
 } // namespace
 
-// Where the items are few, the FP32 kernel's four waves per item and shorter start win: up to one item per CU (d = 64, 128
-// items of 32 tiles: 22.3 against 23.9 µs; d = 32, 32 items of 8: 5.6 against 7.5), under a ramp up to two (d = 64, 384 items
-// of up to 16: 14.1 against 15.7; d = 32: 8.6 against 10.8), and at d = 32 for short items (512 of 5: 7.6 against 8.3; 1536 of
-// 3: 9.9 against 11.7). At d = 32 the FP32 kernel's planned grid, up to three items per CU, also balances what a ramp or a radius
-// window leaves uneven: it wins while the ramp is short (594 of up to 11: 9.5 against 10.4; but 768, 32: 18.2 against 17.1) or the
-// window's work small (280 of 21: 11.3 against 13.1; 552 of 11: 11.8 against 14.1; but 748 of 33: 34.3 against 23.6).
+// Where the FP32 kernel wins, from 7230 launches of 130 to 4096 items and 1 to 64 tiles on both kernels (µs: FP32 against this one;
+// by this rule three of them are slower than on the FP32 kernel by more than 3%, the worst by 6%):
+//   * Few items, whose work its four waves per item and shorter start finish sooner: up to one item per CU (d = 64, 128 of 32: 23.4
+//     against 24.6), up to two under a ramp, and above that short items (d = 64, 384 of 5: 12.6 against 12.5, of 8: 15.1 against
+//     12.9; d = 32, 384 of 8: 9.2 against 9.4, of 12: 11.8 against 10.8) and sequences of odd query tiles that make more
+//     workgroups than CUs (d = 64, 102 x 5 query tiles, 12: 24.1 against 29.9).
+//   * Waves without a query tile, if they are more than a third (d = 64, 2048 x 1 query tile, 24: 164 against 218; d = 32, 600 x 1, 16:
+//     21.3 against 37.8; but half of them for two query tiles of some keys: d = 64, 768 x 2, 8: 44.5 against 30.5).
+//   * Launches of a tile or so per item, which are all start and end (d = 64, 1024 of 1: 9.0 against 9.8; d = 32, 600 of 1: 5.9
+//     against 7.0, of 3: 8.2 both).
+//   * At d = 32 its planned grid, up to three items per CU, also balances what a ramp or a window leaves uneven: while the ramp is
+//     short (608 of up to 16: 11.4 against 12.0; 600 of 24: 15.9 both), or some waves are idle up to four per CU (900 of up to 5: 10.8
+//     against 13.6), or the window's work is small (264 of 17: 11.1 against 13.7; 768 of 33: 33.2 against 23.8; and at d = 64 up
+//     to two items per CU: 264 of 9: 13.2 against 14.5).
 bool forward_split_pays(const int D, const ForwardArgs &a, const int cus) {
     const Work w = work_of(a);
-    if (w.items <= cus || (w.ramp && w.items < 2ll * cus)) return false;
-    if (D == 64) return true;
-    if (w.items <= 3ll * cus && (w.ramp ? w.tiles < 24 : a.radius >= 0 && w.items * w.tiles < 32ll * cus)) return false;
-    return w.items <= 2ll * cus ? w.tiles >= 9 : a.radius < 0 || w.tiles >= 5 || w.items >= 16ll * cus;
+    if (w.items <= (w.ramp ? 2ll : 1ll) * cus) return false;
+    const int width = workgroup_of(D, a, w, cus).tiles, qtiles = static_cast<int>(w.items / w.seqs);
+    const int64_t groups = w.seqs * ((qtiles + width - 1) / width), waves = groups * width;
+    if (2 * waves > 3 * w.items && (waves > 2 * w.items || qtiles != 2 || w.tiles < 5 || w.items <= 3ll * cus)) return false;
+    if (w.items <= 2ll * cus)
+        return groups <= cus && (a.radius < 0 ? w.tiles >= (D == 32 ? 9 : 8) : w.items * w.tiles >= (D == 32 ? 32ll : 18ll) * cus);
+    if (D == 64) return w.tiles >= 2;
+    if (w.ramp) return w.items <= 3ll * cus ? w.tiles >= 24 : w.items <= 4ll * cus ? w.tiles >= 4 && 10 * waves <= 11 * w.items : w.tiles >= 3;
+    if (a.radius >= 0) return w.items <= 3ll * cus ? w.items * w.tiles >= 32ll * cus : w.tiles >= 5 || w.items >= 16ll * cus;
+    return w.tiles >= (w.items <= 3ll * cus ? 5 : 2);
 }
 
 void launch_forward_split(const int D, const bool vec, const ForwardArgs &a, const int cus, hipStream_t stream) {

@@ -82,6 +82,8 @@ def test_query_row_outside_the_scales(device, width, batch, heads, queries, keys
     (32, 7, 1, 2208, True), (32, 7, 1, 2300, True),  # causal ramps either side of two items per CU
     (64, 24, 1, 1023, True), (64, 24, 1, 991, True),  # and of three
     (64, 21, 1, 412, False), (64, 24, 1, 415, False),  # 273 and 312 items
+    (64, 102, 1, 160, False), (64, 85, 1, 160, False),  # more two-tile workgroups than CUs, and as many
+    (32, 52, 1, 160, False), (32, 70, 1, 160, False),  # short items, 260 and 350
 ])
 def test_default_backward_either_side_of_the_line(device, width, batch, heads, length, causal):
     q, k, v, du = normal_case(415, width, batch, heads, length, length)

@@ -28,6 +28,12 @@ SHAPES = [
     (32, 32, 1, 737, 737, -1, True),
     (32, 24, 1, 711, 711, 300, True),
     (32, 32, 1, 737, 737, 180, False),
+    # Few query tiles a sequence: waves without one, more workgroups than CUs.
+    (64, 102, 1, 160, 384, -1, False),
+    (64, 96, 1, 160, 384, -1, False),
+    (64, 400, 1, 60, 250, -1, False),
+    (32, 1100, 1, 31, 160, -1, False),
+    (32, 180, 1, 160, 160, -1, True),
 ]
 
 
