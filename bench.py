@@ -356,74 +356,35 @@ def forward_kernel_name(cfg, cus):
     return f"rk::attention_forward_kernel<{cfg['width']}, false, true, {split}, 0>"
 
 
-def forward_split_kernel_name(cfg, cus):
-    """Name rocprofv3 reports for the split-product forward instance that runs on this config, or None where the FP32-MFMA
-    kernel of forward_kernel_name runs: rk::forward_split_pays and rk::dispatch
-    (rocmkernels_amd/csrc/attention_forward_split.hip). Template arguments: head width, 16-byte vector loads, query tiles
-    per workgroup, key streams, waves per SIMD the registers are held to."""
-    width, length, radius = cfg["width"], cfg["length"], cfg["radius"]
-    qtiles = (length + 31) // 32
-    items = qtiles * cfg["batch"] * cfg["heads"]
-    ramp = radius < 0  # every config is causal
+# Workgroup shapes (tiles, streams) that the library picks for these configs on 256 CUs where the split-product kernels run (None:
+# the FP32-MFMA ones do): forward, dQ and dK/dV of either backward. tests/test_bench.py holds them against the library's own rules
+# (rocmkernels_amd/csrc/attention_forward_split.hip, attention_backward_split.hip).
+SPLIT_WORKGROUPS = {
+    1: {"forward": None, "dq": None, "dkdv": None},
+    2: {"forward": (2, 2), "dq": (2, 2), "dkdv": (2, 2)},
+    3: {"forward": (2, 2), "dq": (2, 2), "dkdv": (2, 2)},
+    4: {"forward": (4, 2), "dq": (4, 2), "dkdv": (4, 2)},
+    5: {"forward": (4, 1), "dq": (4, 1), "dkdv": (4, 1)},
+}
 
-    def tiles(qt):
-        first = max(0, 32 * qt - radius) if radius >= 0 else 0
-        return -(-(min(length, 32 * qt + 32) - first) // 32)
 
-    widest = max(tiles(qtiles // 2), tiles(qtiles - 1))
-    if items <= cus or (ramp and items < 2 * cus):
+def forward_split_kernel_name(config):
+    """Name rocprofv3 reports for the split-product forward instance that runs on a config, or None. Template arguments: head
+    width, 16-byte vector loads, query tiles per workgroup, key streams, waves per SIMD the registers are held to."""
+    shape, width = SPLIT_WORKGROUPS[config]["forward"], CONFIGS[config]["width"]
+    if shape is None:
         return None
-    if width == 32 and not (widest >= 9 if items <= 2 * cus else radius < 0 or widest >= 5 or items >= 16 * cus):
+    waves = 1 if width == 64 and shape == (2, 2) else 3 if width == 32 and shape == (4, 1) else 2
+    return f"rk::attention_forward_split_kernel<{width}, true, {shape[0]}, {shape[1]}, {waves}>"
+
+
+def backward_split_kernel_names(config):
+    """Names rocprofv3 reports for the split-product dQ and dK/dV instances of both backwards on a config, or None. Template
+    arguments: head width, 16-byte vector loads, tiles per workgroup, streams."""
+    shapes, width = SPLIT_WORKGROUPS[config], CONFIGS[config]["width"]
+    if shapes["dq"] is None:
         return None
-    if items <= 2 * cus:
-        shape = (2, 4, 2) if width == 32 and widest >= 20 else (2, 2, 2 if width == 32 else 1)
-    elif items <= 4 * cus and width == 32 and ramp:
-        shape = (2, 2, 2)
-    elif items <= 4 * cus and widest >= (16 if width == 32 else 24):
-        shape = (4, 2, 2)
-    elif 4 * cus < items <= 8 * cus and ramp and widest >= (32 if width == 32 else 48):
-        shape = (4, 2, 2)
-    else:  # (the eight-tile instance is for calls without a causal mask)
-        shape = (4, 1, 3 if width == 32 else 2)
-    return f"rk::attention_forward_split_kernel<{width}, true, {shape[0]}, {shape[1]}, {shape[2]}>"
-
-
-def backward_split_kernel_names(cfg, cus, deterministic):
-    """Names rocprofv3 reports for the split-product dQ and dK/dV instances that run on this config, or None where other
-    kernels run: rk::backward_split_pays, rk::dispatch_dq and rk::dispatch_dkdv
-    (rocmkernels_amd/csrc/attention_backward_split.hip). Template arguments: head width, 16-byte vector loads, tiles per
-    workgroup, streams."""
-    width, length, radius = cfg["width"], cfg["length"], cfg["radius"]
-    tiles = (length + 31) // 32
-    items = tiles * cfg["batch"] * cfg["heads"]
-    ramp = radius < 0 or radius >= length // 2  # every config is causal
-
-    def keys_of(qt):  # 32-key tiles a query tile sees
-        return -(-(min(length, 32 * qt + 32) - (max(0, 32 * qt - radius) if radius >= 0 else 0)) // 32)
-
-    def queries_of(kt):  # 32-query tiles that see a key tile
-        return -(-((min(length, 32 * kt + 32 + radius) if radius >= 0 else length) - 32 * kt) // 32)
-
-    dq, dkdv = max(keys_of(tiles // 2), keys_of(tiles - 1)), max(queries_of(0), queries_of(tiles // 2))
-    widest = max(dq, dkdv)
-    if not (deterministic and widest >= 32):
-        if items <= cus:
-            return None
-        if ramp and width == 32 and (deterministic or radius >= 0) and items < 2 * cus:
-            return None
-        if ramp and width == 64 and not (items > 2 * cus or widest <= 4 or (deterministic and radius < 0)):
-            return None
-    if (dq > 2) if items <= 2 * cus else (ramp and items <= 4 * cus and dq >= width // 2):
-        first = (2, 2)
-    else:
-        first = (4, 2) if dq >= 64 and items <= (8 if ramp else 4) * cus else (4, 1)
-    second = (4, 1)
-    if items <= 2 * cus:
-        second = (2, 4) if dkdv >= 16 else (2, 2) if dkdv > 2 else (4, 1)
-    elif (width == 32 or dkdv > 4) if items <= 4 * cus else (ramp and items <= 8 * cus and dkdv >= width // 2):
-        second = (4, 2) if width == 64 or (not ramp and dkdv >= 16) else (2, 2)
-    return [f"rk::attention_{name}_split_kernel<{width}, true, {shape[0]}, {shape[1]}>"
-            for name, shape in (("dq", first), ("dkdv", second))]
+    return [f"rk::attention_{name}_split_kernel<{width}, true, {shapes[name][0]}, {shapes[name][1]}>" for name in ("dq", "dkdv")]
 
 
 def traffic_table():
@@ -728,7 +689,7 @@ def main():
     measured = measure(cfg, args.steps, args.warmup, backward=not args.no_backward)
     fwd = measured["forward"]
     cus = torch.cuda.get_device_properties(0).multi_processor_count
-    split = forward_split_kernel_name(cfg, cus)
+    split = forward_split_kernel_name(args.config)
     kernel = split or forward_kernel_name(cfg, cus)
     peak = PEAK_SPLIT_TFLOPS if split else PEAK_FP32_MFMA_TFLOPS
     result = {
@@ -764,8 +725,7 @@ def main():
     for part in ("backward", "backward_deterministic"):
         if part in measured:
             result[part] = rounded(measured[part])
-            names = backward_split_kernel_names(cfg, cus, part == "backward_deterministic")
-            result[part]["traffic"] = backward_traffic(args.config, part, names)
+            result[part]["traffic"] = backward_traffic(args.config, part, backward_split_kernel_names(args.config))
     result["rotary"] = measure_rotary(cfg, args.steps, args.warmup)
     result["generic_forward"] = measure_generic(cfg, args.steps)
     if args.config == 2:

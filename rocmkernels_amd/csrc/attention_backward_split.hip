@@ -1073,6 +1073,8 @@ Work key_work(const BackwardArgs &a) {
 // Whether item costs run from one tile to many over much of the sequence.
 bool ramp(const BackwardArgs &a) { return a.causal != 0 && (a.radius < 0 || a.radius >= a.queries / 2); }
 
+} // namespace
+
 // Workgroup shapes. Every µs below: items, tiles of the widest: this choice against the next best one.
 //   Kernel 1. Up to two items per CU two query tiles and two streams, so that every CU has work (d = 32: 256, 64: 28.2 against
 //   37.2; d = 64: 384, 32: 18.3 against 22.3), also under a ramp up to four if its items are long, where the longest end last
@@ -1080,12 +1082,11 @@ bool ramp(const BackwardArgs &a) { return a.causal != 0 && (a.radius < 0 || a.ra
 //   and the workgroups few (1024, 64: d = 32 48.1 against 50.2, d = 64 84.5 against 86.4; ramps of 2048, 128: 99.7 against 107.9
 //   and 169 against 184). Else four and one, whose waves are in step with the fewest others (d = 32: 3072, 32: 72.9 against
 //   85.0; d = 64: 123 against 143; 768, 8: 10.1 against 11.4).
-template<int D, bool VEC>
-void dispatch_dq(const BackwardArgs &a, const int cus, hipStream_t stream) {
+SplitWorkgroup dq_split_workgroup(const int D, const BackwardArgs &a, const int cus) {
     const Work w = query_work(a);
-    if (w.items <= 2ll * cus ? w.tiles > 2 : ramp(a) && w.items <= 4ll * cus && w.tiles >= D / 2) return launch_dq<D, VEC, 2, 2>(a, stream);
-    if (w.tiles >= 64 && w.items <= (ramp(a) ? 8ll : 4ll) * cus) return launch_dq<D, VEC, 4, 2>(a, stream);
-    launch_dq<D, VEC, 4, 1>(a, stream);
+    if (w.items <= 2ll * cus ? w.tiles > 2 : ramp(a) && w.items <= 4ll * cus && w.tiles >= D / 2) return SplitWorkgroup{2, 2};
+    if (w.tiles >= 64 && w.items <= (ramp(a) ? 8ll : 4ll) * cus) return SplitWorkgroup{4, 2};
+    return SplitWorkgroup{4, 1};
 }
 
 //   Kernel 2. Up to two items per CU two key tiles and four streams if the items are long (d = 32: 512, 128: 72 against 89; d =
@@ -1094,17 +1095,33 @@ void dispatch_dq(const BackwardArgs &a, const int cus, hipStream_t stream) {
 //   without a ramp (768, 32: 33.6 against 35.4) and at d = 64, where the steps of a workgroup with more key tiles share more
 //   (768, 32: 60.4 against 71.5; ramp of 2048, 128: 242 against 290). Else four and one (3072, 32: 107 against 116 and 198
 //   against 203; 2048, 8: 24.0 against 28.6).
-template<int D, bool VEC>
-void dispatch_dkdv(const BackwardArgs &a, const int cus, hipStream_t stream) {
+SplitWorkgroup dkdv_split_workgroup(const int D, const BackwardArgs &a, const int cus) {
     const Work w = key_work(a);
     if (w.items <= 2ll * cus) {
-        if (w.tiles >= 16) return launch_dkdv<D, VEC, 2, 4>(a, stream);
-        if (w.tiles > 2) return launch_dkdv<D, VEC, 2, 2>(a, stream);
+        if (w.tiles >= 16) return SplitWorkgroup{2, 4};
+        if (w.tiles > 2) return SplitWorkgroup{2, 2};
     } else if (w.items <= 4ll * cus ? D == 32 || w.tiles > 4 : ramp(a) && w.items <= 8ll * cus && w.tiles >= D / 2) {
-        if (D == 64 || (!ramp(a) && w.tiles >= 16)) return launch_dkdv<D, VEC, 4, 2>(a, stream);
-        if constexpr (D == 32) return launch_dkdv<D, VEC, 2, 2>(a, stream);
+        return D == 64 || (!ramp(a) && w.tiles >= 16) ? SplitWorkgroup{4, 2} : SplitWorkgroup{2, 2};
     }
-    launch_dkdv<D, VEC, 4, 1>(a, stream);
+    return SplitWorkgroup{4, 1};
+}
+
+namespace {
+
+template<int D, bool VEC>
+void dispatch_dq(const BackwardArgs &a, const int cus, hipStream_t stream) {
+    const SplitWorkgroup g = dq_split_workgroup(D, a, cus);
+    if (g.tiles == 2) launch_dq<D, VEC, 2, 2>(a, stream);
+    else if (g.streams == 2) launch_dq<D, VEC, 4, 2>(a, stream);
+    else launch_dq<D, VEC, 4, 1>(a, stream);
+}
+
+template<int D, bool VEC>
+void dispatch_dkdv(const BackwardArgs &a, const int cus, hipStream_t stream) {
+    const SplitWorkgroup g = dkdv_split_workgroup(D, a, cus);
+    if (g.tiles == 2) g.streams == 4 ? launch_dkdv<D, VEC, 2, 4>(a, stream) : launch_dkdv<D, VEC, 2, 2>(a, stream);
+    else if (g.streams == 2) launch_dkdv<D, VEC, 4, 2>(a, stream);
+    else launch_dkdv<D, VEC, 4, 1>(a, stream);
 }
 
 template<int D, bool VEC>

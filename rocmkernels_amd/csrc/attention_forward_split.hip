@@ -737,10 +737,7 @@ Work work_of(const ForwardArgs &a) {
             a.causal != 0 && (a.radius < 0 || a.radius >= a.queries / 2)};
 }
 
-// Query tiles and key streams of a workgroup.
-struct Workgroup {
-    int tiles, streams;
-};
+} // namespace
 
 // Workgroup shape. Every µs below: items, key tiles per item: this choice against the next best one.
 //   * Up to two items per CU: two query tiles per workgroup, so that every CU has work, and as many key streams as LDS
@@ -754,23 +751,26 @@ struct Workgroup {
 //     74 against 86): there all workgroups are resident at once and the longest ones would end alone. At d = 64 eight query
 //     tiles split K and V half as often, and are taken where their workgroups fill whole rounds of the CUs (2048, 128: 195
 //     against 209; 1536, 32: 47.0 against 51.5; but 3072, 32, one and a half rounds: 97 against 88).
-Workgroup workgroup_of(const int D, const ForwardArgs &a, const Work &w, const int cus) {
+SplitWorkgroup forward_split_workgroup(const int D, const ForwardArgs &a, const int cus) {
+    const Work w = work_of(a);
     const bool ramp = w.ramp && a.radius < 0;
-    if (w.items <= 2ll * cus) return D == 32 && w.tiles >= 20 ? Workgroup{2, 4} : Workgroup{2, 2};
+    if (w.items <= 2ll * cus) return D == 32 && w.tiles >= 20 ? SplitWorkgroup{2, 4} : SplitWorkgroup{2, 2};
     if (w.items <= 4ll * cus) {
-        if (D == 32 && ramp) return Workgroup{2, 2};
-        if (w.tiles >= (D == 32 ? 16 : 24)) return Workgroup{4, 2};
+        if (D == 32 && ramp) return SplitWorkgroup{2, 2};
+        if (w.tiles >= (D == 32 ? 16 : 24)) return SplitWorkgroup{4, 2};
     } else if (ramp && w.items <= 8ll * cus && w.tiles >= (D == 32 ? 32 : 48)) {
-        return Workgroup{4, 2};
+        return SplitWorkgroup{4, 2};
     }
     const int64_t wide = w.seqs * ((a.queries + 8 * kTile - 1) / (8 * kTile));
-    if (D == 64 && w.items > 4ll * cus && !ramp && a.radius < 0 && w.tiles >= 24 && (wide <= cus || wide >= 3ll * cus)) return Workgroup{8, 1};
-    return Workgroup{4, 1};
+    if (D == 64 && w.items > 4ll * cus && !ramp && a.radius < 0 && w.tiles >= 24 && (wide <= cus || wide >= 3ll * cus)) return SplitWorkgroup{8, 1};
+    return SplitWorkgroup{4, 1};
 }
 
+namespace {
+
 template<int D, bool VEC>
-void dispatch(const ForwardArgs &a, const Work &w, const int cus, hipStream_t stream) {
-    const Workgroup g = workgroup_of(D, a, w, cus);
+void dispatch(const ForwardArgs &a, const int cus, hipStream_t stream) {
+    const SplitWorkgroup g = forward_split_workgroup(D, a, cus);
     if (g.tiles == 2) {
         if constexpr (D == 32) {
             if (g.streams == 4) return launch<D, VEC, 2, 4>(a, stream);
@@ -803,7 +803,7 @@ void dispatch(const ForwardArgs &a, const Work &w, const int cus, hipStream_t st
 bool forward_split_pays(const int D, const ForwardArgs &a, const int cus) {
     const Work w = work_of(a);
     if (w.items <= (w.ramp ? 2ll : 1ll) * cus) return false;
-    const int width = workgroup_of(D, a, w, cus).tiles, qtiles = static_cast<int>(w.items / w.seqs);
+    const int width = forward_split_workgroup(D, a, cus).tiles, qtiles = static_cast<int>(w.items / w.seqs);
     const int64_t groups = w.seqs * ((qtiles + width - 1) / width), waves = groups * width;
     if (2 * waves > 3 * w.items && (waves > 2 * w.items || qtiles != 2 || w.tiles < 5 || w.items <= 3ll * cus)) return false;
     if (w.items <= 2ll * cus)
@@ -815,9 +815,8 @@ bool forward_split_pays(const int D, const ForwardArgs &a, const int cus) {
 }
 
 void launch_forward_split(const int D, const bool vec, const ForwardArgs &a, const int cus, hipStream_t stream) {
-    const Work w = work_of(a);
-    if (D == 32) vec ? dispatch<32, true>(a, w, cus, stream) : dispatch<32, false>(a, w, cus, stream);
-    else vec ? dispatch<64, true>(a, w, cus, stream) : dispatch<64, false>(a, w, cus, stream);
+    if (D == 32) vec ? dispatch<32, true>(a, cus, stream) : dispatch<32, false>(a, cus, stream);
+    else vec ? dispatch<64, true>(a, cus, stream) : dispatch<64, false>(a, cus, stream);
 }
 
 } // namespace rk

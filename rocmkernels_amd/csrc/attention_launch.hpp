@@ -87,6 +87,10 @@ hipError_t launch_forward(int D, bool statistics_only, const ForwardArgs &a, hip
 // FP32 forward on the fp16 matrix cores (attention_forward_split.hip), D = 32 or 64: whether it is the faster one for the
 // call, and its launch (vec: every pointer 16-byte aligned, every stride a multiple of 4).
 bool forward_split_pays(int D, const ForwardArgs &a, int cus);
+struct SplitWorkgroup {
+    int tiles, streams; // 32-row tiles it owns and streams of the other operand's tiles
+};
+SplitWorkgroup forward_split_workgroup(int D, const ForwardArgs &a, int cus);
 void launch_forward_split(int D, bool vec, const ForwardArgs &a, int cus, hipStream_t stream);
 
 struct RotaryArgs {
@@ -117,6 +121,8 @@ hipError_t launch_backward(int D, BackwardStage stage, const BackwardArgs &a, hi
 // the call than the deterministic FP32 pair (deterministic) or what kBackwardAuto would run instead, and its launch (vec: every
 // pointer 16-byte aligned, every stride a multiple of 4).
 bool backward_split_pays(int D, const BackwardArgs &a, int cus, bool vec, bool deterministic);
+SplitWorkgroup dq_split_workgroup(int D, const BackwardArgs &a, int cus);
+SplitWorkgroup dkdv_split_workgroup(int D, const BackwardArgs &a, int cus);
 hipError_t launch_backward_split(int D, bool vec, const BackwardArgs &a, int cus, hipStream_t stream);
 
 // Fused single-kernel backward over key blocks (attention_backward_fused.hip) for D = 32 or 64 with 128-bit access

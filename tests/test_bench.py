@@ -46,6 +46,28 @@ def test_forward_kernel_names_follow_the_launch_policy():
     assert bench.forward_kernel_name(bench.CONFIGS[5], 256) == "rk::attention_forward_kernel<64, false, true, 1, 0>"
 
 
+def test_split_kernels_follow_the_library_rules(tmp_path):
+    # The table of kernels that bench.py names against the functions the library launches by (host code of the static library).
+    from rocmkernels_amd import attention
+
+    archive = os.path.join(os.path.dirname(attention.library_path()), "libROCmKernels.Kernels.a")
+    binary = str(tmp_path / "split_rule_check")
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Wextra", "-Werror", "-D__HIP_PLATFORM_AMD__", f"-I{ROOT}/include",
+                    f"-I{ROOT}/rocmkernels_amd/csrc", "-I/opt/rocm/include", os.path.join(ROOT, "tests", "cpp", "split_rule_check.cpp"),
+                    archive, "-o", binary, "-L/opt/rocm/lib", "-Wl,-rpath,/opt/rocm/lib", "-lamdhip64"], check=True, capture_output=True,
+                   text=True)
+    launches = [str(cfg[key]) for cfg in bench.CONFIGS.values() for key in ("width", "batch", "heads", "length", "radius")]
+    lines = subprocess.run([binary, *launches], check=True, capture_output=True, text=True, timeout=60).stdout.splitlines()
+    assert len(lines) == len(bench.CONFIGS)
+    for config, line in zip(bench.CONFIGS, lines):
+        *shapes, forward, default, deterministic = (int(x) for x in line.split())
+        want = {name: tuple(shapes[2 * i:2 * i + 2]) if runs else None
+                for i, (name, runs) in enumerate((("forward", forward), ("dq", default), ("dkdv", default)))}
+        assert bench.SPLIT_WORKGROUPS[config] == want, config
+        assert default == deterministic, config
+    assert bench.forward_split_kernel_name(4) == "rk::attention_forward_split_kernel<64, true, 4, 2, 2>"
+
+
 def test_roofline_kernels_have_profiled_traffic():
     # The kernel each config's roofline names, and every kernel of each backward, has a counter row in
     # profiles/traffic.json (rocprofv3 FETCH_SIZE / WRITE_SIZE of the same instance).
