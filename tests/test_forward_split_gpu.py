@@ -6,14 +6,14 @@ import pytest
 import torch
 
 import oracle
-from parity import check_forward, host, norm_rel, normal_case, padding_mask, reference64, to_dev
+from parity import check_forward, fp32_score_floor, host, norm_rel, normal_case, padding_mask, reference64, to_dev
 from rocmkernels_amd import attention
 
 pytestmark = pytest.mark.gpu
 
 # (width, batch, heads, queries, keys, radius, causal): each workgroup shape on a 256-CU device, sizes off every tile edge.
 SHAPES = [
-    (32, 8, 1, 2043, 2043, -1, True),     # two query tiles, four key streams
+    (32, 8, 1, 2043, 2043, -1, False),    # two query tiles, four key streams
     (32, 24, 1, 500, 470, -1, False),     # two and two
     (32, 24, 1, 1000, 1000, -1, True),    # two and two, causal ramp
     (32, 24, 1, 1001, 999, -1, False),    # four and two
@@ -24,13 +24,15 @@ SHAPES = [
     (64, 48, 2, 515, 515, 77, False),     # four and one
     (64, 17, 1, 1023, 33, -1, False),     # fewer keys than one 64-key step
     # Either side of the line to the FP32 kernel's planned grid: short ramps, small windows.
+    (32, 8, 1, 2043, 2043, -1, True),
+    (32, 9, 1, 2043, 2043, -1, True),
     (32, 32, 1, 735, 735, -1, True),
     (32, 32, 1, 737, 737, -1, True),
     (32, 24, 1, 711, 711, 300, True),
     (32, 32, 1, 737, 737, 180, False),
     # Few query tiles a sequence: waves without one, more workgroups than CUs.
     (64, 102, 1, 160, 384, -1, False),
-    (64, 96, 1, 160, 384, -1, False),
+    (64, 85, 1, 160, 384, -1, False),
     (64, 400, 1, 60, 250, -1, False),
     (32, 1100, 1, 31, 160, -1, False),
     (32, 180, 1, 160, 160, -1, True),
@@ -141,6 +143,20 @@ def test_large_rows_outside_the_result(device, width, batch, heads, queries, key
             continue
         for name, got in (("output", out), ("lse", lse)):
             assert norm_rel(got[b, 0, rows], want[name][b, 0, rows]) <= 1e-6, (b, name)
+
+
+@pytest.mark.parametrize("gain", [3.0, 6.0])
+@pytest.mark.parametrize("width,batch,heads,queries,keys,radius,causal", SHAPES[1:9])
+def test_large_scores(device, width, batch, heads, queries, keys, radius, causal, gain):
+    # Q and K scaled by `gain`: row maxima of 40 to 180, each row's weights on a few keys. O and lse within 1e-5, or twice what
+    # plain FP32 dot products for the scores alone cost, where that is more (as test_attention_gpu.py::test_large_logits). The first
+    # head of four batch entries is compared.
+    q, k, v, _ = normal_case(360 + width + queries, width, batch, heads, queries, keys)
+    mask = np.ones((batch, keys), np.uint8)
+    out, lse = host(*attention.forward(*to_dev(device, q * np.float32(gain), k * np.float32(gain), v, mask), radius=radius, causal=causal))
+    q, k, v, mask = q[:4, :1] * np.float32(gain), k[:4, :1] * np.float32(gain), v[:4, :1], mask[:4]
+    want = oracle.attention(q, k, v, mask, radius=radius, causal=causal)
+    check_forward(out[:4, :1], lse[:4, :1], want, f"large scores d{width}", floor=fp32_score_floor(q, k, v, mask, radius, causal))
 
 
 @pytest.mark.parametrize("width", [32, 64])
