@@ -579,9 +579,11 @@ def f16_valu_ceiling_us(tiles):
 def measure_generic(cfg, steps):
     """attention_generic_forward (the reference's Generic/Attention/AttentionGeneric.hip:36-309) on the config's Q, K,
     V and radius with fp32 and fp16 storage. The generic entry point has no causal flag, so every (query, key) pair
-    inside the radius window is visited. fp32 storage runs the FP32 MFMA kernel; fp16 storage runs v_mfma_f32_32x32x16_f16, whose matrix work per
-    tile is 1/16 of the FP32 kernel's, so it is bound by the softmax VALU work (exp, max, sum: about 62 operations
-    and 16 exponentials per 32 x 32 tile and wave) rather than by the FP16 matrix peak it is reported against."""
+    inside the radius window is visited. fp32 storage runs the split-product kernel (each product from three fp16 ones) from more
+    than one 32-query tile per CU on, as every config but the smallest has, else the FP32 MFMA kernel; fp16 storage runs
+    v_mfma_f32_32x32x16_f16, whose matrix work per tile is 1/16 of the FP32 kernel's, so it is bound by the softmax VALU work
+    (exp, max, sum: about 62 operations and 16 exponentials per 32 x 32 tile and wave) rather than by the FP16 matrix peak it
+    is reported against."""
     import torch
 
     from rocmkernels_amd import attention
@@ -598,7 +600,9 @@ def measure_generic(cfg, steps):
         pairs = batch * heads * sum(per_query)
     flops = 4.0 * width * pairs
     out = {}
-    for name, dtype, peak in (("f32", torch.float32, PEAK_FP32_MFMA_TFLOPS), ("f16", torch.float16, PEAK_FP16_MFMA_TFLOPS)):
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    peak_f32 = PEAK_SPLIT_TFLOPS if batch * heads * ((length + 31) // 32) > cus else PEAK_FP32_MFMA_TFLOPS
+    for name, dtype, peak in (("f32", torch.float32, peak_f32), ("f16", torch.float16, PEAK_FP16_MFMA_TFLOPS)):
         q, k, v = (t.to(dtype) for t in (q32, k32, v32))
         o = torch.empty_like(q)
         lse = torch.empty((batch, heads, length, 2), device=device)
@@ -610,7 +614,7 @@ def measure_generic(cfg, steps):
         timing = time_samples(launch, [o, lse], steps)
         tflops = flops / (timing["ms_per_launch"] * 1e-3) / 1e12
         out[name] = {"ms_per_launch": round(timing["ms_per_launch"], 6), "ms_min": round(timing["ms_min"], 6),
-                     "ms_p95": round(timing["ms_p95"], 6), "tflops_visited": round(tflops, 4), "peak_tflops": peak,
+                     "ms_p95": round(timing["ms_p95"], 6), "tflops_visited": round(tflops, 4), "peak_tflops": round(peak, 1),
                      "frac_of_mfma_peak": round(tflops / peak, 4), "samples": timing["samples"],
                      "launches_per_sample": timing["launches_per_sample"]}
         if name == "f16":

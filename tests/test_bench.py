@@ -65,12 +65,18 @@ def test_split_kernels_follow_the_library_rules(tmp_path):
                 for i, (name, runs) in enumerate((("forward", forward), ("dq", default), ("dkdv", default)))}
         assert bench.SPLIT_WORKGROUPS[config] == want, config
         assert default == deterministic, config
+        if forward: # profiles/traffic.json has a row for each kernel that runs
+            assert bench.load_traffic(bench.forward_split_kernel_name(config), config) is not None, config
+        if default:
+            for part in ("backward", "backward_deterministic"):
+                assert bench.backward_traffic(config, part, bench.backward_split_kernel_names(config)) is not None, config
     assert bench.forward_split_kernel_name(4) == "rk::attention_forward_split_kernel<64, true, 4, 2, 2>"
 
 
 def test_roofline_kernels_have_profiled_traffic():
-    # The kernel each config's roofline names, and every kernel of each backward, has a counter row in
-    # profiles/traffic.json (rocprofv3 FETCH_SIZE / WRITE_SIZE of the same instance).
+    # The FP32 kernels that ran these configs before the split-product ones keep their counter rows in profiles/traffic.json
+    # (rocprofv3 FETCH_SIZE / WRITE_SIZE of the same instance); test_split_kernels_follow_the_library_rules checks the rows
+    # of the kernels that run now.
     for config in (2, 3, 4, 5):
         name = bench.forward_kernel_name(bench.CONFIGS[config], 256)
         assert bench.load_traffic(name, config) is not None, (config, name)
