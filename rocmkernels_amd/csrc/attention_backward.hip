@@ -825,11 +825,13 @@ hipError_t run(BackwardStage stage, const BackwardArgs &a, const int cus, hipStr
     const int64_t kitems = static_cast<int64_t>((a.keys + kTile - 1) / kTile) * a.batch * a.heads;
     const int64_t kblocks = static_cast<int64_t>((a.keys + kBlockKeys - 1) / kBlockKeys) * a.batch * a.heads;
     // Auto and the deterministic backward take the pair on the fp16 matrix cores wherever it pays (backward_split_pays: more
-    // than about one 32-row item per CU). Below, Auto takes the fused kernels wherever they exist (128-bit access; without it
+    // than about one 32-row item per CU). Elsewhere Auto takes the fused kernels wherever they exist (128-bit access; without it
     // the deterministic FP32 pair measured faster), under a radius window only if they fill the CUs: the band kernel runs one
     // persistent workgroup per 128-key block and never splits a block, while the pair spreads 32-row tiles over every CU:
     // measured, causal, 1 x 8192 at D = 64, radius 256 (64 blocks) 64.9 against 40.0 us, 2 x 8192 (128 blocks) 67.5 against
-    // 59.0 us; at D = 32, 64 / 128 blocks 38.0 / 39.1 against 22.2 / 32.0 us; 256 blocks 42.4 against 58.3.
+    // 59.0 us; at D = 32, 64 / 128 blocks 38.0 / 39.1 against 22.2 / 32.0 us; 256 blocks 42.4 against 58.3. As many blocks as
+    // that mean four times as many key tiles, so Auto reaches the band kernel mainly where blocks are mostly padding (sequences
+    // of about one block) or queries are few against the keys; otherwise the pair on the fp16 matrix cores has taken the call.
     if ((stage == kBackwardAuto || stage == kBackwardAll) && backward_split_pays(D, a, cus, VEC, stage == kBackwardAll || !VEC))
         return launch_backward_split(D, VEC, a, cus, stream);
     if (stage == kBackwardAuto) {

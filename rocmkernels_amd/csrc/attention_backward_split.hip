@@ -22,12 +22,12 @@
 //
 // What bounds them: 21 fp16 MFMAs of 32 x 32 x 16 per 32 x 32 tile and 16 columns of width in the two (12 and 9) do what 7 x 8 FP32
 // ones of twice the time did, beside 16 exponentials and about 100 other VALU instructions per lane and kernel; at d = 64, 32 x
-// 2048 causal, MFMAs take a third of the SIMD cycles, VALU issue a fifth to a third, and waits a third of the wave cycles: with
-// the terms of two operands and the accumulators in registers only two waves fit a SIMD. Measured, whole
-// backward, against the faster FP32 one before (µs): d = 64, 32 x 2048 causal, padded 390 -> 215 (dQ 91, dK/dV 126), 16 x 8192
-// causal, radius 256 263 -> 174 (71 and 98), 96 x 2048 full 2109 -> 1128; d = 32, 24 x 1024 causal 54.8 -> 46.4 (19.2 and 27.0),
-// full and deterministic 99.6 -> 58.6, 96 x 2048 full 1069 -> 623. Errors against 64 bits fell too (dQ 3e-7, dK and dV 4e-7 to
-// 6e-7 of the norm, FP32 pair 4e-7 to 1.1e-6): fp16 products are exact and their terms are summed 16 at a time.
+// 2048 causal, MFMAs take a third of the SIMD cycles, VALU issue a third, and waits a third of the wave cycles: with the terms
+// of two operands and the accumulators in registers only two waves fit a SIMD. Measured, whole backward, back-to-back launches,
+// against the deterministic FP32 pair (µs): d = 64, 32 x 2048 causal 510 -> 232, 96 x 2048 full 2640 -> 1067; d = 32, 24 x 1024
+// full 103 -> 69, 96 x 2048 full 1353 -> 622; against the fused FP32 kernels 16 x 8192 causal, radius 256 257 -> 172, 24 x 1024
+// causal at d = 32 54.6 -> 50.7. Errors against 64 bits fell too (dQ 3e-7, dK and dV 4e-7 to 6e-7 of the norm, FP32 pair 4e-7 to
+// 1.1e-6, N(0,1) values): fp16 products are exact and their terms are summed 16 at a time.
 #include <algorithm>
 
 #include "attention_launch.hpp"

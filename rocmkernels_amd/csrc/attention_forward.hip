@@ -399,7 +399,10 @@ bool launch_planned(const ForwardArgs &a, const Plan &plan, hipStream_t stream) 
 // (two waves per SIMD at d = 64, three at d <= 32) win, since a wave's start and the merge of an item's waves cost more
 // than they balance: config 5 forward 90.2 µs with one wave per item against 96.5 with two and 114.4 with four; without
 // a mask, 32 x 2048 at d = 64 256.8 against 266.6 µs (four waves) and 16 x 8192 at d = 64, radius 256, 149.9 against
-// 158.3 µs (two).
+// 158.3 µs (two). These are this kernel's times with an output. At d >= 32 such launches with an output now run
+// attention_forward_split.hip in less; the rule stays for the statistics-only entry point and 16-wide heads at every
+// size, and for what forward_split_pays leaves here: few items, and large launches of one query tile a sequence or, at
+// d = 32 and 64, of one key tile (4096 x 32 queries, 1024 x 32 keys).
 template<int D>
 int dispatch_split(const ForwardArgs &a, const int64_t items, const int cus) {
     // A radius window over more than a quarter of the sequence ramps item costs up over most of it.

@@ -17,9 +17,9 @@
 // Scales (powers of two): each query row its own; K and V one each for the workgroup, from the largest magnitudes of rows
 // sampled over its window (of all its rows where the sampled ones are 0). They put those at 2^8 (K) and 2^9 (V), so rows up to
 // 64 times larger than any sampled one are still in range; larger ones make the result NaN. A query tile is computed again with
-// FP32 MFMAs, by the whole workgroup, where its wave finds a non-finite result (as it must anyway for infinities, whose meaning the split products lose)
-// or a row whose keys and values all lie so far below the scales that their terms lost bits: the rows that set a scale may
-// be hidden from it by the masks, or have no weight.
+// FP32 MFMAs, by the whole workgroup, where its wave finds a non-finite result (as it must anyway for infinities, whose
+// meaning the split products lose) or a row whose keys and values all lie so far below the scales that their terms lost
+// bits: the rows that set a scale may be hidden from it by the masks, or have no weight.
 #include <algorithm>
 #include <type_traits>
 
@@ -85,8 +85,8 @@ __device__ __forceinline__ void store_rows(const SplitForwardParams &P, const in
 // One query tile on FP32 MFMAs by the workgroup's WAVES waves, for inputs that the split products cannot carry: the arithmetic of
 // attention_forward.hip, operands straight from memory, K a tile ahead. The waves take alternate key tiles and are merged in order
 // through `slots` (3 + D/2 floats a lane for each wave but one). Kept out of line (and given the kernel's arguments by
-// address), so that the main loop's registers do not depend on it, and one for each register budget of a kernel (WPE). With one wave a tile instead, a single tile that needed
-// it held its launch up for 200 µs (24 x 1024 at width 32).
+// address), so that the main loop's registers do not depend on it, and one for each register budget of a kernel (WPE). With
+// one wave a tile instead, a single tile that needed it held its launch up for 200 µs (24 x 1024 at width 32).
 template<int D, bool VEC, int WAVES, int WPE>
 __device__ __attribute__((noinline)) void exact_query_tile(const SplitForwardParams *params, LdsFloats slots, const int seq_, const int q0_) {
     const auto address = reinterpret_cast<uint64_t>(params);
@@ -278,12 +278,6 @@ __global__ __launch_bounds__(kWave * QB * KS) __attribute__((amdgpu_waves_per_eu
         vread[t2] = v_chunk<D>(4 * h + ((lane & 15) >> 2), 4 * t2 + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) + 4 * (lane & 1);
     uint16_t *const stages = reinterpret_cast<uint16_t *>(smem) + stream * (2 * STAGE);
 
-    auto load4 = [&](const Buffer r, const uint32_t voffset, const uint32_t soffset) __attribute__((always_inline)) {
-        if constexpr (VEC) return buffer_load4(r, voffset, soffset);
-        else return f32x4{buffer_load(r, voffset, soffset), buffer_load(r, voffset + 4u, soffset), buffer_load(r, voffset + 8u, soffset),
-                buffer_load(r, voffset + 12u, soffset)};
-    };
-
     const int qb = s.causal ? nblocks - 1 - rank : rank;
     const int q0 = (qb * QB + qi) * kTile;
     const int query = q0 + col;
@@ -309,7 +303,7 @@ __global__ __launch_bounds__(kWave * QB * KS) __attribute__((amdgpu_waves_per_eu
     auto load_chunks = [&](f32x4 (&raw)[CH], const Buffer buf, const uint32_t at, const uint32_t step, const int i) __attribute__((always_inline)) {
         const uint32_t row0 = i * KS + stream < ntiles ? static_cast<uint32_t>(tile_key(i)) * step : kNoRow;
 #pragma unroll
-        for (int c = 0; c < CH; ++c) raw[c] = load4(buf, at, row0 + static_cast<uint32_t>(RPC * c) * step);
+        for (int c = 0; c < CH; ++c) raw[c] = load_chunk<VEC>(buf, at, row0 + static_cast<uint32_t>(RPC * c) * step);
     };
     // Scales. Every thread reads a chunk of K and V in one of ROWS rows spread over the workgroup's window; masked rows
     // (keys past the end too) count as 0.
@@ -326,13 +320,13 @@ __global__ __launch_bounds__(kWave * QB * KS) __attribute__((amdgpu_waves_per_eu
         const int key = ufirst + (n > 0 ? static_cast<int>(static_cast<int64_t>(static_cast<int>(threadIdx.x) / CPR) * n / ROWS) : 0);
         const uint32_t at = 16u * (threadIdx.x % CPR);
         const int seen = buffer_load_byte(mbuf, static_cast<uint32_t>(key));
-        const f32x4 x = load4(kbuf, static_cast<uint32_t>(key) * kstep + at, 0), y = load4(vbuf, static_cast<uint32_t>(key) * vstep + at, 0);
+        const f32x4 x = load_chunk<VEC>(kbuf, static_cast<uint32_t>(key) * kstep + at, 0), y = load_chunk<VEC>(vbuf, static_cast<uint32_t>(key) * vstep + at, 0);
         // Q and the first tile behind them: one round trip for all.
 #pragma unroll
         for (int i = 0; i < KC; ++i) {
             const uint32_t at = tile_valid ? static_cast<uint32_t>(query) * qstep + 4u * (16 * i + 8 * h) : kNoRow;
-            qraw[2 * i] = load4(qbuf, at, 0);
-            qraw[2 * i + 1] = load4(qbuf, at + 16u, 0);
+            qraw[2 * i] = load_chunk<VEC>(qbuf, at, 0);
+            qraw[2 * i + 1] = load_chunk<VEC>(qbuf, at + 16u, 0);
         }
         load_chunks(kraw, kbuf, kofs, kstep, 0);
         load_chunks(vraw, vbuf, vofs, vstep, 0);
@@ -787,7 +781,8 @@ void dispatch(const ForwardArgs &a, const int cus, hipStream_t stream) {
 } // namespace
 
 // Where the FP32 kernel wins, from 7230 launches of 130 to 4096 items and 1 to 64 tiles on both kernels (µs: FP32 against this one;
-// by this rule three of them are slower than on the FP32 kernel by more than 3%, the worst by 6%):
+// by this rule 3761 of them run here, 1.53 times as fast in the geometric mean, and three of those are slower than on the FP32 kernel by
+// more than 3%, the worst by 5%):
 //   * Few items, whose work its four waves per item and shorter start finish sooner: up to one item per CU (d = 64, 128 of 32: 23.4
 //     against 24.6), up to two under a ramp, and above that short items (d = 64, 384 of 5: 12.6 against 12.5, of 8: 15.1 against
 //     12.9; d = 32, 384 of 8: 9.2 against 9.4, of 12: 11.8 against 10.8) and sequences of odd query tiles that make more
