@@ -31,12 +31,18 @@
  *     accumulated with FP32 atomics, and so are dK/dV of the key blocks whose query range is split over several
  *     workgroups, so those values' low-order bits may differ from run to run (delta is bit-reproducible);
  *   - deterministic: the reference's arrangement, a query-major dQ kernel and a key-major dK/dV kernel (7 matrix
- *     products per tile, S and dP computed in both); bit-identical results run to run. Where there is enough work its
- *     products are formed from fp16 products of two-term operands, with no larger errors than FP32 ones.
+ *     products per tile, S and dP computed in both); bit-identical results run to run.
  *   With neither bit 1 nor bit 2 set the library takes the faster one for the call: deterministic from about one
- *   32-row tile of queries and keys per compute unit on; below that fused for inputs with 128-bit access (16-byte
- *   aligned pointers, strides multiples of 4), under a radius window the band kernel when there are at least 5/8 as many
- *   128-key blocks (batch x heads x ceil(keys / 128)) as compute units, and deterministic otherwise.
+ *   32-row tile of queries and keys per compute unit on (causal calls without a radius: up to two or three); else fused
+ *   for inputs with 128-bit access (16-byte aligned pointers, strides multiples of 4), under a radius window the band
+ *   kernel when there are at least 5/8 as many 128-key blocks (batch x heads x ceil(keys / 128)) as compute units (so
+ *   many blocks with so few tiles: sequences of about one block, or few queries against many keys), and deterministic
+ *   otherwise.
+ * Where there is enough work the forward's and the deterministic backward's products are formed from fp16 products of
+ * operands split in two terms (22 bits of each) and summed in FP32. Errors against 64-bit results are then no larger
+ * than the FP32 products' while a tensor's rows are of like size; rows that lie so far below others that their terms
+ * lose bits, infinities and NaN are found out by the kernels and computed again with FP32 products, 32 rows at a time
+ * (to the same tolerances; such tiles take several times as long).
  *   Bit 1 (ROCMKERNELS_ATTENTION_FUSED_BACKWARD) asks for fused wherever it exists (inputs with 128-bit access); bit 2
  *   (ROCMKERNELS_ATTENTION_DETERMINISTIC) asks for deterministic. Setting both, or any other bit, returns
  *   hipErrorInvalidValue.
