@@ -995,21 +995,28 @@ __global__ __launch_bounds__(kWave * KB * QS) __attribute__((amdgpu_waves_per_eu
         // Keys whose sums are made of terms that lost bits (below 2^-3 they are off by 2^-25): because the rows of dO or Q that count for
         // the key lie far below the ones that set the scales (hidden from it, or without weight), or its weights or dS are small
         // throughout. With Σ P'² of n rows, dV' is off by 2^-25·√(Σ P'²) from dO' and by 2^-26·√n·|dO'| from P': the first is below
-        // 2^-21 of the largest |dV'| if that reaches 2^-4·√(Σ P'²), the second below 2^-20 if Σ P'² reaches 2^-12·n. The same for dK' with
-        // dS' and Q', whose second loss also does no harm where it is below FP32's own rounding of dP (a key of weight near 1, whose
-        // dP - δ cancels): 2^-24·|dO'|·|V'|·√D in units of 2^24, |dO'| taken from dV'.
+        // 2^-21 of the largest |dV'| if that reaches 2^-4·√(Σ P'²), the second below 2^-20 if Σ P'² reaches 2^-12·n and, where the
+        // rows that make Σ P'² up are not those that make dV up, |dV'| 2·√n (|dO'| of 2^7). The same for dK' with dS' and Q' (of 2^10:
+        // 16·√n). A small Σ dS'² also does no harm where FP32's own rounding of dP is larger (a key of weight near 1, whose dP - δ
+        // cancels): 2^-24·Σ |dO'|·|V'| in units of 2^24, |dO'| taken from dV' feature by feature.
         p_norm = halves_sum(p_norm);
         ds_norm = halves_sum(ds_norm);
         const float top_v = halves_max(largest(acc_v)), top_k = halves_max(largest(acc_k));
         const float seen = static_cast<float>(min(qhi - max(qlo, 0) + 1, gradient_chunks)); // rows that can be off (dO = 0: exact)
-        bool faint = visible && ((!no_dv && (256.0f * top_v * top_v < p_norm || p_norm < 0x1p-12f * seen)) || (!no_dk && 256.0f * top_k * top_k < ds_norm));
+        const float root = sqrtf(seen);
+        bool faint = visible && ((!no_dv && (256.0f * top_v * top_v < p_norm || p_norm < 0x1p-12f * seen || top_v < 2.0f * root)) ||
+                (!no_dk && (256.0f * top_k * top_k < ds_norm || (ds_norm >= 0x1p-12f * seen && top_k < 16.0f * root))));
         const bool faint_ds = visible && !no_dk && ds_norm < 0x1p-12f * seen;
         if (__builtin_expect(__ballot(faint_ds) != 0, 0)) {
-            float own = 0.0f;
-#pragma unroll
-            for (int i = 0; i < 2 * KC; ++i)
-                own = fmaxf(own, largest(load_chunk<VEC>(vbuf, visible ? static_cast<uint32_t>(key) * (4u * P.v.st) + 4u * (16 * (i / 2) + 8 * h + 4 * (i % 2)) : kNoRow, 0)));
-            faint = faint || (faint_ds && top_v * 8.0f * halves_max(own) * scale_down(ev) < 0x1p24f * sqrtf(seen));
+            float products = 0.0f;
+            unrolled<DT>([&](auto t) {
+                unrolled<4>([&](auto g) { // features of accumulator registers 4g .. 4g + 3
+                    const uint32_t f = 4u * (32 * t.value + 8 * g.value + 4 * h);
+                    const f32x4 own = load_chunk<VEC>(vbuf, visible ? static_cast<uint32_t>(key) * (4u * P.v.st) + f : kNoRow, 0);
+                    unrolled<4>([&](auto x) { products += fabsf(acc_v[t.value][4 * g.value + x.value] * own[x.value]); });
+                });
+            });
+            faint = faint || (faint_ds && halves_sum(products) * scale_down(ev) < 0x1p24f * root);
         }
         redo = unfit || own_unfit || __ballot(faint) != 0 || !finite(acc_k) || !finite(acc_v);
     }

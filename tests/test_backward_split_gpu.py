@@ -195,6 +195,38 @@ def test_keys_of_small_weights(device, width):
             assert norm_rel(got[0, 0, rows], want[name][0, 0, rows]) <= 2e-5, (name, rows)
 
 
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("exponent", [6, 12])
+@pytest.mark.parametrize("width", [32, 64])
+def test_large_feature_of_v_that_meets_a_small_one_of_the_gradient(device, width, exponent, causal):
+    # One feature of V 2^exponent times the others, and that feature of dO as much smaller: dP is far below the product of their
+    # largest magnitudes, which sets its unit. An FP32 backward is at 1e-6 of 64 bits on each sequence.
+    q, k, v, du = normal_case(475 + width, width, 24, 1, 1001, 1001)
+    mask = np.ones((24, 1001), np.uint8)
+    v[..., 3] *= np.float32(2.0**exponent)
+    du[..., 3] *= np.float32(2.0**-exponent)
+    want = reference64(q[:2], k[:2], v[:2], mask[:2], du[:2], causal=causal)
+    got = gradients(device, q, k, v, du, mask, causal=causal)
+    for name, x in zip(("gq", "gk", "gv"), got):
+        for b in range(2):
+            assert norm_rel(x[b], want[name][b]) <= 3e-6, (name, b)
+
+
+@pytest.mark.parametrize("width", [32, 64])
+def test_gradient_from_rows_of_small_dS(device, width):
+    # The few rows of dO that are 2^12 times the others meet rows of Q that are 0, so dK is the others' alone, whose dS is as much
+    # smaller than the unit. An FP32 backward is at 1e-6 of 64 bits.
+    q, k, v, du = normal_case(485 + width, width, 24, 1, 1001, 1001)
+    mask = np.ones((24, 1001), np.uint8)
+    q[:, :, 0:1001:125] = 0.0
+    du[:, :, 0:1001:125] *= np.float32(2.0**12)
+    want = reference64(q[:2], k[:2], v[:2], mask[:2], du[:2])
+    _, gk, gv, _ = gradients(device, q, k, v, du, mask)
+    for name, x in (("gk", gk), ("gv", gv)):
+        for b in range(2):
+            assert norm_rel(x[b], want[name][b]) <= 3e-6, (name, b)
+
+
 @pytest.mark.parametrize("width", [32, 64])
 def test_peaked_weights_row_by_row(device, width):
     # Scores of standard deviation 4 under a causal mask: some of the last keys, which few queries see, have next to no weight. Every
