@@ -38,15 +38,17 @@
  *   kernel when there are at least 5/8 as many 128-key blocks (batch x heads x ceil(keys / 128)) as compute units (so
  *   many blocks with so few tiles: sequences of about one block, or few queries against many keys), and deterministic
  *   otherwise.
- * Where there is enough work the forward's and the deterministic backward's products are formed from fp16 products of
- * operands split in two terms (22 bits of each) and summed in FP32. Errors against 64-bit results are then no larger
- * than the FP32 products' while a tensor's rows are of like size; rows that lie so far below others that their terms
- * lose bits, infinities and NaN are found out by the kernels and computed again with FP32 products, 32 rows at a time
- * (to the same tolerances; such tiles take several times as long).
  *   Bit 1 (ROCMKERNELS_ATTENTION_FUSED_BACKWARD) asks for fused wherever it exists (inputs with 128-bit access); bit 2
  *   (ROCMKERNELS_ATTENTION_DETERMINISTIC) asks for deterministic. Setting both, or any other bit, returns
  *   hipErrorInvalidValue.
  * The reference-named backward entry points always run the deterministic kernels, as the reference's do.
+ *
+ * Where there is enough work the forward's and the deterministic backward's products are formed from fp16 products of
+ * operands split in two terms (22 bits of each) and summed in FP32. Errors against 64-bit results are then no larger
+ * than the FP32 products' while a tensor's rows and features are of like size. Rows that lie so far below others that
+ * their terms lose bits, infinities and NaN are found out by the kernels and computed again with FP32 products, 32 rows
+ * at a time (such tiles take several times as long). Not found out: scores of tens that come from a few large products
+ * keep their 22 bits (single rows of peaked weights are off by 1e-5 to 1e-4).
  */
 #ifndef ROCMKERNELS_ATTENTION_H
 #define ROCMKERNELS_ATTENTION_H
