@@ -266,8 +266,7 @@ def measure_rotary(cfg, steps, warmup):
 
 def cpu_threads():
     """(visible cores, threads used). The visible count is this process's CPU affinity; the threads used are capped by
-    OMP_NUM_THREADS when it is set (the GPU box exports the CPU share it grants one GPU there, and asks that worker
-    pools stay within it)."""
+    OMP_NUM_THREADS when it is set (a shared machine may export the CPU share it grants one GPU there)."""
     visible = len(os.sched_getaffinity(0))
     try:
         limit = int(os.environ.get("OMP_NUM_THREADS", "0"))

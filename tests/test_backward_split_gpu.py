@@ -6,7 +6,7 @@ import pytest
 import torch
 
 import oracle
-from parity import check_backward, host, norm_rel, normal_case, padding_mask, reference64, to_dev
+from parity import check_backward, check_forward, host, norm_rel, normal_case, padding_mask, reference64, to_dev
 from rocmkernels_amd import attention
 
 pytestmark = pytest.mark.gpu
@@ -93,6 +93,25 @@ def test_default_backward_either_side_of_the_line(device, width, batch, heads, l
     out, lse = attention.forward(tq, tk, tv, tm, causal=causal)
     got = host(*attention.backward(tq, tk, tv, tm, out, lse, tdu, causal=causal, entry="ex", deterministic=False))
     check_backward(*got, want, f"default d{width}")
+
+
+@pytest.mark.parametrize("seed", range(20))
+def test_random_launches(device, seed):
+    # Launches of 257 to about 2000 tiles of queries, any raggedness, window and mask, forward and deterministic backward.
+    rng = np.random.default_rng(490 + seed)
+    width = (32, 64)[seed % 2]
+    queries = int(rng.integers(33, 1100))
+    keys = queries if rng.random() < 0.5 else int(rng.integers(33, 1100))
+    batch = int(rng.integers(257, 1200)) // -(-queries // 32) + 1
+    causal = bool(rng.random() < 0.5)
+    radius = int(rng.integers(1, keys)) if rng.random() < 0.4 else -1
+    q, k, v, du = normal_case(491 + seed, width, batch, 1, queries, keys)
+    mask = padding_mask(492 + seed, batch, keys, keys // 3 + 1)
+    want = oracle.attention(q, k, v, mask, upstream=du, radius=radius, causal=causal)
+    label = f"d{width} {batch} x {queries} x {keys} radius {radius} causal {causal}"
+    out, lse = host(*attention.forward(*to_dev(device, q, k, v, mask), radius=radius, causal=causal))
+    check_forward(out, lse, want, label)
+    check_backward(*gradients(device, q, k, v, du, mask, radius, causal), want, label)
 
 
 @pytest.mark.parametrize("width", [32, 64])

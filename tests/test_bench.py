@@ -88,7 +88,7 @@ def test_roofline_kernels_have_profiled_traffic():
 
 
 def test_cpu_baseline_reports_single_thread_and_all_core_rates():
-    # Config 1 is small enough to time here; the GPU box runs the same code on its own cores.
+    # Config 1 is small enough to time here; a GPU machine runs the same code on its own cores.
     result = bench.cpu_baseline(1, 0.2)
     visible, threads = bench.cpu_threads()
     assert result["kind"] == "port" and result["unit"] == "TFLOP/s" and result["value"] > 0
